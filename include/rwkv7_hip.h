@@ -297,6 +297,26 @@ int rwkv7_wkv7_backward(const float *hist, const float *S_T, const float *r,
                         float *gk, float *gv, float *ga, float *gb, int32_t B,
                         int32_t T, int32_t H, void *stream);
 
+/* rwkv7_wkv7_f32 (no history) by the chunked algorithm of rwkv7_wkv7_chunked,
+ * with its workspace (rwkv7_wkv7_chunked_workspace_bytes). RWKV7_ESHAPE when a
+ * sequence's chunk records pass 2 GiB (T beyond about a million tokens). */
+int rwkv7_wkv7_f32_chunked(float *S, const float *r, const float *w, const float *k, const float *v, const float *a,
+                           const float *b, float *y, int32_t B, int32_t T, int32_t H, void *workspace,
+                           int64_t workspace_bytes, void *stream);
+
+/* The gradients rwkv7_wkv7_backward gives, from the forward's inputs alone:
+ * S0 [B, H, 64, 64] is the state before the sequence (not written), no history
+ * is read. Chunked scans of the states and of their adjoint, then every
+ * 16-token chunk at once; the workspace holds the chunk records and boundary
+ * states (about 5 KB per token and head). The gradient half of the DPLR
+ * backward the reference plans (TODO.md:46-54), recomputing its states.
+ * RWKV7_ESHAPE as rwkv7_wkv7_f32_chunked. */
+int64_t rwkv7_wkv7_grad_workspace_bytes(int32_t B, int32_t T, int32_t H);
+int rwkv7_wkv7_grad(const float *S0, const float *r, const float *w, const float *k, const float *v, const float *a,
+                    const float *b, const float *gy, const float *gS_T, float *gS0, float *gr, float *gw, float *gk,
+                    float *gv, float *ga, float *gb, int32_t B, int32_t T, int32_t H, void *workspace,
+                    int64_t workspace_bytes, void *stream);
+
 /* LayerNorm over the last dimension (eps 1e-5): x f32 or f16 [M, C]
  * (x_is_f32), weight/bias f32 [C], y f32 [M, C]. Stands in for LNWeight
  * (src/rwkv_tl/weight.py:14-15). */

@@ -722,6 +722,33 @@ int rwkv7_wkv7_backward(const float *hist, const float *S_T, const float *r, con
   return launch_wkv7_bwd(p, static_cast<hipStream_t>(stream));
 }
 
+int rwkv7_wkv7_f32_chunked(float *S, const float *r, const float *w, const float *k, const float *v, const float *a,
+                           const float *b, float *y, int32_t B, int32_t T, int32_t H, void *workspace,
+                           int64_t workspace_bytes, void *stream) {
+  if (!S || !r || !w || !k || !v || !a || !b || !y || !workspace) return RWKV7_EINVAL;
+  if (B < 1 || T < 1 || H < 1) return RWKV7_ESHAPE;
+  if (workspace_bytes < wkv7_chunk_rec_bytes(B, T, H)) return RWKV7_EWORKSPACE;
+  ScanArgs<float, float, float> p = {S, r, k, v, a, b, w, y, B, T, H, nullptr};
+  return launch_wkv7_chunked(p, static_cast<float *>(workspace), static_cast<hipStream_t>(stream));
+}
+
+int64_t rwkv7_wkv7_grad_workspace_bytes(int32_t B, int32_t T, int32_t H) {
+  if (B < 1 || T < 1 || H < 1) return 0;
+  return wkv7_grad_ws_bytes(B, T, H);
+}
+
+int rwkv7_wkv7_grad(const float *S0, const float *r, const float *w, const float *k, const float *v, const float *a,
+                    const float *b, const float *gy, const float *gS_T, float *gS0, float *gr, float *gw, float *gk,
+                    float *gv, float *ga, float *gb, int32_t B, int32_t T, int32_t H, void *workspace,
+                    int64_t workspace_bytes, void *stream) {
+  if (!S0 || !r || !w || !k || !v || !a || !b || !gy || !gS0 || !gr || !gw || !gk || !gv || !ga || !gb || !workspace)
+    return RWKV7_EINVAL;
+  if (B < 1 || T < 1 || H < 1) return RWKV7_ESHAPE;
+  if (workspace_bytes < wkv7_grad_ws_bytes(B, T, H)) return RWKV7_EWORKSPACE;
+  Wkv7GradArgs p = {S0, r, w, k, v, a, b, gy, gS_T, gS0, gr, gw, gk, gv, ga, gb, B, T, H};
+  return launch_wkv7_grad(p, static_cast<float *>(workspace), static_cast<hipStream_t>(stream));
+}
+
 int rwkv7_layernorm(const void *x, int32_t x_is_f32, const float *weight, const float *bias, float *y, int32_t M,
                     int32_t C, int32_t bf16, void *stream) {
   if (!x || !weight || !bias || !y) return RWKV7_EINVAL;

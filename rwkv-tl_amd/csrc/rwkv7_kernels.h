@@ -77,6 +77,17 @@ struct Wkv7BwdArgs {
 };
 int launch_wkv7_bwd(const Wkv7BwdArgs &p, hipStream_t st);
 
+// Gradient of a sequence from its inputs alone (nothing recorded by the
+// forward): S0, r, w, k, v, a, b as given to the forward, gy and gS_T (or null:
+// zero) to gS0 and the gradients of the six inputs. ws: wkv7_grad_ws_bytes.
+struct Wkv7GradArgs {
+  const float *S0, *r, *w, *k, *v, *a, *b, *gy, *gS_T;
+  float *gS0, *gr, *gw, *gk, *gv, *ga, *gb;
+  int B, T, H;
+};
+int64_t wkv7_grad_ws_bytes(int B, int T, int H);
+int launch_wkv7_grad(const Wkv7GradArgs &p, float *ws, hipStream_t st);
+
 struct LnShiftArgs {
   const float *x0;
   const float *ln_w, *ln_b;

@@ -203,6 +203,7 @@ using StageBuf = float4[6][CH][kN / 4];
 template <int CH>
 struct GateStager {
   using Args = PrefillScanArgs;
+  static constexpr bool kAdj = false;
   const PrefillScanArgs &p;
   int64_t base, MC;
   int t1, quarter, st_tok, q, C;
@@ -308,6 +309,7 @@ struct GateStager {
 template <int CH, typename TI, typename TW, typename TY>
 struct RawStager {
   using Args = ScanArgs<TI, TW, TY>;
+  static constexpr bool kAdj = false;
   const Args &p;
   int64_t base;
   int t1, st_tok, q, C;
@@ -347,6 +349,64 @@ struct RawStager {
   // state entering token tt: row `row`, key columns 4 lc .. 4 lc + 3
   RWKV7_DEV void record(int tt, int row, int lc, const float4 &S) {
     if (p.hist) *reinterpret_cast<float4 *>(p.hist + hbase + (int64_t)tt * (kN * kN) + row * kN + 4 * lc) = S;
+  }
+};
+
+// The adjoint of a sequence as the same recurrence run backward in time
+// (launch_wkv7_grad): the adjoint arriving at the state before token t,
+//   G'_{t-1} = G'_t diag(w_t) + (G'_t b_t) a_t^T + gy_t (w_t r_t + (r_t . b_t) a_t)^T,
+// is a step on G' with a and b changed, v = gy_t and k = w_t r_t + (r_t . b_t) a_t.
+// Step i of the scan is token Tp - 1 - i of the sequence padded to Tp tokens
+// (whole chunks, so that its chunks are the forward scan's); the row "y" of a
+// step is gv_t = G'_t k_t + gy_t (r_t . k_t), taken before the step's update.
+template <int CH>
+struct AdjStager {
+  struct Args {
+    const float *r, *w, *k, *a, *b, *gy;
+    int B, T, H;
+  };
+  static constexpr bool kAdj = true;
+  const Args &p;
+  int64_t base;
+  int Tp, st_tok, q, C;
+  bool stager;
+  float4 g_r, g_w, g_k, g_a, g_b, g_y;
+  float *diag = nullptr;  // LDS [CH]: r_t . k_t of the chunk's steps
+
+  RWKV7_DEV AdjStager(const Args &p_, int, int, int64_t base_, int) : p(p_), base(base_) {
+    C = p.H * kN;
+    Tp = (p.T + CH - 1) / CH * CH;
+    st_tok = threadIdx.x >> 4;
+    q = threadIdx.x & 15;
+    stager = st_tok < CH;
+  }
+  // whether step i (of the whole scan) is a token of the sequence
+  RWKV7_DEV bool live(int i) const { return Tp - 1 - i < p.T; }
+  RWKV7_DEV void fetch(int c0) {
+    const int tt = min(max(Tp - 1 - (c0 + st_tok), 0), p.T - 1);
+    const int64_t o = base + (int64_t)tt * C + 4 * q;
+    g_r = ld4_as_f(p.r + o);
+    g_w = ld4_as_f(p.w + o);
+    g_k = ld4_as_f(p.k + o);
+    g_a = ld4_as_f(p.a + o);
+    g_b = ld4_as_f(p.b + o);
+    g_y = ld4_as_f(p.gy + o);
+  }
+  template <class Sink>
+  RWKV7_DEV void commit_to(int c0, Sink &&sink) {
+    auto dot = [](const float4 &x, const float4 &y) {
+      return fmaf(x.x, y.x, x.y * y.y) + fmaf(x.z, y.z, x.w * y.w);
+    };
+    const float2 d = sum16x2(dot(g_r, g_b), dot(g_r, g_k));
+    if (!stager) return;
+    sink(0, st_tok, q, g_w);
+    sink(1, st_tok, q, g_b);
+    sink(2, st_tok, q, g_a);
+    sink(3, st_tok, q, make_float4(fmaf(d.x, g_a.x, g_w.x * g_r.x), fmaf(d.x, g_a.y, g_w.y * g_r.y),
+                                   fmaf(d.x, g_a.z, g_w.z * g_r.z), fmaf(d.x, g_a.w, g_w.w * g_r.w)));
+    sink(4, st_tok, q, g_k);
+    sink(5, st_tok, q, g_y);
+    if (q == 0) diag[st_tok] = live(c0 + st_tok) ? d.y : 0.f;
   }
 };
 
@@ -761,14 +821,17 @@ int prefill_segments(int T, int B, int H, int cus, int *seg_len) {
 // k^_s = k_s D(s, 15], gam = D(-1, 15], and the 16 x 16 token matrices are
 //   Aba[t][s] = b_s^T D(s, t-1] a_t,  Aka[t][s] = k_s^T D(s, t-1] a_t  (s < t)
 //   Bbr[t][s] = b_s^T D(s, t] r_t,    Bkr[t][s] = k_s^T D(s, t] r_t    (s <= t).
+// For the adjoint scan (AdjStager) the rows are taken before the step's
+// update, Y row t = G'_t k_t + gy_t (r_t . k_t): r~ and the masks of Bbr, Bkr
+// are then those of a~ and Aba, Aka, with r_t . k_t on Bkr's diagonal.
 // Two kernels:
 // 1. wkv7_chunk_prep_kernel, one workgroup per (chunk, head, sequence), all at
 //    once: stages the chunk through the serial scan's staging policies, forms
 //    the token matrices -- on MFMA as (a~)(b / P_s)^T etc. with the prefix
 //    products P_t = D(-1, t] when every P_t of the chunk lies in [1e-30,
-//    1e30], otherwise straight from products of w -- solves for T by forward
+//    1e30], otherwise straight from products of w -- applies T by forward
 //    substitution, and writes G1, G2, B^, K^, U, Y0, V and gam as a chunk
-//    record laid out in the chain kernel's MFMA operand order.
+//    record.
 // 2. wkv7_chunk_chain_kernel, grid (4 H / NQ, B): each workgroup carries
 //    16 NQ value rows of a head's state through the chunks in order; per
 //    chunk and quarter, Sig and Y from S (16 x 64 by 64 x 16), then
@@ -779,13 +842,13 @@ int prefill_segments(int T, int B, int H, int cus, int *seg_len) {
 // a = b = k = r = v = 0), whose outputs are not stored.
 // ---------------------------------------------------------------------------
 constexpr int kCk = 16;
-// Chunk record (f32). G1, G2, B^, K^: [wave][lane][kk]; U, V: [quarter][lane][kk];
-// Y0: [quarter][t][i]; gam: [64]. The chain kernel's lane l of wave w (rows
-// 16 q .. of the state) reads element kk of [w or q][l] as its operand of the
-// kk-th MFMA step.
+// Chunk record (f32). G1, G2, Y0: [token][channel]; B^, K^: [wave][lane][kk];
+// U, V: [quarter][lane][kk]; gam: [64]. The chain kernel's lane l of wave w
+// (rows 16 q .. of the state) reads element kk of [w or q][l] as its operand
+// of the kk-th MFMA step; its DMA gathers G1, G2 and Y0 into that order from
+// the plain rows, which the prep kernel can store one channel per lane.
 constexpr int kRecG1 = 0, kRecG2 = 1024, kRecBh = 2048, kRecKh = 3072, kRecU = 4096, kRecY0 = 5120,
               kRecV = 6144, kRecGam = 7168, kRecFloats = 7232;
-constexpr int kPad = kN + 1;  // a padded 64-channel LDS row
 
 // the chain kernel addresses a (sequence, head)'s records and a sequence's y
 // through 32-bit buffer offsets
@@ -895,31 +958,54 @@ RWKV7_DEV void lora2_chunk(const PrefillScanArgs &p, St &st, int h, int bi, int 
   lora2_compute<BF, F32>(p, g, h, bi, T, t0, t1, s_d);
 }
 
+// What bounds it: LDS instructions and the latency between its barriers, not
+// the products. So beyond the staged rows and the token matrices everything
+// stays in registers with one channel per lane: each wave scales one of a, k,
+// r, b by the prefix products (wave-local, every wave forms them for itself),
+// the forward substitutions and products with the token matrices are FMAs
+// whose coefficients are LDS broadcasts (one 16-byte read per four), and the
+// record is stored from the registers that hold it. Three barriers after the
+// staging (four where U passes between waves) against eight when each
+// intermediate went through LDS. Measured (kernel trace): 1024 chunks of raw
+// half inputs 20.4 -> 14.0 us; 2048 of f32 inputs 23 us, 109 MB moved (4.7
+// TB/s, the rate of a large copy here).
+//
 // L2: the model path with the LoRA second steps formed here (GateStager and
-// p.l1 set); a separate instance, whose registers those products no longer
-// hold, keeps three workgroups per CU for the other cases.
+// p.l1 set); a separate instance, whose registers and LDS those products no
+// longer hold, keeps more workgroups per CU for the other cases.
+constexpr int kXs = kN + 4;  // floats per staged row (16-byte aligned, rows 4 banks apart)
+
+// acc[t] += sum over s < t (s <= t with DIAG) of M[t][s] x[s], one channel per
+// lane; M's rows are read as LDS broadcasts. With SOLVE x is acc itself:
+// forward substitution with the unit lower triangular I - M.
+template <bool DIAG, bool SOLVE>
+RWKV7_DEV void tri_apply(const float (*M)[kCk], const float (&x)[kCk], float (&acc)[kCk]) {
+#pragma unroll
+  for (int t = DIAG ? 0 : 1; t < kCk; ++t) {
+    const float4 *m4 = reinterpret_cast<const float4 *>(M[t]);
+#pragma unroll
+    for (int g = 0; g <= (DIAG ? t : t - 1) / 4; ++g) {
+      const float4 q = m4[g];
+      const float c[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int s = 4 * g + e;
+        if (s < t || (DIAG && s == t)) acc[t] = fmaf(c[e], SOLVE ? acc[s] : x[s], acc[t]);
+      }
+    }
+  }
+}
+
 template <class St, bool L2>
 __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args p, float *rec, int T, int H) {
-  // 35 KB of LDS without the LoRA steps (43 KB with them, which stage there),
-  // so that four workgroups share a CU (the 1.5B-shaped 4 x 1024 prefill
-  // runs 8192 of them): the stager writes its padded rows straight into s_x,
-  // b^ and k^ go from registers straight into the record, and the later
-  // 16 x 64 results take the rows that are dead by then -- AkaV and then G2
-  // the prefix products', G1 w's, U b's and Y0 k's (each phase below ends
-  // with a barrier before the next reuses a row)
-  constexpr int NB = L2 ? 3 : 1;
-  __shared__ float s_x[6][kCk][kPad];     // w, a (a~), b (b / P), k (k / P), r (r~), v
-  __shared__ float s_bkp[NB][kCk][kPad];  // prefix products P_t = D(-1, t] (and the LoRA steps before them)
-  __shared__ float s_m[4][kCk][kCk + 1];  // Aba, Aka, Bbr, Bkr
-  __shared__ float s_t[kCk][kCk + 1];
-  __shared__ float s_gam[kN];
-  typedef float Row[kPad];
-  Row *s_p = s_bkp[NB - 1];
-  Row *s_akav = s_bkp[NB - 1], *s_g2 = s_bkp[NB - 1], *s_g1 = s_x[0], *s_u = s_x[2], *s_y0 = s_x[3];
-  static_assert(!L2 || sizeof(s_bkp) >= 3 * kCk * kN * sizeof(float), "LoRA steps staged in s_bkp");
+  __shared__ __align__(16) float s_x[6][kCk][kXs];  // w, a (a~, then U), b (b / P), k (k / P), r (r~), v
+  __shared__ __align__(16) float s_m[4][kCk][kCk];  // Aba, Aka, Bbr, Bkr
+  __shared__ float s_d[L2 ? 3 * kCk * kN : 1];      // the LoRA steps v, w, a
+  constexpr bool ADJ = St::kAdj;  // rows taken before the step's update (AdjStager)
+  __shared__ float s_diag[ADJ ? kCk : 1];
 
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int row = lane & 15, kq = lane >> 4, col = 16 * wv + row;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = lane & 15, kq = lane >> 4;
   const int c = blockIdx.x, h = blockIdx.y, bi = blockIdx.z;
   const int C = H * kN;
   const int t0 = c * kCk, t1 = min(T, t0 + kCk), Tl = t1 - t0;
@@ -928,62 +1014,51 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
   St st(p, h, -1, (int64_t)bi * T * C + (int64_t)h * kN, t1);
   bool fetched = false;
   if constexpr (L2 && std::is_same<St, GateStager<kCk>>::value) {
-    {
-      float *s_d = &s_bkp[0][0][0];  // free until the products below
-      if (p.bf) {
-        if (p.l1_f32) lora2_chunk<true, true>(p, st, h, bi, T, t0, t1, s_d);
-        else lora2_chunk<true, false>(p, st, h, bi, T, t0, t1, s_d);
-      } else {
-        if (p.l1_f32) lora2_chunk<false, true>(p, st, h, bi, T, t0, t1, s_d);
-        else lora2_chunk<false, false>(p, st, h, bi, T, t0, t1, s_d);
-      }
-      st.lds_d = s_d;
-      st.lds_ld = kN;
-      fetched = true;
-      __syncthreads();
+    if (p.bf) {
+      if (p.l1_f32) lora2_chunk<true, true>(p, st, h, bi, T, t0, t1, s_d);
+      else lora2_chunk<true, false>(p, st, h, bi, T, t0, t1, s_d);
+    } else {
+      if (p.l1_f32) lora2_chunk<false, true>(p, st, h, bi, T, t0, t1, s_d);
+      else lora2_chunk<false, false>(p, st, h, bi, T, t0, t1, s_d);
     }
+    st.lds_d = s_d;
+    st.lds_ld = kN;
+    fetched = true;
+    __syncthreads();
   }
   if (!fetched) st.fetch(t0);
-  // padded f32 rows; tokens past the end become identity steps
+  if constexpr (ADJ) st.diag = s_diag;
+  // padded f32 rows; steps past the sequence become identity steps
   st.commit_to(t0, [&](int i, int tt, int qq, float4 x) {
-    if (tt >= Tl) x = i == 0 ? make_float4(1.f, 1.f, 1.f, 1.f) : make_float4(0.f, 0.f, 0.f, 0.f);
-    s_x[i][tt][4 * qq] = x.x;
-    s_x[i][tt][4 * qq + 1] = x.y;
-    s_x[i][tt][4 * qq + 2] = x.z;
-    s_x[i][tt][4 * qq + 3] = x.w;
+    bool pad = tt >= Tl;
+    if constexpr (ADJ) pad = !st.live(t0 + tt);
+    if (pad) x = i == 0 ? make_float4(1.f, 1.f, 1.f, 1.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float4 *>(&s_x[i][tt][4 * qq]) = x;
   });
   __syncthreads();
+
+  // One channel per lane from here on. Wave 0 holds a, 1 k, 2 r (and k), 3 b.
+  const int xi = wv == 0 ? 1 : wv == 1 ? 3 : wv == 2 ? 4 : 2;
+  float w[kCk], x[kCk], z[kCk];
+#pragma unroll
+  for (int t = 0; t < kCk; ++t) {
+    w[t] = s_x[0][t][lane];
+    x[t] = s_x[xi][t][lane];
+    if (wv == 2) z[t] = s_x[3][t][lane];
+  }
   bool ok = true;
-  if (tid < kN) {  // wave 0: prefix products P_t, and whether they stay in range
-    const int j = tid;
+  {
     float P = 1.f;
 #pragma unroll
     for (int t = 0; t < kCk; ++t) {
-      P *= s_x[0][t][j];
-      s_p[t][j] = P;
+      P *= w[t];
       ok = ok && P >= 1e-30f && P <= 1e30f;  // false for NaN too
     }
-  } else if (tid < 2 * kN) {  // wave 1: suffix products (b^, k^, gam), exact products of w
-    const int j = tid - kN;
-    float Q = 1.f, bh[kCk], kh[kCk];
-#pragma unroll
-    for (int t = kCk - 1; t >= 0; --t) {
-      bh[t] = s_x[2][t][j] * Q;
-      kh[t] = s_x[3][t][j] * Q;
-      Q *= s_x[0][t][j];
-    }
-    s_gam[j] = Q;
-    // B operand of the state update, X[4 kk + kq][16 w + row], as the chain
-    // kernel's thread 64 w + 16 kq + row reads it (kk = 0..3 in one float4)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int off = 4 * (64 * (j >> 4) + 16 * q + (j & 15));
-      *reinterpret_cast<float4 *>(R + kRecBh + off) = make_float4(bh[q], bh[4 + q], bh[8 + q], bh[12 + q]);
-      *reinterpret_cast<float4 *>(R + kRecKh + off) = make_float4(kh[q], kh[4 + q], kh[8 + q], kh[12 + q]);
-    }
   }
-  const bool fast = __syncthreads_and(ok);  // block-uniform
-  if (!fast) {  // token matrices straight from products of w: thread (t, s)
+  // the same w in every wave, so the same answer: uniform over the workgroup
+  const bool fast = __all(ok);
+  __syncthreads();  // the rows are read: they may be overwritten
+  if (!fast) {      // token matrices straight from products of w: thread (t, s)
     const int t = tid >> 4, s = tid & 15;
     float aba = 0.f, aka = 0.f, bbr = 0.f, bkr = 0.f;
     if (s <= t) {
@@ -996,122 +1071,133 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
           aba = fmaf(bs * d, at, aba);
           aka = fmaf(ks * d, at, aka);
         }
-        bbr = fmaf(bs * dt, rt, bbr);
-        bkr = fmaf(ks * dt, rt, bkr);
+        if (!ADJ || s < t) {
+          bbr = fmaf(bs * (ADJ ? d : dt), rt, bbr);
+          bkr = fmaf(ks * (ADJ ? d : dt), rt, bkr);
+        }
       }
     }
+    if (ADJ && s == t) bkr = s_diag[t];
     s_m[0][t][s] = aba;
     s_m[1][t][s] = aka;
     s_m[2][t][s] = bbr;
     s_m[3][t][s] = bkr;
     __syncthreads();
   }
-  {  // a~, r~ (and b / P, k / P for the MFMA form) in place: token tid / 16, 4 channels
-    const int t = tid >> 4, j0 = 4 * (tid & 15);
+  // a~ = a D(-1, t-1], r~ = r D(-1, t] and (for the MFMA form) k / P, b / P
+  {
+    float P = 1.f;
+    if (wv == 0) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int j = j0 + u;
-      const float P = s_p[t][j], Pp = t > 0 ? s_p[t - 1][j] : 1.f;
-      s_x[1][t][j] *= Pp;
-      s_x[4][t][j] *= P;
-      if (fast) {
-        s_x[2][t][j] = s_x[2][t][j] / P;
-        s_x[3][t][j] = s_x[3][t][j] / P;
+      for (int t = 0; t < kCk; ++t) {
+        x[t] *= P;
+        P *= w[t];
+        s_x[1][t][lane] = x[t];
+      }
+    } else if (wv == 2) {
+#pragma unroll
+      for (int t = 0; t < kCk; ++t) {
+        if (!ADJ) P *= w[t];
+        s_x[4][t][lane] = x[t] * P;
+        if (ADJ) P *= w[t];
+      }
+    } else if (fast) {
+#pragma unroll
+      for (int t = 0; t < kCk; ++t) {
+        P *= w[t];
+        s_x[xi][t][lane] = x[t] / P;
       }
     }
   }
   __syncthreads();
   if (fast) {  // wave m: token matrix m, (a~ or r~) (b / P or k / P)^T, masked
-    const int m = wv;
-    const Row *X = s_x[m < 2 ? 1 : 4];
-    const Row *Y = s_x[(m & 1) ? 3 : 2];
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    const float4 *X = reinterpret_cast<const float4 *>(&s_x[wv < 2 ? 1 : 4][row][16 * kq]);
+    const float4 *Y = reinterpret_cast<const float4 *>(&s_x[(wv & 1) ? 3 : 2][row][16 * kq]);
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kk = 0; kk < kN / 4; ++kk) acc = mfma4(X[row][4 * kk + kq], Y[row][4 * kk + kq], acc);
+    for (int u = 0; u < 4; ++u) {  // channels 16 kq + 4 u + e
+      const float4 xv = X[u], yv = Y[u];
+      acc = mfma4(xv.x, yv.x, acc);
+      acc2 = mfma4(xv.y, yv.y, acc2);
+      acc = mfma4(xv.z, yv.z, acc);
+      acc2 = mfma4(xv.w, yv.w, acc2);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 4 * kq + r, s = row;
-      s_m[m][t][s] = (m < 2 ? s < t : s <= t) ? acc[r] : 0.f;
+      float m = (wv < 2 || ADJ ? s < t : s <= t) ? acc[r] + acc2[r] : 0.f;
+      if (ADJ && wv == 3 && s == t) m = s_diag[t];
+      s_m[wv][t][s] = m;
     }
     __syncthreads();
   }
-  {  // AkaV, value columns 16 wv ..
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  // Operand of the state update for the chain kernel, X[4 kk + kq][16 w + row]
+  // as its thread 64 w + 16 kq + row reads it (kk = 0..3 in one float4).
+  auto put_frag = [&](int off, const float (&f)[kCk]) {
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) acc = mfma4(s_m[1][row][4 * kk + kq], s_x[5][4 * kk + kq][col], acc);
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<float4 *>(R + off + 4 * (64 * (lane >> 4) + 16 * q + (lane & 15))) =
+          make_float4(f[q], f[4 + q], f[8 + q], f[12 + q]);
+  };
+  auto put_rows = [&](int off, const float (&f)[kCk]) {  // [token][channel]
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s_akav[4 * kq + r][col] = acc[r];
-  }
-  if (tid < kCk) {  // T = (I - Aba)^-1 by forward substitution, lane = column
-    const int cc = tid;
-    float tc[kCk];
+    for (int t = 0; t < kCk; ++t) R[off + t * kN + lane] = f[t];
+  };
+  // x D(t, 15] by suffix products, exact products of w; returns D(-1, 15]
+  auto suffix = [&](const float (&f)[kCk], float (&out)[kCk]) {
+    float Q = 1.f;
+#pragma unroll
+    for (int t = kCk - 1; t >= 0; --t) {
+      out[t] = f[t] * Q;
+      Q *= w[t];
+    }
+    return Q;
+  };
+  float f[kCk], y0[kCk];  // wave 3, across the barrier below
+  if (wv == 0) {  // G1 = T A~, G2 = R~ + Bbr G1
+    tri_apply<false, true>(s_m[0], x, x);
+    put_rows(kRecG1, x);
+    float g2[kCk];
+#pragma unroll
+    for (int t = 0; t < kCk; ++t) g2[t] = s_x[4][t][lane];
+    tri_apply<true, false>(s_m[2], x, g2);
+    put_rows(kRecG2, g2);
+  } else if (wv == 1) {  // U = T Aka V
+    float u[kCk];
 #pragma unroll
     for (int t = 0; t < kCk; ++t) {
-      float acc = t == cc ? 1.f : 0.f;
-#pragma unroll
-      for (int s = 0; s < t; ++s) acc = fmaf(s_m[0][t][s], tc[s], acc);
-      tc[t] = acc;
-      s_t[t][cc] = acc;
+      z[t] = s_x[5][t][lane];
+      u[t] = 0.f;
     }
+    tri_apply<false, false>(s_m[1], z, u);
+    tri_apply<false, true>(s_m[0], u, u);
+#pragma unroll
+    for (int t = 0; t < kCk; ++t) s_x[1][t][lane] = u[t];
+    put_frag(kRecU, u);
+  } else if (wv == 2) {  // k^, gam
+    float kh[kCk];
+    const float Q = suffix(z, kh);
+    R[kRecGam + lane] = Q;
+    put_frag(kRecKh, kh);
+  } else {  // b^, V, Y0 = Bkr V + Bbr U
+    suffix(x, f);
+    put_frag(kRecBh, f);
+#pragma unroll
+    for (int t = 0; t < kCk; ++t) {
+      f[t] = s_x[5][t][lane];
+      y0[t] = 0.f;
+    }
+    put_frag(kRecV, f);
+    tri_apply<true, false>(s_m[3], f, y0);
   }
   __syncthreads();
-  {  // G1 = T A~, U = T AkaV (column block wv)
-    floatx4 g = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
+  if (wv == 3) {
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const float tv = s_t[row][4 * kk + kq];
-      g = mfma4(tv, s_x[1][4 * kk + kq][col], g);
-      u = mfma4(tv, s_akav[4 * kk + kq][col], u);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s_g1[4 * kq + r][col] = g[r];
-      s_u[4 * kq + r][col] = u[r];
-    }
+    for (int t = 0; t < kCk; ++t) f[t] = s_x[1][t][lane];
+    tri_apply<true, false>(s_m[2], f, y0);
+    put_rows(kRecY0, y0);
   }
-  __syncthreads();
-  {  // G2 = R~ + Bbr G1, Y0 = Bbr U + Bkr V
-    floatx4 g2, y0 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int r = 0; r < 4; ++r) g2[r] = s_x[4][4 * kq + r][col];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const float bb = s_m[2][row][4 * kk + kq], bk = s_m[3][row][4 * kk + kq];
-      g2 = mfma4(bb, s_g1[4 * kk + kq][col], g2);
-      y0 = mfma4(bb, s_u[4 * kk + kq][col], y0);
-      y0 = mfma4(bk, s_x[5][4 * kk + kq][col], y0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s_g2[4 * kq + r][col] = g2[r];
-      s_y0[4 * kq + r][col] = y0[r];
-    }
-  }
-  __syncthreads();
-  // the rest of the record, one float4 per thread and array (thread = wave
-  // 64 + lane of the chain kernel's reader)
-  const int w = tid >> 6;
-  auto put = [&](int off, float a0, float a1, float a2, float a3) {
-    *reinterpret_cast<float4 *>(R + off + 4 * tid) = make_float4(a0, a1, a2, a3);
-  };
-  // A operand of the chain's Sig / Y step: G[row][16 w + 4 kk + kq]
-  put(kRecG1, s_g1[row][16 * w + kq], s_g1[row][16 * w + 4 + kq], s_g1[row][16 * w + 8 + kq],
-      s_g1[row][16 * w + 12 + kq]);
-  put(kRecG2, s_g2[row][16 * w + kq], s_g2[row][16 * w + 4 + kq], s_g2[row][16 * w + 8 + kq],
-      s_g2[row][16 * w + 12 + kq]);
-  // A operand of the state update (value rows 16 q + row, q = w here)
-  put(kRecU, s_u[kq][16 * w + row], s_u[4 + kq][16 * w + row], s_u[8 + kq][16 * w + row],
-      s_u[12 + kq][16 * w + row]);
-  put(kRecV, s_x[5][kq][16 * w + row], s_x[5][4 + kq][16 * w + row], s_x[5][8 + kq][16 * w + row],
-      s_x[5][12 + kq][16 * w + row]);
-  {  // Y0[q][t][i] = Y0[t][16 q + i]
-    const int e = 4 * tid, q = e >> 8, t = (e >> 4) & 15, i = e & 15;
-    put(kRecY0, s_y0[t][16 * q + i], s_y0[t][16 * q + i + 1], s_y0[t][16 * q + i + 2], s_y0[t][16 * q + i + 3]);
-  }
-  if (tid < kN / 4) put(kRecGam, s_gam[4 * tid], s_gam[4 * tid + 1], s_gam[4 * tid + 2], s_gam[4 * tid + 3]);
 }
-
-
 
 // One chunk record in LDS as a chain workgroup of NQ value quarters uses it:
 // G1, G2, B^, K^ of the four column blocks, then 1 KiB pieces: U, V and Y0
@@ -1142,10 +1228,30 @@ RWKV7_DEV void store_y(__amdgpu_buffer_rsrc_t r, unsigned off, bf16_t v) {
 // of a head per workgroup; wave w takes quarter w / 4 of the workgroup and key
 // column block w % 4. With NQ = 2 each record is fetched once for two
 // quarters: at many heads the record stream is what bounds the chain.
-template <typename TY, int NQ>
-__global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, const float *rec, TY *y, int T, int H) {
+//
+// GRAD (launch_wkv7_grad): grid z picks one of two scans, the forward one and
+// the adjoint one backward in time (rev: step i is token NC kCk - 1 - i). It
+// also stores the state entering each chunk, [B, H, chunk in token order, 64,
+// 64], and the row sums Sig of every token, and the final state of the second
+// scan only; y is stored by the second scan only.
+struct ChainGrad {
+  const float *S_in;       // state entering the scan, or null (zero)
+  float *S_out;            // state after it, or null
+  const float *rec;
+  float *y;                // null: not stored
+  float *bound, *sig;
+  int rev;
+};
+struct ChainArgs2 {
+  ChainGrad z[2];
+};
+struct NoChainArgs {};
+template <typename TY, int NQ, bool GRAD>
+__global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
+    float *S, const float *rec, TY *y, int T, int H,
+    std::conditional_t<GRAD, ChainArgs2, NoChainArgs> ga) {
   static_assert(NQ == 1 || NQ == 2, "one or two quarters per workgroup");
-  __shared__ float s_s[16 * NQ][kPad];  // the workgroup's state rows
+  __shared__ __align__(16) float s_s[16 * NQ][kXs];  // the workgroup's state rows
   __shared__ float s_xp[NQ][4][kCk][kCk + 1], s_yp[NQ][4][kCk][kCk + 1];  // per-block Sig^T / Y partials [t][i]
   // the ring, one object per slot
   __shared__ ChainSlot<NQ> s_rec0, s_rec1, s_rec2;
@@ -1159,19 +1265,46 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
   const int q = blockIdx.x % (4 / NQ) * NQ + qq;  // the quarter's value rows 16 q ..
   const int NC = (T + kCk - 1) / kCk, C = H * kN;
   // lane holds S[16 q + 4 kq + r][16 cb + row], r = 0..3 (the MFMA D layout)
-  float *Sp = S + (((int64_t)bi * H + h) * kN + 16 * q) * kN;
-  floatx4 st;
+  const int64_t soff = (((int64_t)bi * H + h) * kN + 16 * q) * kN + 4 * kq * kN + 16 * cb + row;
+  const float *S_in = S;
+  float *S_out = S, *bound = nullptr, *sig = nullptr;
+  int rev = 0;
+  if constexpr (GRAD) {
+    const ChainGrad &gz = ga.z[blockIdx.z];
+    S_in = gz.S_in;
+    S_out = gz.S_out;
+    rec = gz.rec;
+    y = gz.y;
+    bound = gz.bound + ((int64_t)bi * H + h) * NC * (kN * kN);
+    sig = gz.sig + (int64_t)bi * T * C;
+    rev = gz.rev;
+  }
+  floatx4 st = {0.f, 0.f, 0.f, 0.f};
+  if (!GRAD || S_in) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) st[r] = Sp[(4 * kq + r) * kN + 16 * cb + row];
+    for (int r = 0; r < 4; ++r) st[r] = S_in[soff + r * kN];
+  }
   // this (sequence, head)'s records, and this sequence's y, as buffers
   const i32x4 rr = buffer_words(rec + ((int64_t)bi * H + h) * NC * kRecFloats, NC * kRecFloats * 4);
-  const __amdgpu_buffer_rsrc_t yr =
-      __builtin_amdgcn_make_buffer_rsrc(y + (int64_t)bi * T * C, 0, (int)((int64_t)T * C * sizeof(TY)), 0x00020000);
+  // (a null y: a buffer of no bytes, every store dropped)
+  const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+      GRAD && !y ? reinterpret_cast<TY *>(sig) : y + (int64_t)bi * T * C, 0,
+      GRAD && !y ? 0 : (int)((int64_t)T * C * sizeof(TY)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t br =
+      __builtin_amdgcn_make_buffer_rsrc(bound, 0, GRAD ? NC * (kN * kN) * 4 : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(sig, 0, GRAD ? T * C * 4 : 0, 0x00020000);
+  // token of a step, out of range (and its stores dropped) for padding
+  auto token = [&](int i) { return GRAD && rev ? NC * kCk - 1 - i : i; };
   // the record piece that this wave fetches: U, V, Y0 of the workgroup's
   // quarters, then gam (repeated by the waves left over)
   const int q0 = q - qq;  // the workgroup's first quarter
   const int psrc = wv < NQ ? kRecU * 4 + (q0 + wv) * 1024 : wv < 2 * NQ ? kRecV * 4 + (q0 + wv - NQ) * 1024
-                 : wv < 3 * NQ ? kRecY0 * 4 + (q0 + wv - 2 * NQ) * 1024 : kRecGam * 4;
+                 : wv < 3 * NQ ? kRecY0 * 4 + (q0 + wv - 2 * NQ) * 64 : kRecGam * 4;
+  // byte offsets in a record of this lane's 16 bytes: of B^ or K^ in operand
+  // order, of G1 or G2 (row `row`, channels 16 cb + 4 kq ..), of the wave's piece
+  const int vfrag = (64 * cb + lane) * 16, vrow = (row * kN + 16 * cb + 4 * kq) * 4;
+  const bool py0 = wv >= 2 * NQ && wv < 3 * NQ;
+  const int vpiece = py0 ? psrc + (lane >> 2) * (kN * 4) + (lane & 3) * 16 : psrc + lane * 16;
   // Record of chunk c into a ring slot: block cb of G1, G2, B^, K^ and one
   // piece per wave (16 bytes per lane landing in lane order). Past the last
   // chunk the last one is loaded again (unused), so the count per step never
@@ -1185,26 +1318,29 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
 #pragma unroll
     for (int u = 0; u < 4 / NQ; ++u) {
       const int a = qq * (4 / NQ) + u;  // the waves of column block cb share its four arrays
-      dma16(rr, lds_addr(&sl.g[a][cb][0]), offs[a] * 4 + (64 * cb + lane) * 16, base);
+      dma16(rr, lds_addr(&sl.g[a][cb][0]), offs[a] * 4 + (a < 2 ? vrow : vfrag), base);
     }
     // one piece per wave into p5[wave] (past the record's end the buffer
     // returns zeros)
-    dma16(rr, lds_addr(&sl.p5[wv][0]), psrc + lane * 16, base);
+    dma16(rr, lds_addr(&sl.p5[wv][0]), vpiece, base);
   };
-  // Each step issues one record's DMAs and then one y store per wave; the
-  // prologue pairs each record with a y store that the buffer drops. So at
-  // the wait of chunk c's step exactly kVm memory operations were issued
-  // after chunk c's DMAs: the y stores of the kRing - 1 steps (or prologue
-  // entries) since, and the DMAs of the kRing - 2 records in between. The
-  // counter counts loads and stores in issue order, so waiting for at most
-  // kVm outstanding waits for chunk c's record and nothing later.
-  constexpr int kVm = kDmaPerWave * (kRing - 2) + (kRing - 1);
-  static_assert(kVm < 16, "vmcnt field (low bits only)");
-  constexpr int kWaitRec = 0x0F70 | kVm;
+  // Each step issues one record's DMAs and then kStores stores per wave (y;
+  // GRAD also Sig and four of the entering state); the prologue pairs each
+  // record with as many stores that the buffer drops. So at the wait of chunk
+  // c's step exactly kVm memory operations were issued after chunk c's DMAs:
+  // the stores of the kRing - 1 steps (or prologue entries) since, and the
+  // DMAs of the kRing - 2 records in between. The counter counts loads and
+  // stores in issue order, so waiting for at most kVm outstanding waits for
+  // chunk c's record and nothing later.
+  constexpr int kStores = GRAD ? 6 : 1;
+  constexpr int kVm = kDmaPerWave * (kRing - 2) + kStores * (kRing - 1);
+  static_assert(kVm < 64, "vmcnt field: bits 3..0 and 15..14");
+  constexpr int kWaitRec = 0x0F70 | (kVm & 15) | ((kVm >> 4) << 14);
 #pragma unroll
   for (int c = 0; c < kRing - 1; ++c) {
     dma(c, c);
-    store_y(yr, 0xFFFFFFF0u, from_f<TY>(0.f));  // past the buffer: dropped
+#pragma unroll
+    for (int u = 0; u < kStores; ++u) store_y(yr, 0xFFFFFFF0u, from_f<TY>(0.f));  // past the buffer: dropped
   }
   // slot: c % kRing, a constant in the unrolled loop below, so that every
   // slot address is a constant offset
@@ -1217,6 +1353,12 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
     // LDS stores (a memory fence would also wait for the DMAs still in flight)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     dma(c + kRing - 1, (slot + kRing - 1) % kRing);  // the slot of chunk c - 1: its readers passed the barrier
+    if constexpr (GRAD) {  // the state entering the chunk
+      const int ct = rev ? NC - 1 - c : c;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        store_y(br, (unsigned)((ct * kN + 16 * q + 4 * kq + r) * kN + 16 * cb + row) * 4u, (float)st[r]);
+    }
     const float4 g1 = sl.g[0][cb][lane], g2 = sl.g[1][cb][lane], kh = sl.g[3][cb][lane];
     const float4 vv = reinterpret_cast<const float4 *>(sl.p5[NQ + qq])[lane];
     const float G1[4] = {g1.x, g1.y, g1.z, g1.w}, G2[4] = {g2.x, g2.y, g2.z, g2.w};
@@ -1230,12 +1372,13 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) acc = mfma4(V[kk], KH[kk], acc);
     // Sig^T and Y over this wave's 16 key columns: D[t][i] = sum_j G[t][j] S[i][j]
+    const float4 s4 = *reinterpret_cast<const float4 *>(&s_s[16 * qq + row][16 * cb + 4 * kq]);
+    const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
     floatx4 xa = {0.f, 0.f, 0.f, 0.f}, ya = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const float sv = s_s[16 * qq + row][16 * cb + 4 * kk + kq];
-      xa = mfma4(G1[kk], sv, xa);
-      ya = mfma4(G2[kk], sv, ya);
+    for (int kk = 0; kk < 4; ++kk) {  // columns 16 cb + 4 kq + kk
+      xa = mfma4(G1[kk], sv[kk], xa);
+      ya = mfma4(G2[kk], sv[kk], ya);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1247,15 +1390,21 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
     const float4 bh = sl.g[2][cb][lane];
     const float4 u = reinterpret_cast<const float4 *>(sl.p5[qq])[lane];
     const float BH[4] = {bh.x, bh.y, bh.z, bh.w}, U[4] = {u.x, u.y, u.z, u.w};
+    float xv[4];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int t = 4 * kk + kq;
-      const float xv = ((s_xp[qq][0][t][row] + s_xp[qq][1][t][row]) + (s_xp[qq][2][t][row] + s_xp[qq][3][t][row])) + U[kk];
-      acc = mfma4(xv, BH[kk], acc);
+      xv[kk] = ((s_xp[qq][0][t][row] + s_xp[qq][1][t][row]) + (s_xp[qq][2][t][row] + s_xp[qq][3][t][row])) + U[kk];
+      acc = mfma4(xv[kk], BH[kk], acc);
     }
     st = acc;
+    if constexpr (GRAD) {  // Sig of token 4 cb + kq, value row 16 q + row (every block holds all of them)
+      const float sv1 = cb == 0 ? xv[0] : cb == 1 ? xv[1] : cb == 2 ? xv[2] : xv[3];
+      const int tt = token(c * kCk + 4 * cb + kq);
+      store_y(sr, tt < T ? (unsigned)(((int64_t)tt * C + h * kN + 16 * q + row) * 4) : 0xFFFFFFF0u, sv1);
+    }
     {  // y of token t, value row 16 q + i (past the sequence: dropped by the buffer)
-      const int lt = tid & 255, t = lt >> 4, i = lt & 15, tt = c * kCk + t;
+      const int lt = tid & 255, t = lt >> 4, i = lt & 15, tt = token(c * kCk + t);
       const float yv = ((s_yp[qq][0][t][i] + s_yp[qq][1][t][i]) + (s_yp[qq][2][t][i] + s_yp[qq][3][t][i])) + sl.p5[2 * NQ + qq][lt];
       const unsigned off = tt < T ? (unsigned)(((int64_t)tt * C + h * kN + 16 * q + i) * sizeof(TY)) : 0xFFFFFFF0u;
       store_y(yr, off, from_f<TY>(yv));
@@ -1267,8 +1416,10 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(float *S, co
       if (c0 + k < NC) step(c0 + k, k);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // the clamped DMAs land before the workgroup's LDS is reused
+  if (!GRAD || S_out) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) Sp[(4 * kq + r) * kN + 16 * cb + row] = st[r];
+    for (int r = 0; r < 4; ++r) S_out[soff + r * kN] = st[r];
+  }
 }
 
 template <class St, typename TY>
@@ -1286,9 +1437,9 @@ static int launch_chunked(const typename St::Args &p, float *S, TY *y, float *re
   // two value quarters per workgroup (each record fetched once for both)
   // where that still leaves a workgroup per CU
   if (2 * B * H >= (mk_cus() > 0 ? mk_cus() : 256))
-    wkv7_chunk_chain_kernel<TY, 2><<<dim3(2 * H, B), 512, 0, st>>>(S, rec, y, T, H);
+    wkv7_chunk_chain_kernel<TY, 2, false><<<dim3(2 * H, B), 512, 0, st>>>(S, rec, y, T, H, {});
   else
-    wkv7_chunk_chain_kernel<TY, 1><<<dim3(4 * H, B), 256, 0, st>>>(S, rec, y, T, H);
+    wkv7_chunk_chain_kernel<TY, 1, false><<<dim3(4 * H, B), 256, 0, st>>>(S, rec, y, T, H, {});
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;
 }
@@ -1308,6 +1459,195 @@ template int launch_wkv7_chunked<bf16_t, float, bf16_t>(const ScanArgs<bf16_t, f
 template int launch_wkv7_chunked<bf16_t, bf16_t, bf16_t>(const ScanArgs<bf16_t, bf16_t, bf16_t> &, float *,
                                                          hipStream_t);
 template int launch_wkv7_chunked<float, float, float>(const ScanArgs<float, float, float> &, float *, hipStream_t);
+
+// ---------------------------------------------------------------------------
+// Gradient of a sequence (training; launch_wkv7_grad). Two chunked scans at
+// once -- S forward and its adjoint backward in time (AdjStager) -- leave the
+// state S entering and the adjoint G' leaving every 16-token chunk, the row
+// sums sa = S a and G' b of every token, and gv. What remains per token,
+//   G_t = G'_t + gy_t r_t^T ;  gsa_t = G_t b_t = G'_t b_t + gy_t (r_t . b_t) ;
+//   gr = S_t^T gy ;  gk = G_t^T v ;  gw = diag(G_t^T S_{t-1}) ;
+//   gb = G_t^T sa ;  ga = S_{t-1}^T gsa,
+// are sums over the rows of a head, and no chunk waits for another:
+// wkv7_grad_kernel, one workgroup per (chunk, head, sequence). Lane = key
+// column, wave = 8 rows, so the states are advanced by two products with
+// scalars per element (v, sa, gy, gsa of a row are wave-uniform: LDS
+// broadcasts; as scalar loads, one memory round trip per token, the kernel
+// took 154 us at B = 4, T = 512, H = 16) and the column sums run inside a lane; the eight waves' partial sums
+// meet in LDS, four tokens at a time. The states of 8 tokens stay in
+// registers, so a chunk runs as two halves, the later one first (its entering
+// state recomputed from the chunk's). Bound by its VALU work: 11 operations
+// per token and state element, three of them the recomputation.
+// Measured at B = 4, T = 512, H = 16 (2048 chunks): 80 us, 184 MB moved; with
+// 129 registers, one workgroup per CU instead of two, 110 us. With the two
+// prep launches (23 + 25 us, 4.7 TB/s of inputs and records) and the chain
+// (62 us) the gradient takes 190 us there; the history-recording scan and the
+// reverse scan over it took 110 + 2887 us.
+// ---------------------------------------------------------------------------
+struct GradArgs {
+  const float *r, *w, *k, *v, *a, *b, *gy;
+  const float *sbound, *gbound;  // [B, H, chunk, 64, 64]: S entering, G' leaving
+  const float *sa, *gsig;        // [B, T, H, 64]: S a, G' b
+  float *gr, *gw, *gk, *ga, *gb;
+  int B, T, H;
+};
+constexpr int kGradRows = 8, kGradHalf = 8, kGradBatch = 4;
+__global__ __launch_bounds__(512, 4) void wkv7_grad_kernel(GradArgs p) {
+  __shared__ __align__(16) float s_c[9][kCk][kN];     // r, w, k, a, b (columns); v, gy, sa, G' b (rows)
+  __shared__ float s_part[kGradBatch][8][5][kN];      // [token][wave][gr, gw, gk, ga, gb]
+  __shared__ float s_rb[kCk];                         // r . b
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = blockIdx.x, h = blockIdx.y, bi = blockIdx.z;
+  const int T = p.T, H = p.H, C = H * kN, NC = gridDim.x;
+  const int t0 = c * kCk, nt = min(kCk, T - t0);
+  const int64_t tok0 = ((int64_t)bi * T + t0) * C + (int64_t)h * kN;  // token t0, channel 0 of the head
+  const int64_t sb = (((int64_t)bi * H + h) * NC + c) * (kN * kN) + kGradRows * wv * kN + lane;
+  float S0[kGradRows], G[kGradRows];
+#pragma unroll
+  for (int e = 0; e < kGradRows; ++e) {
+    S0[e] = p.sbound[sb + e * kN];
+    G[e] = p.gbound[sb + e * kN];
+  }
+  {
+    // thread -> token, float4; two arrays at a time over the 512 threads
+    const float *const src[9] = {p.r, p.w, p.k, p.a, p.b, p.v, p.gy, p.sa, p.gsig};
+    const int t = tid >> 4 & 15, q = tid & 15;
+    const int64_t o = tok0 + (int64_t)min(t, nt - 1) * C + 4 * q;
+    float4 x[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      const float *s = tid < 256 || i == 4 ? src[2 * i] : src[i < 4 ? 2 * i + 1 : 8];
+      x[i] = *reinterpret_cast<const float4 *>(s + o);
+    }
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      if (i < 4 || tid < 256) *reinterpret_cast<float4 *>(&s_c[i < 4 && tid >= 256 ? 2 * i + 1 : 2 * i][t][4 * q]) = x[i];
+  }
+  __syncthreads();
+  {
+    const float2 d = wave_sum2(s_c[0][2 * wv][lane] * s_c[4][2 * wv][lane],
+                               s_c[0][2 * wv + 1][lane] * s_c[4][2 * wv + 1][lane]);
+    if (lane == 0) {
+      s_rb[2 * wv] = d.x;
+      s_rb[2 * wv + 1] = d.y;
+    }
+  }
+  __syncthreads();
+  // this wave's eight rows of row array i at a token (LDS broadcasts)
+  struct Rows {
+    float x[kGradRows];
+  };
+  auto rows = [&](int i, int t) {
+    const float4 *q = reinterpret_cast<const float4 *>(&s_c[i][t][kGradRows * wv]);
+    const float4 u = q[0], z = q[1];
+    return Rows{{u.x, u.y, u.z, u.w, z.x, z.y, z.z, z.w}};
+  };
+  auto advance = [&](float (&S)[kGradRows], int t) {
+    const float w = s_c[1][t][lane], k = s_c[2][t][lane], b = s_c[4][t][lane];
+    const Rows sa = rows(7, t), v = rows(5, t);
+#pragma unroll
+    for (int e = 0; e < kGradRows; ++e) S[e] = fmaf(sa.x[e], b, fmaf(v.x[e], k, S[e] * w));
+  };
+  float *const dst[5] = {p.gr, p.gw, p.gk, p.ga, p.gb};
+  // tokens tb .. tb + 7 of the chunk (those below nt), entered with S
+  auto half = [&](float (&S)[kGradRows], int tb) {
+    float hist[kGradHalf][kGradRows];
+#pragma unroll
+    for (int t = 0; t < kGradHalf; ++t) {
+#pragma unroll
+      for (int e = 0; e < kGradRows; ++e) hist[t][e] = S[e];
+      if (tb + t < nt) advance(S, tb + t);
+    }
+#pragma unroll
+    for (int t = kGradHalf - 1; t >= 0; --t) {
+      if (tb + t < nt) {
+        const int tt = tb + t;
+        const float r = s_c[0][tt][lane], w = s_c[1][tt][lane], a = s_c[3][tt][lane], rb = s_rb[tt];
+        const Rows gy = rows(6, tt), v = rows(5, tt), sa = rows(7, tt), gs = rows(8, tt);
+        float pr = 0.f, pw = 0.f, pk = 0.f, pa = 0.f, pb = 0.f;
+#pragma unroll
+        for (int e = 0; e < kGradRows; ++e) {
+          const float gsa = fmaf(gy.x[e], rb, gs.x[e]);
+          const float g = fmaf(gy.x[e], r, G[e]);
+          pr = fmaf(S[e], gy.x[e], pr);
+          pw = fmaf(g, hist[t][e], pw);
+          pk = fmaf(g, v.x[e], pk);
+          pb = fmaf(g, sa.x[e], pb);
+          pa = fmaf(hist[t][e], gsa, pa);
+          G[e] = fmaf(gsa, a, g * w);
+          S[e] = hist[t][e];
+        }
+        float(*o)[kN] = s_part[t % kGradBatch][wv];
+        o[0][lane] = pr;
+        o[1][lane] = pw;
+        o[2][lane] = pk;
+        o[3][lane] = pa;
+        o[4][lane] = pb;
+      }
+      if (t % kGradBatch == 0) {  // tokens tb + t .. + 3 are in LDS
+        __syncthreads();
+        for (int e = tid; e < kGradBatch * 5 * kN; e += 512) {
+          const int u = e / (5 * kN), q = e / kN % 5, j = e % kN;
+          if (tb + t + u < nt) {
+            float x = 0.f;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) x += s_part[u][w][q][j];
+            float *d = q == 0 ? dst[0] : q == 1 ? dst[1] : q == 2 ? dst[2] : q == 3 ? dst[3] : dst[4];
+            d[tok0 + (int64_t)(tb + t + u) * C + j] = x;
+          }
+        }
+        __syncthreads();
+      }
+    }
+  };
+  float S[kGradRows];
+  if (nt > kGradHalf) {
+#pragma unroll
+    for (int e = 0; e < kGradRows; ++e) S[e] = S0[e];
+    for (int t = 0; t < kGradHalf; ++t) advance(S, t);
+    half(S, kGradHalf);
+  }
+#pragma unroll
+  for (int e = 0; e < kGradRows; ++e) S[e] = S0[e];
+  half(S, 0);
+}
+
+// floats of the workspace: two sets of chunk records, the two scans' boundary
+// states and row sums
+int64_t wkv7_grad_ws_bytes(int B, int T, int H) {
+  const int64_t nc = (T + kCk - 1) / kCk, bh = (int64_t)B * H;
+  return 4 * (2 * bh * nc * (kRecFloats + kN * kN) + 2 * bh * T * kN);
+}
+
+int launch_wkv7_grad(const Wkv7GradArgs &p, float *ws, hipStream_t st) {
+  if (p.T <= 0 || p.B <= 0 || p.H <= 0) return RWKV7_OK;
+  if (!chunk_offsets_fit(p.T, p.H, 4)) return RWKV7_ESHAPE;
+  const int nc = (p.T + kCk - 1) / kCk;
+  const int64_t bh = (int64_t)p.B * p.H, recf = bh * nc * kRecFloats, bnd = bh * nc * kN * kN, tok = bh * p.T * kN;
+  float *rec_f = ws, *rec_b = rec_f + recf, *sbound = rec_b + recf, *gbound = sbound + bnd, *sa = gbound + bnd,
+        *gsig = sa + tok;
+  const dim3 grid(nc, p.H, p.B);
+  using Fwd = RawStager<kCk, float, float, float>;
+  using Adj = AdjStager<kCk>;
+  const typename Fwd::Args fa = {nullptr, p.r, p.k, p.v, p.a, p.b, p.w, nullptr, p.B, p.T, p.H};
+  const typename Adj::Args aa = {p.r, p.w, p.k, p.a, p.b, p.gy, p.B, p.T, p.H};
+  wkv7_chunk_prep_kernel<Fwd, false><<<grid, 256, 0, st>>>(fa, rec_f, p.T, p.H);
+  RWKV7_CHECK_LAUNCH();
+  wkv7_chunk_prep_kernel<Adj, false><<<grid, 256, 0, st>>>(aa, rec_b, p.T, p.H);
+  RWKV7_CHECK_LAUNCH();
+  const ChainArgs2 ch = {{{p.S0, nullptr, rec_f, nullptr, sbound, sa, 0}, {p.gS_T, p.gS0, rec_b, p.gv, gbound, gsig, 1}}};
+  // as launch_chunked, with both scans' workgroups counted
+  if (4 * p.B * p.H >= (mk_cus() > 0 ? mk_cus() : 256))
+    wkv7_chunk_chain_kernel<float, 2, true><<<dim3(2 * p.H, p.B, 2), 512, 0, st>>>(nullptr, nullptr, nullptr, p.T, p.H, ch);
+  else
+    wkv7_chunk_chain_kernel<float, 1, true><<<dim3(4 * p.H, p.B, 2), 256, 0, st>>>(nullptr, nullptr, nullptr, p.T, p.H, ch);
+  RWKV7_CHECK_LAUNCH();
+  const GradArgs g = {p.r, p.w, p.k, p.v, p.a, p.b, p.gy, sbound, gbound, sa, gsig, p.gr, p.gw, p.gk, p.ga, p.gb,
+                      p.B, p.T, p.H};
+  wkv7_grad_kernel<<<grid, 512, 0, st>>>(g);
+  RWKV7_CHECK_LAUNCH();
+  return RWKV7_OK;
+}
 
 int launch_wkv7_prefill(const PrefillScanArgs &p, hipStream_t st) {
   if (p.T <= 0 || p.B <= 0 || p.H <= 0) return RWKV7_OK;

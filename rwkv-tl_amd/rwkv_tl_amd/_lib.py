@@ -49,6 +49,9 @@ SYMBOLS = (
     "rwkv7_wkv7_chunked",
     "rwkv7_wkv7_f32",
     "rwkv7_wkv7_backward",
+    "rwkv7_wkv7_f32_chunked",
+    "rwkv7_wkv7_grad_workspace_bytes",
+    "rwkv7_wkv7_grad",
     "rwkv7_layernorm",
     "rwkv7_lerp",
     "rwkv7_gemv_f16",
@@ -174,6 +177,9 @@ def _declare(lib: ctypes.CDLL) -> None:
         "rwkv7_wkv7_chunked": (ctypes.c_int, [vp, vp, vp, i32, vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, i64, vp]),
         "rwkv7_wkv7_f32": (ctypes.c_int, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp]),
         "rwkv7_wkv7_backward": (ctypes.c_int, [vp] * 17 + [i32, i32, i32, vp]),
+        "rwkv7_wkv7_f32_chunked": (ctypes.c_int, [vp] * 8 + [i32, i32, i32, vp, i64, vp]),
+        "rwkv7_wkv7_grad_workspace_bytes": (i64, [i32, i32, i32]),
+        "rwkv7_wkv7_grad": (ctypes.c_int, [vp] * 16 + [i32, i32, i32, vp, i64, vp]),
         "rwkv7_layernorm": (ctypes.c_int, [vp, i32, vp, vp, vp, i32, i32, i32, vp]),
         "rwkv7_lerp": (ctypes.c_int, [vp, vp, vp, i32, vp, vp, i32, i32, vp]),
         "rwkv7_gemv_f16": (ctypes.c_int, [vp, vp, i64, vp, i32, i32, i32, vp]),

@@ -69,19 +69,21 @@ def _h16(*ts: Tensor) -> int:
     return int(dt == torch.bfloat16)
 
 
-# The operator takes the chunked scan for sequences at least this long when
-# the serial scan's 4 workgroups per head and sequence would leave CUs idle
-# (measured on MI355X: B=1, H=16, T=128 faster chunked; the survey's C2,
-# B=8, H=16, T=128, faster serial).
-CHUNK_MIN_T = 32
-_CUS: dict[int, int] = {}
+# The operators take the chunked scan for sequences at least this long
+# (measured on MI355X, us per call, serial / chunked: B=1, H=16, T=64 14.9 /
+# 19.2, T=128 21.4 / 19.1; B=8, H=16, T=64 15.4 / 20.5, T=128 28.1 / 24.4;
+# B=16, H=32, T=128 102 / 74, T=1024 840 / 539).
+CHUNK_MIN_T = 128
 
 
-def _cus(dev: torch.device) -> int:
-    i = dev.index if dev.index is not None else torch.cuda.current_device()
-    if i not in _CUS:
-        _CUS[i] = torch.cuda.get_device_properties(i).multi_processor_count
-    return _CUS[i]
+def _chunk_fits(T: int, H: int) -> bool:
+    """Whether a sequence's chunk records (28,928 bytes per 16 tokens and
+    head) and its f32 outputs stay inside the chunked kernels' 32-bit offsets."""
+    return T <= 1 << 20 and T * H * N * 4 < 2**31 - 1
+
+
+def _chunk_pays(Bsz: int, T: int, H: int) -> bool:
+    return T >= CHUNK_MIN_T and _chunk_fits(T, H)
 
 
 def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Tensor,
@@ -92,8 +94,7 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
     dtype or f32. Returns ``y`` [B, T, H, 64] of r's dtype with ``y_t = S_t r_t``.
     ``chunked``: run the chunked (MFMA) algorithm, ``rwkv7_wkv7_chunked``,
     with a workspace allocated per call, or the serial scan ``rwkv7_wkv7``;
-    ``None`` chooses the chunked one for ``T >= CHUNK_MIN_T`` when
-    ``4 B H`` is below the device's CU count.
+    ``None`` chooses the chunked one for ``T >= CHUNK_MIN_T``.
     """
     _dev(S, r, w, k, v, a, b)
     _need(S.dtype == torch.float32 and S.dim() == 4 and S.shape[2:] == (N, N), "S must be f32 [B,H,64,64]")
@@ -110,7 +111,7 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
     args = (S.data_ptr(), r.data_ptr(), w.data_ptr(), int(w.dtype == torch.float32), k.data_ptr(), v.data_ptr(),
             a.data_ptr(), b.data_ptr(), y.data_ptr(), Bsz, T, H, bf)
     if chunked is None:
-        chunked = T >= CHUNK_MIN_T and 4 * Bsz * H < _cus(S.device)
+        chunked = _chunk_pays(Bsz, T, H)
     if chunked:
         nb = int(lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H))
         ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
@@ -175,24 +176,50 @@ def dplr_seq_forward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: T
     batched = S.dim() == 4
     S1 = (S if batched else S.unsqueeze(0)).contiguous().clone()
     ins = [(x if batched else x.unsqueeze(0)).contiguous() for x in (R, W, K, V, A, B)]
-    y = wkv7_f32(S1, ins[0], ins[1], ins[2], ins[3], ins[4], ins[5])
+    _dev(S1, *ins)
+    Bsz, T, H = _wkv7_f32_shapes(S1, *ins)
+    if _chunk_pays(Bsz, T, H):
+        y = torch.empty_like(ins[0])
+        lib = _lib.load()
+        nb = int(lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H))
+        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+        _lib.check(lib.rwkv7_wkv7_f32_chunked(S1.data_ptr(), *(x.data_ptr() for x in ins), y.data_ptr(), Bsz, T, H,
+                                              ws.data_ptr(), nb, _lib.stream_handle()), "rwkv7_wkv7_f32_chunked")
+    else:
+        y = wkv7_f32(S1, *ins)
     return (y, S1) if batched else (y[0], S1[0])
 
 
 def dplr_seq_backward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: Tensor, B: Tensor,
                       gy: Tensor, gS: Tensor | None) -> tuple[Tensor, ...]:
-    """Gradients of ``dplr_seq_forward`` w.r.t. ``(S, R, W, K, V, A, B)``:
-    the forward is run again to record the per-step states (the reference's
-    plan, TODO.md:46-54), then the reverse-time scan."""
+    """Gradients of ``dplr_seq_forward`` w.r.t. ``(S, R, W, K, V, A, B)`` from
+    its inputs (the reference's plan, TODO.md:46-54, recomputes the states
+    too): chunked scans of the states and of their adjoint, then every chunk at
+    once (``rwkv7_wkv7_grad``)."""
     batched = S.dim() == 4
     u = (lambda x: x) if batched else (lambda x: x.unsqueeze(0))
-    S1 = u(S).contiguous().clone()
+    S1 = u(S).contiguous()
     ins = [u(x).contiguous() for x in (R, W, K, V, A, B)]
-    Bsz, H = S1.shape[:2]
-    T = ins[0].shape[1]
-    hist = torch.empty(Bsz, H, T, N, N, dtype=torch.float32, device=S.device)
-    wkv7_f32(S1, *ins, hist=hist)
-    out = wkv7_backward(hist, S1, *ins, u(gy).contiguous(), None if gS is None else u(gS).contiguous())
+    gy = u(gy).contiguous()
+    gS = None if gS is None else u(gS).contiguous()
+    _dev(S1, *ins, gy)
+    Bsz, T, H = _wkv7_f32_shapes(S1, *ins, gy)
+    if not _chunk_fits(T, H):
+        S1 = S1.clone()
+        hist = torch.empty(Bsz, H, T, N, N, dtype=torch.float32, device=S.device)
+        wkv7_f32(S1, *ins, hist=hist)
+        out = wkv7_backward(hist, S1, *ins, gy, gS)
+    else:
+        if gS is not None:
+            _dev(gS)
+            _need(gS.shape == S1.shape and gS.dtype == torch.float32, "gS must be like S")
+        out = (torch.empty_like(S1), *(torch.empty_like(x) for x in ins))
+        lib = _lib.load()
+        nb = int(lib.rwkv7_wkv7_grad_workspace_bytes(Bsz, T, H))
+        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+        rc = lib.rwkv7_wkv7_grad(S1.data_ptr(), *(x.data_ptr() for x in ins), gy.data_ptr(), _lib.ptr(gS),
+                                 *(g.data_ptr() for g in out), Bsz, T, H, ws.data_ptr(), nb, _lib.stream_handle())
+        _lib.check(rc, "rwkv7_wkv7_grad")
     return out if batched else tuple(g[0] for g in out)
 
 

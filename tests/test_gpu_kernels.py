@@ -550,3 +550,49 @@ def test_dplr_seq_operator_autograd(cuda):
     ref = R.wkv7_scan_grads(S, r, w, k, v, a, b, gy.unsqueeze(0), gS.unsqueeze(0))
     for name, x, xr in zip(("S0", "r", "w", "k", "v", "a", "b"), xs, ref):
         assert _rel(x.grad.cpu(), xr[0]) < 2e-4, f"grad {name}"
+
+
+@pytest.mark.parametrize("B,T,H,with_gS,decay", [
+    (1, 1, 1, True, "plain"), (1, 15, 2, False, "plain"), (2, 16, 1, True, "plain"), (1, 17, 3, True, "plain"),
+    (1, 24, 1, True, "plain"), (2, 129, 2, True, "plain"), (1, 40, 2, True, "strong"), (1, 33, 1, False, "zero"),
+])
+def test_dplr_seq_gradient_matches_oracle(B, T, H, with_gS, decay, cuda):
+    """dplr_seq_forward / dplr_seq_backward (chunked scans of the state and of
+    its adjoint, then every 16-token chunk at once) against the oracle's
+    autograd gradients in fp32, around the chunk (16) and half-chunk (8)
+    edges, for two workgroup sizes of the chains, and with decays whose
+    products leave the range the scaled form is used in (strong: w^40, products
+    below 1e-30 in a chunk; zero: some w = 0). Both sides sum the same fp32
+    terms in another order: relative rounding of at most T + 64 ulps (1.2e-7
+    each) in the worst case, 1e-5 at these sizes."""
+    S, r, w, k, v, a, b = _dplr_inputs(B, T, H, seed=31 * T + H)
+    g = torch.Generator().manual_seed(11)
+    if decay == "strong":
+        w = w**40
+    elif decay == "zero":
+        w = torch.where(torch.rand(w.shape, generator=g) < 0.05, torch.zeros_like(w), w)
+    gy = torch.randn(B, T, H, 64, generator=g)
+    gS = torch.randn(B, H, 64, 64, generator=g) if with_gS else None
+    y_ref, S_ref = R.wkv7_scan(S, r, w, k, v, a, b)
+    ref = R.wkv7_scan_grads(S, r, w, k, v, a, b, gy, gS)
+    d = [x.to(cuda) for x in (S, r, w, k, v, a, b)]
+    y, S_T = K.dplr_seq_forward(*d)
+    assert _rel(y.cpu(), y_ref) < 1e-5 and _rel(S_T.cpu(), S_ref) < 1e-5
+    got = K.dplr_seq_backward(*d, gy.to(cuda), None if gS is None else gS.to(cuda))
+    assert torch.equal(d[0].cpu(), S)
+    for name, x, xr in zip(("S0", "r", "w", "k", "v", "a", "b"), got, ref):
+        assert _rel(x.cpu(), xr) < 1e-5, f"grad {name}: rel {_rel(x.cpu(), xr):.2e}"
+
+
+def test_dplr_seq_gradient_many_heads_matches_history_backward(cuda):
+    """A grid of more heads than CUs (two value quarters per chain workgroup)
+    against the history-based backward (rwkv7_wkv7_backward) on the same
+    device; both fp32, 1e-5 as above."""
+    d = [x.to(cuda) for x in _dplr_inputs(3, 50, 24, seed=77)]
+    gy = torch.randn(3, 50, 24, 64, device=cuda)
+    S1 = d[0].clone()
+    hist = torch.empty(3, 24, 50, 64, 64, device=cuda)
+    K.wkv7_f32(S1, *d[1:], hist=hist)
+    want = K.wkv7_backward(hist, S1, *d[1:], gy, None)
+    for x, xr in zip(K.dplr_seq_backward(*d, gy, None), want):
+        assert _rel(x, xr) < 1e-5
