@@ -784,11 +784,10 @@ static int launch_big(const GemmProb *probs, int nprob, int M, int cus, hipStrea
 // ---------------------------------------------------------------------------
 constexpr int kSkW = 4;           // waves per workgroup
 constexpr int kSkinnyMaxM = 32;   // M up to this runs the skinny path
-// with f32 A only up to 8 rows: from 9 rows the 16-row tiles are faster
-// (measured: 0.4B prefill 1 x 32 1.37 vs 1.68 ms, decode B = 32 1.28 vs
+// with f32 A only up to kA32SkinnyMaxM rows: from 9 rows the 16-row tiles are
+// faster (measured: 0.4B prefill 1 x 32 1.37 vs 1.68 ms, decode B = 32 1.28 vs
 // 1.59 ms/step, the 1.5B shape at B = 32 2.08 vs 3.24 and B = 16 1.77 vs
 // 2.18 ms/step; at 2 and 4 rows the skinny strips are 5-7 % faster)
-constexpr int kA32SkinnyMaxM = 8;
 
 struct SkinnyGroup {
   GemmProb p[kMaxProb];

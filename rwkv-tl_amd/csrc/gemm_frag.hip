@@ -1,0 +1,361 @@
+// MFMA GEMM on fragment-ordered operands: Y = epi(A W^T) for steps of 9 rows
+// up to the large-M path with f32-grade activations.
+//
+// Both operands are stored as MFMA reads them, in 16-row x 32-k blocks of one
+// contiguous KiB per 64-lane load: W in the model's fragment arena, A in split
+// order (split_put8) by the kernels that produce it: the activations' 16-bit
+// parts and their 16-bit remainders (split_hi_lo's two values). So a wave loads
+// both operands straight into MFMA registers, and the main loop is loads and
+// MFMAs: no LDS, no conversion, no barrier until the waves' partial tiles meet.
+//
+// At these sizes (M up to ~2000) a product is neither MFMA- nor HBM-bound but
+// bound by the operand bytes that each CU pulls through its L1 (64 bytes per
+// cycle) and by the round trips in a workgroup's life. The tiled kernels of
+// gemm.hip (16 or 32 rows x 64 columns, A split and staged through LDS) moved
+// more bytes per product and waited for load, LDS and product phases in turn.
+// Here 8 waves share a tile as SM x SN sub-tiles of MB x NB blocks and SK
+// slices of K: few rows take a small tile with K split over the eight waves
+// (every load of the tile in flight at once), many rows a larger tile that
+// reuses each byte more. The K slices' partials are summed in LDS in slice
+// order, where the accumulator layout also becomes rows for vector stores.
+#include "rwkv7_kernels.h"
+
+namespace rwkv7 {
+
+constexpr int kFragProbs = 8;
+constexpr int kFragThreads = 512;
+
+struct FragGroup {
+  GemmProb p[kFragProbs];
+  int wg_begin[kFragProbs + 1];  // first workgroup of each problem
+  int nprob, M, m_tiles;
+  // K cut into `splits` (a power of two), each slice's f32 partial product
+  // stored at Y + slice * part_stride floats: the next stage sums them
+  int splits;
+  int64_t part_stride;
+};
+
+// The epilogue's value for one element (the add epilogue reads Y elsewhere).
+RWKV7_DEV float frag_epi(int epi, float v) {
+  switch (epi) {
+    case GEPI_RELUSQ_F32:
+    case GEPI_RELUSQ_SPLIT: {
+      const float q = fmaxf(v, 0.f);
+      return q * q;
+    }
+    case GEPI_TANH_F32:
+    case GEPI_TANH_SPLIT: return tanhf(v);
+    case GEPI_SIGM_F32:
+    case GEPI_SIGM_SPLIT: return sigmoidf_(v);
+    default: return v;
+  }
+}
+
+// Workgroup order as in gemm.hip: the m-tiles of a column tile get indices 8
+// apart, so they run on one XCD and read W from its L2.
+template <int MB, int NB, int SM, int SN, int SK, int KB, bool BF>
+__global__ __launch_bounds__(kFragThreads) void gemm_frag_kernel(FragGroup g) {
+  constexpr int BM = 16 * MB * SM, BN = 16 * NB * SN, LD = BN + 4;
+  constexpr int UPT = BM * BN / 4 / kFragThreads;  // 4-column output pieces per thread
+  constexpr int PPT = UPT > 0 ? UPT : 1;
+  static_assert(SM * SN * SK * 64 == kFragThreads, "eight waves");
+  __shared__ __align__(16) float s_red[SK][BM][LD];
+
+  const int bx = blockIdx.x;
+  int pi = 0;
+#pragma unroll
+  for (int i = 1; i < kFragProbs; ++i) pi += (i < g.nprob && bx >= g.wg_begin[i]);
+  const GemmProb &P = g.p[pi];
+  const int local = bx - g.wg_begin[pi], mtl = g.m_tiles;
+  const int unit = local / (8 * mtl) * 8 + (local & 7), mt = local % (8 * mtl) / 8;
+  const int N = P.N, M = g.M, S = g.splits;
+  const int nt = unit / S, split = unit & (S - 1);
+  if (nt * BN >= N) return;  // padding of the last group of 8 units
+  const int m0 = mt * BM, n0 = nt * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wv % SM, wn = wv / SM % SN, wk = wv / (SM * SN);
+
+  // operand blocks (rows and columns past the matrices are clamped to their
+  // last block: products nobody stores)
+  const int nks = (P.K + 31) / 32, per = (nks + SK * S - 1) / (SK * S);
+  const int k0 = (split * SK + wk) * per, len = max(0, min(nks, k0 + per) - k0);
+  // each wave and row tile starts elsewhere in its slice, so that the tiles of
+  // a column do not ask for the same lines at once (128 rows of 3360 x 1024
+  // 8.6 -> 7.7 us, 4096 x 1024 9.7 -> 8.6 us)
+  const int rot = len > 0 ? (3 * mt + wv) % len : 0;
+  const uint16_t *pa[MB], *pw[NB];
+  const int mblk = (M + 15) / 16, nstrip = (N + 15) / 16;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+    pa[i] = P.A + (int64_t)min(m0 / 16 + wm * MB + i, mblk - 1) * nks * 1024 + lane * 8;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) pw[j] = P.Wf + (int64_t)min(n0 / 16 + wn * NB + j, nstrip - 1) * P.nksf * 512 + lane * 8;
+
+  uint4 a[2][KB][MB][2], w[2][KB][NB];
+  auto load = [&](int k, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      int kk = min(k + b, len - 1) + rot;  // clamped: never multiplied past the slice
+      kk = kk >= len ? kk - len : kk;
+      kk = min(max(kk + k0, 0), nks - 1);  // (an empty slice loads something valid)
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        a[buf][b][i][0] = *reinterpret_cast<const uint4 *>(pa[i] + (int64_t)kk * 1024);
+        a[buf][b][i][1] = *reinterpret_cast<const uint4 *>(pa[i] + (int64_t)kk * 1024 + 512);
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) w[buf][b][j] = *reinterpret_cast<const uint4 *>(pw[j] + (int64_t)kk * 512);
+    }
+  };
+  floatx4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int k, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      if (k + b < len) {
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = mfma16<BF>(a[buf][b][i][pl], w[buf][b][j], acc[i][j]);
+      }
+    }
+  };
+  load(0, 0);
+  load(KB, 1);
+  // the values an add epilogue accumulates into, behind the first operands
+  float4 yres[PPT];
+  const bool add = P.epi == GEPI_ADD_F32;
+  auto piece = [&](int u, int &row, int &col) {
+    const int e = tid + kFragThreads * u;
+    row = e / (BN / 4);
+    col = 4 * (e % (BN / 4));
+    return e < BM * BN / 4;
+  };
+  if (add) {
+#pragma unroll
+    for (int u = 0; u < PPT; ++u) {
+      int row, col;
+      piece(u, row, col);
+      yres[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(P.Y) +
+                                                  (int64_t)min(m0 + row, M - 1) * P.ldy + min(n0 + col, N - 4));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  for (int k = 0; k < len; k += 2 * KB) {
+    compute(k, 0);
+    load(k + 2 * KB, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(k + KB, 1);
+    load(k + 3 * KB, 1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // lane holds rows 4 (lane >> 4) + r of column lane & 15 of each block
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        s_red[wk][16 * (wm * MB + i) + 4 * (lane >> 4) + r][16 * (wn * NB + j) + (lane & 15)] = acc[i][j][r];
+  __syncthreads();
+  const int epi = P.epi;
+  if (epi >= GEPI_SPLIT) {
+    // the next product's A: a wave per 16 x 32 block of the tile, one
+    // contiguous KiB per part; columns up to the next k-step are zeros
+    constexpr int NBLK = BM / 16 * (BN / 32);
+#pragma unroll
+    for (int q = 0; q < (NBLK + 7) / 8; ++q) {
+      const int blk = wv + 8 * q, row = 16 * (blk / (BN / 32)) + (lane & 15), col = 32 * (blk % (BN / 32)) + 8 * (lane >> 4);
+      const int m = m0 + row, n = n0 + col;
+      if (blk >= NBLK || m >= M || n >= (N + 31) / 32 * 32) continue;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll
+      for (int s = 0; s < SK; ++s) {
+        const float4 x = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
+        const float4 y = *reinterpret_cast<const float4 *>(&s_red[s][row][col + 4]);
+        v[0] += x.x;
+        v[1] += x.y;
+        v[2] += x.z;
+        v[3] += x.w;
+        v[4] += y.x;
+        v[5] += y.y;
+        v[6] += y.z;
+        v[7] += y.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = n + e < N ? frag_epi(epi, v[e]) : 0.f;
+      split_put8<BF>(static_cast<uint16_t *>(P.Y), (N + 31) / 32, m, n, v);
+    }
+    return;
+  }
+  const bool vec = N % 4 == 0 && P.ldy % 4 == 0;
+#pragma unroll
+  for (int u = 0; u < PPT; ++u) {
+    int row, col;
+    if (!piece(u, row, col)) continue;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < SK; ++s) {
+      const float4 q = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
+      v[0] += q.x;
+      v[1] += q.y;
+      v[2] += q.z;
+      v[3] += q.w;
+    }
+    const int m = m0 + row, n = n0 + col;
+    if (m >= M) continue;
+    if (n >= N) continue;
+    const int64_t o = (int64_t)m * P.ldy + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = frag_epi(epi, v[e]);
+    if (epi == GEPI_F16) {
+      uint16_t *y = static_cast<uint16_t *>(P.Y) + o;
+      uint16_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = F16T<BF>::from_f(v[e]);
+      if (vec) {
+        *reinterpret_cast<uint2 *>(y) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) y[e] = h[e];
+      }
+    } else {
+      float *y = static_cast<float *>(P.Y) + split * g.part_stride + o;
+      if (add) {
+        v[0] += yres[u].x;
+        v[1] += yres[u].y;
+        v[2] += yres[u].z;
+        v[3] += yres[u].w;
+      }
+      if (vec) {
+        *reinterpret_cast<float4 *>(y) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) y[e] = v[e];
+      }
+    }
+  }
+}
+
+// Tiles, smallest first.
+struct FragTile {
+  int bm, bn;
+};
+constexpr FragTile kFragTiles[] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {32, 128}, {64, 128}};
+constexpr int kFragNumTiles = 6;
+
+static int64_t frag_units(const FragTile &t, int M, int N) {
+  return (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+}
+
+// The smallest tile whose workgroups all run at once (one per CU): a larger
+// one leaves CUs idle, a smaller one moves more bytes per CU and runs in
+// rounds (measured, us, 0.4B FFN key 4096 x 1024: 64 rows 32 x 32 7.9, 16 x 32
+// 8.9, 32 x 64 8.7; 128 rows 32 x 64 9.1, 32 x 32 11.9, 64 x 64 11.4; 512 rows
+// 64 x 128 16.1, 64 x 64 18.4; FFN value's and the 1.5B sizes order alike).
+// Where none fits at once the largest, with as few rows as M has
+// (an eighth more than the CUs still passes: two of the smaller tiles fit on
+// one).
+static int frag_tile(const GemmProb *probs, int nprob, int M, int cus) {
+  for (int i = 0; i < kFragNumTiles; ++i) {
+    if (i == 4 && M > 32) continue;
+    int64_t n = 0;
+    for (int q = 0; q < nprob; ++q) n += frag_units(kFragTiles[i], M, probs[q].N);
+    if (n <= cus + (i < 4 ? cus / 8 : 0)) return i;
+  }
+  return M <= 32 ? 4 : 5;
+}
+
+// K slices of a product whose partials the next stage can sum. Few rows and a
+// long K leave each CU a small tile with all of K: its operands' bytes are the
+// time. Cutting K lets the tiles be larger; the (tile, slices) with the fewest
+// bytes per workgroup among those that run at once. At most four slices of at
+// least 1024, and only up to 256 rows: beyond, the partials' bytes outweigh it
+// (measured, FFN value, us, best whole / best cut: 0.4B 64 rows 11.1 / 7.8, 128
+// rows 11.0 / 8.7, 512 rows 17.9 / 16.6; 1.5B 64 rows 19.6 / 14.6, and 14.2 with
+// eight slices, less than their extra partials cost the LayerNorm).
+static int frag_plan(int M, int N, int K, int cus, int *splits) {
+  GemmProb p = {};
+  p.N = N;
+  int best = frag_tile(&p, 1, M, cus);
+  *splits = 1;
+  if (M > 256) return best;
+  int64_t bytes = INT64_MAX;
+  for (int i = 0; i < kFragNumTiles; ++i) {
+    for (int s = 1; s <= 4 && K / s >= 1024; s *= 2) {
+      if (frag_units(kFragTiles[i], M, N) * s > cus) break;
+      const int64_t b = (int64_t)(4 * kFragTiles[i].bm + 2 * kFragTiles[i].bn) * ((K + s - 1) / s);
+      if (b < bytes) {
+        bytes = b;
+        best = i;
+        *splits = s;
+      }
+    }
+  }
+  return best;
+}
+
+int gemm_frag_splits(int M, int N, int K) {
+  int s;
+  frag_plan(M, N, K, mk_cus() > 0 ? mk_cus() : 256, &s);
+  return s;
+}
+
+int launch_gemm_frag(const GemmProb *probs, int nprob, int M, hipStream_t st, int splits, int64_t part_stride) {
+  if (nprob < 1 || nprob > kFragProbs || M <= 0 || splits < 1 || (splits & (splits - 1))) return RWKV7_ESHAPE;
+  if (splits > 1 && (nprob != 1 || probs[0].epi != GEPI_F32)) return RWKV7_EINVAL;
+  const int cus = mk_cus() > 0 ? mk_cus() : 256;
+  for (int i = 0; i < nprob; ++i) {
+    const GemmProb &p = probs[i];
+    if (!p.A || !p.Wf || !p.Y) return RWKV7_EINVAL;
+    if (p.N <= 0 || p.K <= 0 || p.nksf != (p.K + 31) / 32 || p.bf != probs[0].bf) return RWKV7_ESHAPE;
+    if (p.epi == GEPI_ADD_F32 && (p.N % 4 || p.ldy % 4)) return RWKV7_ESHAPE;
+  }
+  int planned = 1;
+  const int ti = splits > 1 ? frag_plan(M, probs[0].N, probs[0].K, cus, &planned) : frag_tile(probs, nprob, M, cus);
+  if (splits > 1 && planned != splits) return RWKV7_EINVAL;
+  const FragTile t = kFragTiles[ti];
+  FragGroup g;
+  g.nprob = nprob;
+  g.M = M;
+  g.m_tiles = (M + t.bm - 1) / t.bm;
+  g.splits = splits;
+  g.part_stride = part_stride;
+  int64_t wgs = 0;
+  for (int i = 0; i < kFragProbs; ++i) {
+    g.wg_begin[i] = (int)wgs;
+    g.p[i] = probs[i < nprob ? i : 0];
+    if (i < nprob) wgs += (int64_t)((probs[i].N + t.bn - 1) / t.bn * splits + 7) / 8 * 8 * g.m_tiles;
+  }
+  if (wgs > INT32_MAX) return RWKV7_ESHAPE;
+  g.wg_begin[kFragProbs] = (int)wgs;
+  const bool bf = probs[0].bf != 0;
+  const dim3 grid((unsigned)wgs);
+#define RWKV7_FRAG(...)                                                            \
+  if (bf) gemm_frag_kernel<__VA_ARGS__, true><<<grid, kFragThreads, 0, st>>>(g);   \
+  else gemm_frag_kernel<__VA_ARGS__, false><<<grid, kFragThreads, 0, st>>>(g);     \
+  break;
+  switch (ti) {
+    case 0: RWKV7_FRAG(1, 2, 1, 1, 8, 2)
+    case 1: RWKV7_FRAG(2, 2, 1, 1, 8, 2)
+    case 2: RWKV7_FRAG(2, 4, 1, 1, 8, 1)
+    case 3: RWKV7_FRAG(2, 4, 2, 1, 4, 1)
+    case 4: RWKV7_FRAG(2, 4, 1, 2, 4, 1)
+    default: RWKV7_FRAG(2, 4, 2, 2, 2, 1)
+  }
+#undef RWKV7_FRAG
+  RWKV7_CHECK_LAUNCH();
+  return RWKV7_OK;
+}
+
+}  // namespace rwkv7

@@ -136,6 +136,7 @@ struct BatchWs {
   float *x0, *rkv, *d, *vfirst, *kv, *y, *part;  // kv: gated k, mixed v [2][M][C]
   float *proj1;  // one-token steps: r, k, v, raw LoRA first steps [M, 3C+SR]
   void *xmix, *l1, *yg, *hid, *headin;
+  float *x1;  // the other residual buffer of split steps (LnShiftArgs::x_out)
   float *U, *Send, *Pend;  // segmented scan of long sequences (null with one segment)
   float *rec;              // chunk records of the chunked scan (prefill_chunked)
 };
@@ -148,20 +149,25 @@ static int64_t batch_ws(const rwkv7_dims &d, int64_t B, int64_t T, char *base, B
     return p;
   };
   BatchWs t;
+  // operand buffers hold whole 16-row blocks (split order), the LoRA first
+  // steps' also whole 32-column blocks of each
+  const int64_t M16 = (M + 15) / 16 * 16, B16 = (B + 15) / 16 * 16;
   t.x0 = reinterpret_cast<float *>(take(M * C * 4));
-  t.xmix = take(6 * M * C * 4);
+  t.x1 = reinterpret_cast<float *>(take(M * C * 4));
+  t.xmix = take(6 * M16 * C * 4);
   t.rkv = reinterpret_cast<float *>(take(3 * M * C * 4));
-  t.l1 = take(M * SR * 4);
+  t.l1 = take(M16 * (SR + 4 * 32) * 4);
   t.d = reinterpret_cast<float *>(take(4 * M * C * 4));
   t.vfirst = reinterpret_cast<float *>(take(M * C * 4));
   t.kv = reinterpret_cast<float *>(take(2 * M * C * 4));
   t.y = reinterpret_cast<float *>(take(M * C * 4));
-  t.yg = take(M * C * 4);
-  t.hid = take(M * F * 4);
-  t.headin = take(B * C * 4);
+  t.yg = take(M16 * C * 4);
+  t.hid = take(M16 * F * 4);
+  t.headin = take(B16 * C * 4);
   t.proj1 = T == 1 ? reinterpret_cast<float *>(take(M * (3 * C + SR) * 4)) : nullptr;
   const int cus = mk_cus() > 0 ? mk_cus() : 256;
-  t.part = reinterpret_cast<float *>(take(gemm_ws_bytes((int)(M > B ? M : B), cus)));
+  const int64_t gws = gemm_ws_bytes((int)(M > B ? M : B), cus), fws = gemm_frag_splits((int)M, (int)C, (int)F) * M * C * 4;
+  t.part = reinterpret_cast<float *>(take(gws > fws ? gws : fws));
   int seg_len;
   const int64_t nseg = prefill_segments((int)T, (int)B, d.n_head, cus, &seg_len);
   t.U = t.Send = t.Pend = t.rec = nullptr;
@@ -322,6 +328,13 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
   const int bf = (m.flags & RWKV7_MODEL_BF16) ? 1 : 0;
   const int a32 = batch_a32(d, M) ? 1 : 0;
   const int esz = a32 ? 4 : 2;  // bytes per element of the GEMM operands
+  // f32 activations of more than a few rows run on the fragment GEMMs when the
+  // model has its fragment arenas: the producing kernels store each operand in
+  // split order
+  const int fr = a32 && m.layers_frag && M > kA32SkinnyMaxM ? 1 : 0;
+  const int fsplit = fr ? gemm_frag_splits(M, C, F) : 1;  // slices of the FFN value
+  float *x = w.x0, *x_other = w.x1;  // the residual rows; a sliced FFN value moves them between the two
+  int nparts = 0;                    // partial FFN values not yet added into x
   const int cus = mk_cus() > 0 ? mk_cus() : 256;  // as launch_wkv7_prefill decides
   // every GEMM of the step runs on the model's 16-bit format, with f32 A if a32
   auto gemm = [&](GemmProb *p, int n, int rows) {
@@ -329,7 +342,37 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
       p[i].bf = bf;
       p[i].a32 = a32;
     }
-    return launch_gemm_group(p, n, rows, st, w.part, ctr);
+    return fr ? launch_gemm_frag(p, n, rows, st) : launch_gemm_group(p, n, rows, st, w.part, ctr);
+  };
+  // LayerNorm + shift of the residual rows, adding the pending partials first
+  auto ln_shift = [&](LnShiftArgs &ls) {
+    ls.bf = bf;
+    ls.out_f32 = a32;
+    ls.split = fr;
+    if (nparts > 0) {
+      ls.part = w.part;
+      ls.nparts = nparts;
+      ls.part_stride = MC;
+      ls.x_out = x_other;
+    }
+    RWKV7_TRY(launch_ln_shift(ls, st));
+    if (nparts > 0) {
+      float *t = x;
+      x = x_other;
+      x_other = t;
+      nparts = 0;
+    }
+    return (int)RWKV7_OK;
+  };
+  // the FFN value product: added into x, or left as partials for the next LayerNorm
+  auto ffn_value = [&](GemmProb &gv) {
+    if (fsplit == 1) return gemm(&gv, 1, M);
+    gv.bf = bf;
+    gv.a32 = a32;
+    gv.epi = GEPI_F32;
+    gv.Y = w.part;
+    nparts = fsplit;
+    return launch_gemm_frag(&gv, 1, M, st, fsplit, MC);
   };
   // element offset into an operand buffer, as the uint16_t pointer GemmProb
   // holds for A (at) and as an output pointer (out_at)
@@ -337,7 +380,7 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
     return reinterpret_cast<const uint16_t *>(static_cast<char *>(base) + elems * esz);
   };
   auto out_at = [&](void *base, int64_t elems) { return static_cast<void *>(static_cast<char *>(base) + elems * esz); };
-  const int epi_relusq = a32 ? GEPI_RELUSQ_F32 : GEPI_RELUSQ;
+  const int epi_relusq = fr ? GEPI_RELUSQ_SPLIT : a32 ? GEPI_RELUSQ_F32 : GEPI_RELUSQ;
   const int epi_plain = a32 ? GEPI_F32 : GEPI_F16;
   const int epi_tanh = a32 ? GEPI_TANH_F32 : GEPI_TANH_F16;
   const int epi_sigm = a32 ? GEPI_SIGM_F32 : GEPI_SIGM_F16;
@@ -352,18 +395,17 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
     uint16_t *cshift = static_cast<uint16_t *>(s.cmix_x) + (int64_t)l * B * C;
     float *rnn = static_cast<float *>(s.rnn) + (int64_t)l * B * H * kN * kN;
 
-    LnShiftArgs ls = {w.x0, vec + RWKV7_V_LN1_W * C, vec + RWKV7_V_LN1_B * C, vec + RWKV7_V_X_R * C,
+    LnShiftArgs ls = {x, vec + RWKV7_V_LN1_W * C, vec + RWKV7_V_LN1_B * C, vec + RWKV7_V_X_R * C,
                       6, w.xmix, tshift, C, T, M};
-    ls.bf = bf;
-    ls.out_f32 = a32;
     // 16-bit operands (the large-M path): r, k, v at one stride, for one
     // strided-batched GEMM call (with f32 activations the stored order
     // measured ~1 % faster at 0.4B 1 x 512)
     ls.mix_order = a32 ? 0 : 1;
-    RWKV7_TRY(launch_ln_shift(ls, st));
+    RWKV7_TRY(ln_shift(ls));
     const int64_t sk = a32 ? 2 : 1, sv = a32 ? 3 : 2, sw = a32 ? 1 : 3;  // slots of k, v, w
-    const uint16_t *xr = at(w.xmix, 0), *xk = at(w.xmix, sk * MC), *xv = at(w.xmix, sv * MC),
-                   *xw = at(w.xmix, sw * MC), *xa = at(w.xmix, 4 * MC), *xg = at(w.xmix, 5 * MC);
+    const int64_t ms = fr ? split_halfs(M, C) / 2 : MC;  // elements per mix (split order: two halfs an element)
+    const uint16_t *xr = at(w.xmix, 0), *xk = at(w.xmix, sk * ms), *xv = at(w.xmix, sv * ms),
+                   *xw = at(w.xmix, sw * ms), *xa = at(w.xmix, 4 * ms), *xg = at(w.xmix, 5 * ms);
     if (T == 1) {
       // one token per sequence: r, k, v and the raw LoRA first steps into one
       // [M, 3C+SR] f32 matrix, then the fused per-head kernel (LoRA second
@@ -409,21 +451,20 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
       td.rg = rg;
       td.layer0 = l == 0;
       td.bf = bf;
+      td.yg_split = fr ? static_cast<uint16_t *>(w.yg) : nullptr;
       RWKV7_TRY(launch_tmix_decode(td, B, st));
-      GemmProb go = {at(w.yg, 0), reinterpret_cast<const uint16_t *>(L + lay.w_o), w.x0, C, C, C, C, C, GEPI_ADD_F32};
+      GemmProb go = {at(w.yg, 0), reinterpret_cast<const uint16_t *>(L + lay.w_o), x, C, C, C, C, C, GEPI_ADD_F32};
       frag(go, lay.f_o, 0);
       RWKV7_TRY(gemm(&go, 1, M));
-      LnShiftArgs lc = {w.x0, vec + RWKV7_V_LN2_W * C, vec + RWKV7_V_LN2_B * C, vec + RWKV7_V_FFN_X_K * C,
+      LnShiftArgs lc = {x, vec + RWKV7_V_LN2_W * C, vec + RWKV7_V_LN2_B * C, vec + RWKV7_V_FFN_X_K * C,
                         1, w.xmix, cshift, C, T, M};
-      lc.bf = bf;
-      lc.out_f32 = a32;
-      RWKV7_TRY(launch_ln_shift(lc, st));
+      RWKV7_TRY(ln_shift(lc));
       GemmProb gk = {at(w.xmix, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fk), w.hid, C, C, F, F, C, epi_relusq};
       frag(gk, lay.f_fk, 0);
       RWKV7_TRY(gemm(&gk, 1, M));
-      GemmProb gv = {at(w.hid, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fv), w.x0, F, F, C, C, F, GEPI_ADD_F32};
+      GemmProb gv = {at(w.hid, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fv), x, F, F, C, C, F, GEPI_ADD_F32};
       frag(gv, lay.f_fv, 0);
-      RWKV7_TRY(gemm(&gv, 1, M));
+      RWKV7_TRY(ffn_value(gv));
       continue;
     }
     GemmProb g1[7] = {
@@ -446,6 +487,17 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
     frag(g1[1], lay.f_rkv, C / 16);
     frag(g1[2], lay.f_rkv, 2 * C / 16);
     for (int g = 0; g < 4; ++g) frag(g1[3 + g], lay.f_l1[g], 0);
+    const bool prep_lora2 = prefill_chunked(T, B, H, cus) && lora2_fits(rv, rw, ra, rg);
+    const int rk[4] = {rv, rw, ra, rg};
+    int64_t lf[4] = {0, 0, 0, 0};  // halfs: the four first steps in split order
+    if (fr && !prep_lora2) {
+      const int epis[4] = {GEPI_SPLIT, GEPI_TANH_SPLIT, GEPI_SPLIT, GEPI_SIGM_SPLIT};
+      for (int g = 0; g < 4; ++g) {
+        if (g) lf[g] = lf[g - 1] + split_halfs(M, rk[g - 1]);
+        g1[3 + g].Y = static_cast<uint16_t *>(w.l1) + lf[g];
+        g1[3 + g].epi = epis[g];
+      }
+    }
     RWKV7_TRY(gemm(g1, 7, M));
     GemmProb g2[4] = {
         {at(w.l1, 0), wl2, w.d, SR, SR, C, C, rv, GEPI_F32},
@@ -453,10 +505,13 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
         {at(w.l1, rv + rw), wl2 + rv + rw, w.d + 2 * MC, SR, SR, C, C, ra, GEPI_F32},
         {at(w.l1, rv + rw + ra), wl2 + rv + rw + ra, w.d + 3 * MC, SR, SR, C, C, rg, GEPI_F32},
     };
-    for (int g = 0; g < 4; ++g) frag(g2[g], lay.f_l2[g], 0);
+    for (int g = 0; g < 4; ++g) {
+      frag(g2[g], lay.f_l2[g], 0);
+      if (fr) g2[g].A = static_cast<uint16_t *>(w.l1) + lf[g];
+    }
     PrefillScanArgs sc = {rnn, w.rkv, w.d, vec, w.vfirst, w.y, w.kv, w.kv + MC, B, T, H, C, M, l == 0,
                           w.U, w.Send, w.Pend, w.rec};
-    if (prefill_chunked(T, B, H, cus) && lora2_fits(rv, rw, ra, rg)) {
+    if (prep_lora2) {
       // the chunked scan's prep kernel forms the LoRA second steps itself
       sc.l1 = w.l1;
       sc.w2 = wl2;
@@ -474,27 +529,27 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
     GnGateArgs gn = {w.y, w.rkv, w.kv, w.kv + MC, w.d + 3 * MC, vec, w.yg, C, M};
     gn.bf = bf;
     gn.out_f32 = a32;
+    gn.split = fr;
     RWKV7_TRY(launch_gn_gate(gn, st));
-    GemmProb go = {at(w.yg, 0), reinterpret_cast<const uint16_t *>(L + lay.w_o), w.x0, C, C, C, C, C, GEPI_ADD_F32};
+    GemmProb go = {at(w.yg, 0), reinterpret_cast<const uint16_t *>(L + lay.w_o), x, C, C, C, C, C, GEPI_ADD_F32};
     frag(go, lay.f_o, 0);
     RWKV7_TRY(gemm(&go, 1, M));
 
-    LnShiftArgs lc = {w.x0, vec + RWKV7_V_LN2_W * C, vec + RWKV7_V_LN2_B * C, vec + RWKV7_V_FFN_X_K * C,
+    LnShiftArgs lc = {x, vec + RWKV7_V_LN2_W * C, vec + RWKV7_V_LN2_B * C, vec + RWKV7_V_FFN_X_K * C,
                       1, w.xmix, cshift, C, T, M};
-    lc.bf = bf;
-    lc.out_f32 = a32;
-    RWKV7_TRY(launch_ln_shift(lc, st));
+    RWKV7_TRY(ln_shift(lc));
     GemmProb gk = {at(w.xmix, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fk), w.hid, C, C, F, F, C, epi_relusq};
     frag(gk, lay.f_fk, 0);
     RWKV7_TRY(gemm(&gk, 1, M));
-    GemmProb gv = {at(w.hid, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fv), w.x0, F, F, C, C, F, GEPI_ADD_F32};
+    GemmProb gv = {at(w.hid, 0), reinterpret_cast<const uint16_t *>(L + lay.w_fv), x, F, F, C, C, F, GEPI_ADD_F32};
     frag(gv, lay.f_fv, 0);
-    RWKV7_TRY(gemm(&gv, 1, M));
+    RWKV7_TRY(ffn_value(gv));
   }
   if (logits) {
     // B rows: the head GEMM always takes f32 A (B is far below the large-M path)
     const float *lo = static_cast<const float *>(m.ln_out);
-    RWKV7_TRY(launch_ln_rows(w.x0, 1, lo, lo + C, w.headin, 1, B, C, T, T - 1, bf, st));
+    const bool hf = m.head_frag && B > kA32SkinnyMaxM;
+    RWKV7_TRY(launch_ln_rows(x, 1, lo, lo + C, w.headin, hf ? 2 : 1, B, C, T, T - 1, bf, st, w.part, nparts, MC));
     GemmProb gh = {static_cast<const uint16_t *>(w.headin), static_cast<const uint16_t *>(m.head), logits, C, C,
                    d.vocab, d.vocab, C, GEPI_F16};
     if (m.head_frag) {
@@ -503,6 +558,7 @@ static int run_batched(const rwkv7_model &m, const rwkv7_state &s, const int64_t
     }
     gh.bf = bf;
     gh.a32 = 1;
+    if (hf) return launch_gemm_frag(&gh, 1, B, st);
     RWKV7_TRY(launch_gemm_group(&gh, 1, B, st, w.part, ctr));
   }
   return RWKV7_OK;

@@ -215,6 +215,51 @@ RWKV7_DEV void split_hi_lo(const uint4 &a, const uint4 &b, uint4 &hi, uint4 &lo)
   lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
+// An activation matrix as the A operand of gemm_frag.hip ("split order"):
+// blocks of 16 rows x 32 columns, nks = ceil(columns / 32) of them per 16 rows,
+// each 2 KiB: the 64 lanes' 16 bytes of the values' 16-bit parts (lane l: row l
+// % 16, columns 8 (l / 16) .. +8), then those of the remainders (split_hi_lo's
+// two values). put8 stores eight columns n .. n + 7 (n % 8 == 0) of row m, put4
+// four, put1 one. (With 128 columns of a row contiguous instead, the producers'
+// stores are whole lines but every operand load touches 64 bytes of 16 rows:
+// the GEMMs took 1.3-1.6 times as long.)
+inline int64_t split_halfs(int64_t M, int64_t K) { return (M + 15) / 16 * ((K + 31) / 32) * 1024; }
+RWKV7_DEV int64_t split_at(int nks, int m, int n) {
+  return ((int64_t)(m >> 4) * nks + (n >> 5)) * 1024 + ((m & 15) + 16 * ((n & 31) >> 3)) * 8 + (n & 7);
+}
+template <bool BF>
+RWKV7_DEV void split_put1(uint16_t *base, int nks, int m, int n, float v) {
+  const uint16_t h = F16T<BF>::from_f(v), l = F16T<BF>::from_f(v - F16T<BF>::to_f(h));
+  uint16_t *d = base + split_at(nks, m, n);
+  d[0] = h;
+  d[512] = l;
+}
+template <bool BF>
+RWKV7_DEV void split_put4(uint16_t *base, int nks, int m, int n, const float (&v)[4]) {
+  uint16_t h[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    h[e] = F16T<BF>::from_f(v[e]);
+    l[e] = F16T<BF>::from_f(v[e] - F16T<BF>::to_f(h[e]));
+  }
+  uint16_t *d = base + split_at(nks, m, n);
+  *reinterpret_cast<uint2 *>(d) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+  *reinterpret_cast<uint2 *>(d + 512) = make_uint2((uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16));
+}
+
+template <bool BF>
+RWKV7_DEV void split_put8(uint16_t *base, int nks, int m, int n, const float (&v)[8]) {
+  uint4 a, b, hi, lo;
+  a = make_uint4(__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]), __builtin_bit_cast(uint32_t, v[2]),
+                 __builtin_bit_cast(uint32_t, v[3]));
+  b = make_uint4(__builtin_bit_cast(uint32_t, v[4]), __builtin_bit_cast(uint32_t, v[5]), __builtin_bit_cast(uint32_t, v[6]),
+                 __builtin_bit_cast(uint32_t, v[7]));
+  split_hi_lo<BF>(a, b, hi, lo);
+  uint16_t *d = base + split_at(nks, m, n);
+  *reinterpret_cast<uint4 *>(d) = hi;
+  *reinterpret_cast<uint4 *>(d + 512) = lo;
+}
+
 RWKV7_DEV float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }
 
 // Weight streams are read exactly once per step: load them non-temporally so

@@ -45,6 +45,7 @@ struct TmixDecodeArgs {
   int C, H, rv, rw, ra, rg, layer0;
   uint16_t *yg16;
   int bf;  // w_lora2, shift and yg16 are bfloat16 (else half)
+  uint16_t *yg_split = nullptr;  // when set: the gated output in split order (split_put1) instead
 };
 int launch_tmix_decode(const TmixDecodeArgs &a, int B, hipStream_t st);
 
@@ -101,6 +102,15 @@ struct LnShiftArgs {
   // output slot order of six mixes: 0 as the mix vectors are stored (r, w,
   // k, v, a, g), 1 r, k, v, w, a, g (r, k, v at one stride: one batched GEMM)
   int mix_order = 0;
+  // split: out is n_mix matrices in split order (split_put4), split_halfs(M,
+  // C) halfs apart. A row of x0 may then also be the sum of x0 and nparts (0,
+  // 2 or 4; six mixes) partial products, part_stride floats apart, which goes to x_out
+  // (not x0: other rows' workgroups still read it).
+  int split = 0;
+  const float *part = nullptr;
+  int nparts = 0;
+  int64_t part_stride = 0;
+  float *x_out = nullptr;
 };
 int launch_ln_shift(const LnShiftArgs &a, hipStream_t st);
 
@@ -159,13 +169,17 @@ struct GnGateArgs {
   int C, M;
   int bf;  // a 16-bit out is bfloat16 (else half)
   int out_f32;
+  int split = 0;  // out in split order (split_put1)
 };
 int launch_gn_gate(const GnGateArgs &a, hipStream_t st);
 
 // bf: the 16-bit operands are bfloat16 (else half)
 int launch_embed(const int64_t *tok, const uint16_t *emb, float *x0, int M, int C, int V, int bf, hipStream_t st);
+// out_f32: 0 16-bit, 1 f32, 2 split order (split_put1). x f32 may be x plus
+// nparts partial products (LnShiftArgs).
 int launch_ln_rows(const void *x, int x_f32, const float *w, const float *b, void *out, int out_f32,
-                   int rows, int C, int stride, int offset, int bf, hipStream_t st);
+                   int rows, int C, int stride, int offset, int bf, hipStream_t st, const float *part = nullptr,
+                   int nparts = 0, int64_t part_stride = 0);
 int launch_lerp(const uint16_t *x, const uint16_t *prev, const float *mu, int n_mix, uint16_t *out,
                 uint16_t *x_copy, int C, int bf, hipStream_t st);
 int launch_store_f16(const float *src, uint16_t *dst, int n, int bf, hipStream_t st);
@@ -181,6 +195,12 @@ enum {
   GEPI_RELUSQ_F32 = 6,
   GEPI_TANH_F32 = 7,
   GEPI_SIGM_F32 = 8,
+  // the next product's A in split order (gemm_frag.hip only): plain, then
+  // the activations
+  GEPI_SPLIT = 9,
+  GEPI_RELUSQ_SPLIT = 10,
+  GEPI_TANH_SPLIT = 11,
+  GEPI_SIGM_SPLIT = 12,
 };
 struct GemmProb {
   const uint16_t *A, *W;
@@ -210,6 +230,16 @@ int gemm_big_min_rows(int N);
 constexpr int kGemmCounters = 1024;
 int64_t gemm_ws_bytes(int M, int cus);
 int launch_gemm_group(const GemmProb *probs, int nprob, int M, hipStream_t st, float *part, unsigned *ctr);
+// The same products on fragment-ordered operands (gemm_frag.hip): A as
+// split_put4 writes it, W from the fragment arena (p.Wf), 16-byte aligned f32
+// outputs. splits > 1: K is cut and slice s's f32 product stored at Y + s *
+// part_stride floats (one problem, GEPI_F32); gemm_frag_splits is the count
+// that pays for an N x K problem of M rows (1, 2 or 4).
+int gemm_frag_splits(int M, int N, int K);
+int launch_gemm_frag(const GemmProb *probs, int nprob, int M, hipStream_t st, int splits = 1, int64_t part_stride = 0);
+// rows up to which a step's f32 activations run on the strips of
+// gemm_skinny_kernel rather than the fragment kernel
+constexpr int kA32SkinnyMaxM = 8;
 // Large-M problems with 16-bit operands and a plain epilogue (f32, 16-bit or
 // add into f32), or relu^2 into half (a half product, then an in-place pass),
 // through hipBLASLt (gemm_lt.hip); lt_gemm returns false when it did

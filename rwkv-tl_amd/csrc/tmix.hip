@@ -125,7 +125,8 @@ __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
     const float var = wave_sum(d * d) * (1.f / kN);
     const float yn = d * rsqrtf(var + kGnEps) * vec[RWKV7_V_LNX_W * C + ch] + vec[RWKV7_V_LNX_B * C + ch];
     const float out = (yn + s_rk * s_v[t]) * s_g[t];
-    if (a.yg16) a.yg16[(int64_t)b * C + ch] = T16::from_f(out);
+    if (a.yg_split) split_put1<BF>(a.yg_split, C / 32, b, ch, out);
+    else if (a.yg16) a.yg16[(int64_t)b * C + ch] = T16::from_f(out);
     else a.yg[(int64_t)b * C + ch] = out;
   }
 }
@@ -2024,6 +2025,299 @@ __global__ __launch_bounds__(256) void ln_shift_vec_kernel(LnShiftArgs a, int R)
   }
 }
 
+// LayerNorm + token shift for the fragment GEMMs: the mixes go out as the A
+// operand in fragment order, and a row may still be x0 plus the NPART partial
+// products of the FFN value (summed here instead of in a launch or an arrival
+// count of their own). Four consecutive columns per thread and piece (NP4
+// pieces: C <= 1024 NP4). A row needs at most one other row, its predecessor
+// or (t = 0, OTHER: T > 1) the sequence's last, whose normalised values are the
+// new shift state. Latency-bound: every load is issued up front and
+// unconditionally (columns past C clamped; selects on the loaded values cost a
+// predicated load per float, 15 us where this takes 5).
+template <int NP4, int NPART, int NMIX, bool OTHER>
+__global__ __launch_bounds__(256) void ln_shift_split_kernel(LnShiftArgs a) {
+  __shared__ float red[2][2][4];
+  const int C = a.C, T = a.T, tid = threadIdx.x, M = a.M;
+  int c[NP4];
+  bool live[NP4];
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) {
+    c[p] = min(4 * (tid + 256 * p), C - 4);
+    live[p] = 4 * (tid + 256 * p) < C;
+  }
+  auto ld = [&](const float *row, float4 (&d)[NP4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < NP4; ++p) d[p] = *reinterpret_cast<const float4 *>(row + c[p]);
+  };
+  struct Row {
+    float4 x[NP4], q[NPART > 0 ? NPART : 1][NP4];
+  };
+  auto ld_row = [&](int m, Row &r) __attribute__((always_inline)) {
+    ld(a.x0 + (int64_t)m * C, r.x);
+#pragma unroll
+    for (int s = 0; s < NPART; ++s) ld(a.part + s * a.part_stride + (int64_t)m * C, r.q[s]);
+  };
+  auto sum_row = [&](Row &r) __attribute__((always_inline)) {
+    if constexpr (NPART > 0) {
+#pragma unroll
+      for (int p = 0; p < NP4; ++p) {
+        float4 d = r.q[0][p];
+#pragma unroll
+        for (int s = 1; s < NPART; ++s) {
+          d.x += r.q[s][p].x;
+          d.y += r.q[s][p].y;
+          d.z += r.q[s][p].z;
+          d.w += r.q[s][p].w;
+        }
+        r.x[p].x += d.x;
+        r.x[p].y += d.y;
+        r.x[p].z += d.z;
+        r.x[p].w += d.w;
+      }
+    }
+  };
+  // One row per workgroup: eight consecutive rows, whose 16-byte pieces share
+  // the output's 128-byte lines, to workgroups of one XCD (dealt round-robin),
+  // so that its L2 merges them (509 rows, six mixes: 12.1 us with the rows of a
+  // line on eight XCDs)
+  const int bx = blockIdx.x, m = (bx >> 6) * 64 + (bx & 7) * 8 + ((bx >> 3) & 7), t = m % T;
+  if (m >= M) return;
+  Row rc, ro;
+  uint2 st[NP4];
+  ld_row(m, rc);
+  if (OTHER) ld_row(t > 0 ? m - 1 : m + T - 1, ro);
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) st[p] = *reinterpret_cast<const uint2 *>(a.shift + (int64_t)(m / T) * C + c[p]);
+  float4 lw[NP4], lb[NP4], mu[NMIX][NP4];
+  ld(a.ln_w, lw);
+  ld(a.ln_b, lb);
+#pragma unroll
+  for (int j = 0; j < NMIX; ++j) ld(a.mu + (int64_t)j * C, mu[j]);
+  const float invC = 1.f / (float)C;
+  const int64_t mstride = (int64_t)((M + 15) / 16) * (C / 32) * 1024;
+  sum_row(rc);
+  if (OTHER) sum_row(ro);
+  if constexpr (NPART > 0) {
+#pragma unroll
+    for (int p = 0; p < NP4; ++p)
+      if (live[p]) *reinterpret_cast<float4 *>(a.x_out + (int64_t)m * C + c[p]) = rc.x[p];
+  }
+  // two-pass mean and variance of both rows
+  auto block_sum2 = [&](float &u, float &v, float (&s)[2][4]) __attribute__((always_inline)) {
+    const float2 w = wave_sum2(u, v);
+    if ((tid & 63) == 0) {
+      s[0][tid >> 6] = w.x;
+      s[1][tid >> 6] = w.y;
+    }
+    __syncthreads();
+    u = (s[0][0] + s[0][1]) + (s[0][2] + s[0][3]);
+    v = (s[1][0] + s[1][1]) + (s[1][2] + s[1][3]);
+  };
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) {
+    const float4 &u = rc.x[p], &v = ro.x[p];
+    if (live[p]) {
+      s0 += (u.x + u.y) + (u.z + u.w);
+      if (OTHER) s1 += (v.x + v.y) + (v.z + v.w);
+    }
+  }
+  block_sum2(s0, s1, red[0]);
+  const float mc = s0 * invC, mo = s1 * invC;
+  auto sq = [](const float4 &v, float mean) {
+    const float x = v.x - mean, y = v.y - mean, z = v.z - mean, w = v.w - mean;
+    return (x * x + y * y) + (z * z + w * w);
+  };
+  float q0 = 0.f, q1 = 0.f;
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) {
+    if (live[p]) {
+      q0 += sq(rc.x[p], mc);
+      if (OTHER) q1 += sq(ro.x[p], mo);
+    }
+  }
+  block_sum2(q0, q1, red[1]);
+  const float r0 = rsqrtf(q0 * invC + kLnEps), r1 = rsqrtf(q1 * invC + kLnEps);
+  auto norm = [](const float4 &v, float mean, float rs, const float4 &w, const float4 &b) {
+    return make_float4((v.x - mean) * rs * w.x + b.x, (v.y - mean) * rs * w.y + b.y, (v.z - mean) * rs * w.z + b.z,
+                       (v.w - mean) * rs * w.w + b.w);
+  };
+  float4 xn[NP4], on[NP4], sv[NP4];
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) {
+    xn[p] = norm(rc.x[p], mc, r0, lw[p], lb[p]);
+    if (OTHER) on[p] = norm(ro.x[p], mo, r1, lw[p], lb[p]);
+    sv[p] = make_float4(u16_to_f((uint16_t)st[p].x, a.bf), u16_to_f((uint16_t)(st[p].x >> 16), a.bf),
+                        u16_to_f((uint16_t)st[p].y, a.bf), u16_to_f((uint16_t)(st[p].y >> 16), a.bf));
+  }
+  const bool first = !OTHER || t == 0;  // uniform
+#pragma unroll
+  for (int p = 0; p < NP4; ++p) {
+    const float4 pv = first ? sv[p] : on[p];
+    const float4 d = make_float4(pv.x - xn[p].x, pv.y - xn[p].y, pv.z - xn[p].z, pv.w - xn[p].w);
+    if (live[p]) {
+#pragma unroll
+      for (int j = 0; j < NMIX; ++j) {
+        const float v[4] = {xn[p].x + mu[j][p].x * d.x, xn[p].y + mu[j][p].y * d.y, xn[p].z + mu[j][p].z * d.z,
+                            xn[p].w + mu[j][p].w * d.w};
+        uint16_t *f = static_cast<uint16_t *>(a.out) + j * mstride;
+        if (a.bf) split_put4<true>(f, C / 32, m, c[p], v);
+        else split_put4<false>(f, C / 32, m, c[p], v);
+      }
+      if (first) {  // the new state: the sequence's last row
+        const float4 n = OTHER && T > 1 ? on[p] : xn[p];
+        *reinterpret_cast<uint2 *>(a.shift + (int64_t)(m / T) * C + c[p]) =
+            make_uint2((uint32_t)f_to_u16(n.x, a.bf) | ((uint32_t)f_to_u16(n.y, a.bf) << 16),
+                       (uint32_t)f_to_u16(n.z, a.bf) | ((uint32_t)f_to_u16(n.w, a.bf) << 16));
+      }
+    }
+  }
+}
+
+// The six mixes of many rows: eight consecutive rows per workgroup, a wave per
+// row normalising into LDS, then the mixes with lanes along the rows, so that
+// the eight rows' 16-byte pieces go out as whole 128-byte lines. Taken from 768
+// rows of C <= 1024, where a workgroup's own latency is covered (measured, us,
+// this / one row per workgroup: C = 1024, 509 rows 8.7 / 7.7, 896 rows 9.9 /
+// 11.7, 1600 rows 12.8 / 17.7; C = 768, 1491 rows 10.3 / 13.4; C = 2048, 800
+// rows 19.4 / 19.0; with one mix no faster at any size).
+constexpr int kLnSplit8MinM = 768;
+__global__ __launch_bounds__(1024) void ln_shift_split8_kernel(LnShiftArgs a) {
+  constexpr int NL = 4;  // float4 pieces of a row per lane
+  __shared__ __align__(16) float s_x[17][1024];  // row m0 - 1, rows m0 .. + 7, old states of rows with t = 0
+  const int C = a.C, T = a.T, M = a.M, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = 8 * blockIdx.x;
+  int c[NL];
+  bool live[NL];
+#pragma unroll
+  for (int p = 0; p < NL; ++p) {
+    c[p] = min(4 * (lane + 64 * p), C - 4);
+    live[p] = 4 * (lane + 64 * p) < C;
+  }
+  const float invC = 1.f / (float)C;
+  // LayerNorm of a row, one wave
+  auto norm_row = [&](int m, float4 (&x)[NL]) __attribute__((always_inline)) {
+    float4 w[NL], b[NL];
+#pragma unroll
+    for (int p = 0; p < NL; ++p) {
+      x[p] = *reinterpret_cast<const float4 *>(a.x0 + (int64_t)m * C + c[p]);
+      w[p] = *reinterpret_cast<const float4 *>(a.ln_w + c[p]);
+      b[p] = *reinterpret_cast<const float4 *>(a.ln_b + c[p]);
+    }
+    float s = 0.f, q = 0.f;
+#pragma unroll
+    for (int p = 0; p < NL; ++p)
+      if (live[p]) s += (x[p].x + x[p].y) + (x[p].z + x[p].w);
+    const float mean = wave_sum(s) * invC;
+#pragma unroll
+    for (int p = 0; p < NL; ++p) {
+      x[p] = make_float4(x[p].x - mean, x[p].y - mean, x[p].z - mean, x[p].w - mean);
+      if (live[p]) q += (x[p].x * x[p].x + x[p].y * x[p].y) + (x[p].z * x[p].z + x[p].w * x[p].w);
+    }
+    const float rs = rsqrtf(wave_sum(q) * invC + kLnEps);
+#pragma unroll
+    for (int p = 0; p < NL; ++p)
+      x[p] = make_float4(x[p].x * rs * w[p].x + b[p].x, x[p].y * rs * w[p].y + b[p].y, x[p].z * rs * w[p].z + b[p].z,
+                         x[p].w * rs * w[p].w + b[p].w);
+  };
+  auto put = [&](int slot, const float4 (&x)[NL]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < NL; ++p)
+      if (live[p]) *reinterpret_cast<float4 *>(&s_x[slot][c[p]]) = x[p];
+  };
+  if (wv == 8 && m0 % T > 0) {
+    float4 x[NL];
+    norm_row(m0 - 1, x);
+    put(0, x);
+  }
+  if (wv < 8 && m0 + wv < M) {
+    const int i = wv, m = m0 + i;
+    float4 x[NL];
+    norm_row(m, x);
+    put(1 + i, x);
+    if (m % T == 0) {  // the old state is the row before; the new one the sequence's last row
+      uint16_t *sh = a.shift + (int64_t)(m / T) * C;
+      float4 o[NL];
+#pragma unroll
+      for (int p = 0; p < NL; ++p) {
+        const uint2 u = *reinterpret_cast<const uint2 *>(sh + c[p]);
+        o[p] = make_float4(u16_to_f((uint16_t)u.x, a.bf), u16_to_f((uint16_t)(u.x >> 16), a.bf),
+                           u16_to_f((uint16_t)u.y, a.bf), u16_to_f((uint16_t)(u.y >> 16), a.bf));
+      }
+      put(9 + i, o);
+      if (T > 1) norm_row(m + T - 1, x);
+#pragma unroll
+      for (int p = 0; p < NL; ++p)
+        if (live[p])
+          *reinterpret_cast<uint2 *>(sh + c[p]) =
+              make_uint2((uint32_t)f_to_u16(x[p].x, a.bf) | ((uint32_t)f_to_u16(x[p].y, a.bf) << 16),
+                         (uint32_t)f_to_u16(x[p].z, a.bf) | ((uint32_t)f_to_u16(x[p].w, a.bf) << 16));
+    }
+  }
+  __syncthreads();
+  // lane -> row lane % 8, eight columns per 8 lanes
+  const int r = lane & 7, m = m0 + r;
+  if (m >= M) return;
+  const float *xr = s_x[1 + r], *pr = m % T == 0 ? s_x[9 + r] : s_x[r];
+  const int64_t mstride = (int64_t)((M + 15) / 16) * (C / 32) * 1024;
+  for (int g = threadIdx.x >> 3; g < C / 8; g += 128) {
+    float x[8], d[8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float4 u = *reinterpret_cast<const float4 *>(xr + 8 * g + 4 * h), v = *reinterpret_cast<const float4 *>(pr + 8 * g + 4 * h);
+      x[4 * h] = u.x;
+      x[4 * h + 1] = u.y;
+      x[4 * h + 2] = u.z;
+      x[4 * h + 3] = u.w;
+      d[4 * h] = v.x - u.x;
+      d[4 * h + 1] = v.y - u.y;
+      d[4 * h + 2] = v.z - u.z;
+      d[4 * h + 3] = v.w - u.w;
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const float4 u = *reinterpret_cast<const float4 *>(a.mu + (int64_t)j * C + 8 * g);
+      const float4 z = *reinterpret_cast<const float4 *>(a.mu + (int64_t)j * C + 8 * g + 4);
+      const float mu[8] = {u.x, u.y, u.z, u.w, z.x, z.y, z.z, z.w};
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = x[e] + mu[e] * d[e];
+      uint16_t *f = static_cast<uint16_t *>(a.out) + j * mstride;
+      if (a.bf) split_put8<true>(f, C / 32, m, 8 * g, v);
+      else split_put8<false>(f, C / 32, m, 8 * g, v);
+    }
+  }
+}
+
+template <int NP4>
+static int launch_ln_split(const LnShiftArgs &a, hipStream_t st) {
+  if (a.nparts > 0 && a.n_mix != 6) return RWKV7_EINVAL;
+  if constexpr (NP4 == 1) {
+    if (a.n_mix == 6 && a.nparts == 0 && a.M >= kLnSplit8MinM) {
+      ln_shift_split8_kernel<<<(a.M + 7) / 8, 1024, 0, st>>>(a);
+      RWKV7_CHECK_LAUNCH();
+      return RWKV7_OK;
+    }
+  }
+  const dim3 grid((a.M + 63) / 64 * 64);
+#define RWKV7_LNS6(NPART, NMIX, OTHER) ln_shift_split_kernel<NP4, NPART, NMIX, OTHER><<<grid, 256, 0, st>>>(a)
+  if (a.n_mix == 1) {
+    if (a.T > 1) RWKV7_LNS6(0, 1, true);
+    else RWKV7_LNS6(0, 1, false);
+  } else if (a.T > 1) {
+    if (a.nparts == 0) RWKV7_LNS6(0, 6, true);
+    else if (a.nparts == 2) RWKV7_LNS6(2, 6, true);
+    else RWKV7_LNS6(4, 6, true);
+  } else {
+    if (a.nparts == 0) RWKV7_LNS6(0, 6, false);
+    else if (a.nparts == 2) RWKV7_LNS6(2, 6, false);
+    else RWKV7_LNS6(4, 6, false);
+  }
+#undef RWKV7_LNS6
+  RWKV7_CHECK_LAUNCH();
+  return RWKV7_OK;
+}
+
 int launch_ln_shift(const LnShiftArgs &a, hipStream_t st) {
   if (a.C % 256 || a.C > 256 * kMaxCPer || a.n_mix < 1 || a.n_mix > 6 || a.M <= 0 || a.T <= 0) return RWKV7_ESHAPE;
   const int np = a.C / 256;
@@ -2034,6 +2328,17 @@ int launch_ln_shift(const LnShiftArgs &a, hipStream_t st) {
   // 3.43 with the same grid)
   const int want = 2 * (mk_cus() > 0 ? mk_cus() : 256);
   int R = 1, ncs = 1;
+  if (a.split) {
+    if (a.n_mix != 1 && a.n_mix != 6) return RWKV7_ESHAPE;
+    if (a.nparts != 0 && a.nparts != 2 && a.nparts != 4) return RWKV7_EINVAL;
+    if (a.nparts > 0 && (!a.part || !a.x_out || a.x_out == a.x0)) return RWKV7_EINVAL;
+    switch ((a.C + 1023) / 1024) {
+      case 1: return launch_ln_split<1>(a, st);
+      case 2: return launch_ln_split<2>(a, st);
+      case 3: return launch_ln_split<3>(a, st);
+      default: return launch_ln_split<4>(a, st);
+    }
+  }
   if (a.M >= 2 * want) R = min(8, a.M / want);
   else
     while (ncs * 2 <= np && np % (ncs * 2) == 0 && (int64_t)a.M * ncs < want) ncs *= 2;
@@ -2087,7 +2392,11 @@ __global__ __launch_bounds__(256) void gn_gate_kernel(GnGateArgs a) {
   const float yn = d * rsqrtf(var + kGnEps) * a.vec[RWKV7_V_LNX_W * C + ch] + a.vec[RWKV7_V_LNX_B * C + ch];
   const float rk = wave_sum(a.r[o] * a.kn[o] * a.vec[RWKV7_V_R_K * C + ch]);
   const float out = (yn + rk * a.v[o]) * a.g[o];
-  if (a.out_f32) static_cast<float *>(a.out)[o] = out;
+  if (a.split) {
+    uint16_t *f = static_cast<uint16_t *>(a.out);
+    if (a.bf) split_put1<true>(f, C / 32, m, ch, out);
+    else split_put1<false>(f, C / 32, m, ch, out);
+  } else if (a.out_f32) static_cast<float *>(a.out)[o] = out;
   else static_cast<uint16_t *>(a.out)[o] = f_to_u16(out, a.bf);
 }
 
@@ -2121,7 +2430,8 @@ int launch_embed(const int64_t *tok, const uint16_t *emb, float *x0, int M, int 
 // last token of each sequence before the LM head).
 __global__ __launch_bounds__(256) void ln_rows_kernel(const void *x, int x_f32, const float *w,
                                                       const float *bvec, void *out, int out_f32,
-                                                      int C, int stride, int offset, int bf) {
+                                                      int C, int stride, int offset, int bf, const float *part,
+                                                      int nparts, int64_t part_stride) {
   __shared__ float scratch4[4];
   const int i = blockIdx.x;
   const int64_t src = (int64_t)i * stride + offset;
@@ -2132,6 +2442,11 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(const void *x, int x_f32, 
     const int c = threadIdx.x + 256 * q;
     v[q] = x_f32 ? reinterpret_cast<const float *>(x)[src * C + c]
                  : u16_to_f(reinterpret_cast<const uint16_t *>(x)[src * C + c], bf);
+    if (nparts > 0) {
+      float d = part[src * C + c];
+      for (int u = 1; u < nparts; ++u) d += part[u * part_stride + src * C + c];
+      v[q] += d;
+    }
     s += v[q];
   }
   const float mean = block_sum256(s, scratch4) / (float)C;
@@ -2144,15 +2459,20 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(const void *x, int x_f32, 
   RWKV7_UNROLL_N(q) {
     const int c = threadIdx.x + 256 * q;
     const float y = (v[q] - mean) * rstd * w[c] + bvec[c];
-    if (out_f32) reinterpret_cast<float *>(out)[(int64_t)i * C + c] = y;
+    if (out_f32 == 2) {
+      uint16_t *f = reinterpret_cast<uint16_t *>(out);
+      if (bf) split_put1<true>(f, C / 32, i, c, y);
+      else split_put1<false>(f, C / 32, i, c, y);
+    } else if (out_f32) reinterpret_cast<float *>(out)[(int64_t)i * C + c] = y;
     else reinterpret_cast<uint16_t *>(out)[(int64_t)i * C + c] = f_to_u16(y, bf);
   }
 }
 
 int launch_ln_rows(const void *x, int x_f32, const float *w, const float *b, void *out, int out_f32,
-                   int rows, int C, int stride, int offset, int bf, hipStream_t st) {
+                   int rows, int C, int stride, int offset, int bf, hipStream_t st, const float *part, int nparts,
+                   int64_t part_stride) {
   if (C % 256 || C > 256 * kMaxCPer) return RWKV7_ESHAPE;
-  ln_rows_kernel<<<rows, 256, 0, st>>>(x, x_f32, w, b, out, out_f32, C, stride, offset, bf);
+  ln_rows_kernel<<<rows, 256, 0, st>>>(x, x_f32, w, b, out, out_f32, C, stride, offset, bf, part, nparts, part_stride);
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;
 }

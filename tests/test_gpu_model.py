@@ -23,9 +23,9 @@ import pytest
 import torch
 
 from oracle import rwkv7_ref as R
-from rwkv_tl_amd import RWKV7HIP, HIPGraph, State, make_rwkv7
+from rwkv_tl_amd import RWKV7HIP, RWKV7HIPBF16, HIPGraph, ModelShape, State, make_rwkv7
 from rwkv_tl_amd.checkpoint import make_random_state_dict
-from rwkv_tl_amd.weight import RWKV7Weight
+from rwkv_tl_amd.weight import RWKV7Weight, pack_device_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -567,3 +567,49 @@ def test_persistent_decode_abort_is_visible(cuda):
     _check_logits(lg, l32, "step after an aborted launch")
     _check_state(S, s32, STATE_REL, "state after an aborted launch")
     assert st.model.last_error() == errs0 + 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("C,F,ranks,B,T", [
+    (768, 3072, (64, 64, 32, 128), 1, 17),    # one row past a 16-row block, a sliced FFN value
+    (768, 3072, (24, 8, 16, 40), 17, 1),      # one-token steps, LoRA widths that are no multiple of 32
+    (768, 3072, (64, 64, 32, 128), 2, 129),   # 258 rows: past the sliced FFN value; the chunked scan
+    (256, 2048, (24, 8, 16, 40), 5, 31),      # idle LayerNorm threads, LoRA second steps as GEMMs
+    (1024, 4096, (64, 64, 32, 128), 3, 21),   # four slices
+    (1024, 1024, (64, 64, 32, 128), 97, 8),   # 776 rows: eight rows per LayerNorm workgroup, several sequences in one
+    (2048, 4096, (64, 64, 32, 128), 1, 33),   # two pieces per LayerNorm thread
+])
+def test_fragment_gemm_steps_match_row_major_weights(dtype, C, F, ranks, B, T, cuda):
+    """Steps of more than 16 rows on the fragment arenas (activations stored in
+    split order by their producers, gemm_frag.hip) against the same steps on
+    the row-major arenas (f32 activations split inside gemm.hip's kernels): the
+    same 16-bit products with fp32 sums in another order, so the state agrees
+    to fp32 rounding -- 1e-5 relative for half, and for bfloat16 (whose hi + lo
+    parts hold 16 bits, the same on both sides) the same; logits and shift
+    states to one unit of their 16-bit format."""
+    shape = ModelShape(2, C, F, 512, *ranks)
+    sd = make_random_state_dict(shape, seed=C + T, dtype=dtype)
+    w = RWKV7Weight.from_state_dict(sd, device=cuda, dtype=dtype)
+    cls = RWKV7HIP if dtype == torch.float16 else RWKV7HIPBF16
+    frag, plain = cls(w), cls(w)
+    plain.dev = pack_device_weights(w, fragments=False)
+    toks = _tokens(B * T, 512, seed=B + T).view(B, T).to(cuda)
+    got = []
+    for model in (frag, plain):
+        S = State(w.L, w.C, 64, device=cuda, dtype=dtype, batch=B)
+        g = torch.Generator().manual_seed(3)
+        for t in S.arenas:
+            t.copy_(torch.randn(t.shape, generator=g) * 0.1)
+        lg = torch.empty(0)
+        if T > 1:
+            model.prefill(toks, S)
+        else:
+            lg, S = model.decode(toks.reshape(B), S)
+        got.append((lg, *S.arenas))
+    unit = 2.0**-10 if dtype == torch.float16 else 2.0**-7
+    for i, (x, y) in enumerate(zip(*got)):
+        x, y = x.float(), y.float()
+        if i == 2:
+            assert float((x - y).norm() / y.norm()) < 1e-5
+        elif x.numel():
+            assert float(((x - y).abs() / y.abs().clamp_min(float(y.abs().max()) * 2.0**-6)).max()) <= 2 * unit
