@@ -45,6 +45,8 @@ struct TmixDecodeArgs {
   int C, H, rv, rw, ra, rg, layer0;
   uint16_t *yg16;
   int bf;  // w_lora2, shift and yg16 are bfloat16 (else half)
+  // the second LoRA matrices v, w, a, g in fragment order, or null (w_lora2)
+  const uint16_t *f_l2[4] = {nullptr, nullptr, nullptr, nullptr};
   uint16_t *yg_split = nullptr;  // when set: the gated output in split order (split_put1) instead
 };
 int launch_tmix_decode(const TmixDecodeArgs &a, int B, hipStream_t st);

@@ -25,10 +25,21 @@ namespace rwkv7 {
 
 constexpr int kMaxRanks = 512;  // SR = rv + rw + ra + rg of the batched decode core
 
-template <bool BF>
+// FRAG: the second LoRA matrices from the fragment arena (a.f_l2), else the
+// row-major w_lora2. In fragment order a wave's load is a contiguous KiB, 16
+// channels x 32 ranks; row-major, each lane reads its own channel's row, 64
+// lines per load of which 16 bytes are used, and the eight workgroups of a CU
+// thrash its L1. Taken from kFragRanks ranks in all and kFragGroups
+// workgroups, four per CU (measured, us, row-major / fragments: 1.5B, ranks
+// 96/96/64/256, 3 sequences 8.2 / 9.3, 64 sequences 31.8 / 27.5; 0.4B, ranks
+// 64/64/32/128, 24 sequences 10.0 / 11.2, 128 sequences 24.2 / 24.3).
+constexpr int kFragRanks = 384, kFragGroups = 1024;
+template <bool BF, bool FRAG>
 __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
   using T16 = F16T<BF>;
-  __shared__ float s_lora[kMaxRanks];
+  // the first steps after their activations; FRAG: each gate's padded with
+  // zeros to whole k-steps of 32
+  __shared__ __align__(16) float s_lora[kMaxRanks + (FRAG ? 4 * 32 : 0)];
   __shared__ float s_d[4][kN];
   __shared__ float s_r[kN], s_w[kN], s_k[kN], s_v[kN], s_a[kN], s_b[kN], s_g[kN], s_y[kN];
   __shared__ float s_rk;
@@ -40,15 +51,74 @@ __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
   const float *prow = a.proj + (int64_t)b * a.ldp;
   const float *vec = a.vec;
 
-  for (int i = t; i < SR; i += 256) {
-    float x = prow[3 * C + i];
-    if (i >= a.rv && i < a.rv + a.rw) x = tanhf(x);
-    else if (i >= a.rv + a.rw + a.ra) x = sigmoidf_(x);
-    s_lora[i] = x;
+  const int nv = FRAG ? (a.rv + 31) / 32 : 0, nw = FRAG ? (a.rw + 31) / 32 : 0, na = FRAG ? (a.ra + 31) / 32 : 0,
+            ng = FRAG ? (a.rg + 31) / 32 : 0;  // k-steps of each gate
+  if constexpr (FRAG) {
+    for (int i = t; i < 32 * (nv + nw + na + ng); i += 256) {
+      const int ks = i >> 5;
+      const int g = ks < nv ? 0 : ks < nv + nw ? 1 : ks < nv + nw + na ? 2 : 3;
+      const int r = i - 32 * (g == 0 ? 0 : g == 1 ? nv : g == 2 ? nv + nw : nv + nw + na);
+      const int R = g == 0 ? a.rv : g == 1 ? a.rw : g == 2 ? a.ra : a.rg;
+      const int off = g == 0 ? 0 : g == 1 ? a.rv : g == 2 ? a.rv + a.rw : a.rv + a.rw + a.ra;
+      float x = prow[3 * C + off + min(r, R - 1)];
+      if (g == 1) x = tanhf(x);
+      else if (g == 3) x = sigmoidf_(x);
+      s_lora[i] = r < R ? x : 0.f;
+    }
+  } else {
+    for (int i = t; i < SR; i += 256) {
+      float x = prow[3 * C + i];
+      if (i >= a.rv && i < a.rv + a.rw) x = tanhf(x);
+      else if (i >= a.rv + a.rw + a.ra) x = sigmoidf_(x);
+      s_lora[i] = x;
+    }
   }
   __syncthreads();
 
-  {  // LoRA second step: thread -> (gate q, channel c)
+  if constexpr (FRAG) {
+    // wave -> 16 channels; lane -> channel lane % 16, ranks 8 (lane / 16) .. of
+    // each k-step; the four lane groups are summed at the end
+    const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), strip = h * (kN / 16) + wv;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    const float *act = s_lora + 8 * (lane >> 4);
+    auto gate = [&](const uint16_t *f, int n, float &sum) __attribute__((always_inline)) {
+      const uint4 *w = reinterpret_cast<const uint4 *>(f + (int64_t)strip * n * 512) + lane;
+      constexpr int NB = 4;
+      for (int k0 = 0; k0 < n; k0 += NB) {
+        uint4 q[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) q[b] = w[64 * min(k0 + b, n - 1)];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          if (k0 + b < n) {
+            float wf[8];
+            T16::to_f8(q[b], wf);
+            const float4 u = *reinterpret_cast<const float4 *>(act + 32 * (k0 + b));
+            const float4 z = *reinterpret_cast<const float4 *>(act + 32 * (k0 + b) + 4);
+            sum = fmaf(wf[0], u.x, sum);
+            sum = fmaf(wf[1], u.y, sum);
+            sum = fmaf(wf[2], u.z, sum);
+            sum = fmaf(wf[3], u.w, sum);
+            sum = fmaf(wf[4], z.x, sum);
+            sum = fmaf(wf[5], z.y, sum);
+            sum = fmaf(wf[6], z.z, sum);
+            sum = fmaf(wf[7], z.w, sum);
+          }
+        }
+      }
+      act += 32 * n;
+    };
+    gate(a.f_l2[0], nv, acc[0]);
+    gate(a.f_l2[1], nw, acc[1]);
+    gate(a.f_l2[2], na, acc[2]);
+    gate(a.f_l2[3], ng, acc[3]);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      acc[g] += __shfl_xor(acc[g], 16);
+      acc[g] += __shfl_xor(acc[g], 32);
+      if (lane < 16) s_d[g][16 * wv + lane] = acc[g];
+    }
+  } else {  // LoRA second step: thread -> (gate q, channel c)
     const int c = t & (kN - 1), q = t >> 6;
     const int off = q == 0 ? 0 : q == 1 ? a.rv : q == 2 ? a.rv + a.rw : a.rv + a.rw + a.ra;
     const int R = q == 0 ? a.rv : q == 1 ? a.rw : q == 2 ? a.ra : a.rg;
@@ -63,7 +133,18 @@ __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
     }
     s_d[q][c] = acc;
   }
-  __syncthreads();
+  // this thread's piece of the wkv state (row t >> 2, 16 key columns); FRAG: in
+  // flight while wave 0 forms the gates (bare barriers until its use: a fence
+  // would wait for it)
+  float4 *Sp = reinterpret_cast<float4 *>(a.rnn + (((int64_t)b * a.H + h) * kN + (t >> 2)) * kN + (t & 3) * 16);
+  float4 S4[4];
+  if constexpr (FRAG) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) S4[q] = Sp[q];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+    __syncthreads();
+  }
 
   if (t < kN) {  // gates, one lane per channel of this head
     const int ch = h * kN + t;
@@ -87,15 +168,20 @@ __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
     if (t == 0) s_rk = rk;
     if (a.shift) a.shift[(int64_t)b * C + ch] = T16::from_f(a.xln[(int64_t)b * C + ch]);
   }
-  __syncthreads();
+  if constexpr (FRAG) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) S4[q] = Sp[q];
+  }
 
   {  // wkv7: thread -> row i, 16 key columns
     const int i = t >> 2, j0 = (t & 3) * 16;
-    float4 *Sp = reinterpret_cast<float4 *>(a.rnn + (((int64_t)b * a.H + h) * kN + i) * kN + j0);
     float S[16];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      float4 u = Sp[q];
+      const float4 u = S4[q];
       S[4 * q] = u.x; S[4 * q + 1] = u.y; S[4 * q + 2] = u.z; S[4 * q + 3] = u.w;
     }
     float sa = 0.f;
@@ -134,8 +220,14 @@ __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
 int launch_tmix_decode(const TmixDecodeArgs &a, int B, hipStream_t st) {
   // the LoRA rows are read 8 ranks (16 bytes) at a time, all ranks staged in LDS
   if (a.rv + a.rw + a.ra + a.rg > kMaxRanks || a.rv % 8 || a.rw % 8 || a.ra % 8 || a.rg % 8) return RWKV7_ESHAPE;
-  if (a.bf) tmix_decode_kernel<true><<<dim3(a.H, B), 256, 0, st>>>(a);
-  else tmix_decode_kernel<false><<<dim3(a.H, B), 256, 0, st>>>(a);
+  const dim3 grid(a.H, B);
+  if (a.f_l2[0] && a.rv + a.rw + a.ra + a.rg >= kFragRanks && a.H * B >= kFragGroups) {
+    if (a.bf) tmix_decode_kernel<true, true><<<grid, 256, 0, st>>>(a);
+    else tmix_decode_kernel<false, true><<<grid, 256, 0, st>>>(a);
+  } else {
+    if (a.bf) tmix_decode_kernel<true, false><<<grid, 256, 0, st>>>(a);
+    else tmix_decode_kernel<false, false><<<grid, 256, 0, st>>>(a);
+  }
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;
 }
