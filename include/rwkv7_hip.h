@@ -450,7 +450,7 @@ typedef struct rwkv7_sampling {
  * distribution (one-hot when greedy). No host sync. With a workspace of at
  * least rwkv7_sample_workspace_bytes(B, V) bytes, a call with temperature >
  * 0, 1 <= top_k <= 128 and no probs spreads each row over V / 2048
- * workgroups (each keeps the candidates of its slice of the row, a second
+ * wavefronts (each keeps the candidates of its slice of the row, a second
  * launch draws from them) and draws the same token as without it; otherwise
  * (workspace NULL) one workgroup per row does all of it.
  * Stands in for sample_logits (demo/sampling.py:13-70) as called by

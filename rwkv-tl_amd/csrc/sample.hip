@@ -501,129 +501,358 @@ __global__ __launch_bounds__(kSmpThreads) void sample_kernel(SampleArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Top-k over many CUs (temperature > 0, 1 <= top_k <= kCandMax, no probs):
-// every token top-k keeps is among the top_k largest of its own slice of the
-// row, so the row is cut into slices of kCandSlice logits, each workgroup of
-// sample_cand_kernel keeps the values of its slice >= the slice's top_k-th
-// largest (ties included; exact, by the same selection as above) in index
-// order, and sample_finish_kernel runs draw_tempered on those candidates,
-// which hold the same values at the same vocabulary positions as the
-// one-workgroup kernel would: the thresholds, the fixed-point masses, the
-// draw and therefore the token are identical. A slice with more than
-// kCandMax candidates (a tie group at its threshold) marks its count -1, and
-// the row is sampled by sample_row instead.
+// Top-k over many CUs (temperature > 0, 1 <= top_k <= kCandMax, no probs): the
+// row is cut into slices of kCandSlice logits, one wave each
+// (sample_cand_kernel), that keep a superset of the values top-k can keep, in
+// index order; sample_finish_kernel finds the exact thresholds among them and
+// draws. The candidates hold the same values at the same vocabulary positions
+// as in the one-workgroup kernel and every sum is exact, so the token is the
+// same.
+//
+// What bounds the two kernels is not the row's bytes (128 KB) but the chain of
+// dependent selections. As histogram passes of a 1024-thread workgroup, with
+// barriers between them, they took 15.3 + 23.4 us at 16 f16 rows of V = 65536,
+// top-k 50, top-p 0.9; now 9.9 + 14.7 (top-k 100: 15.4 + 28.2 -> 12.0 + 16.0;
+// 64 f32 rows, top-k 20, top-p 1: 48.5 + 20.2 -> 13.6 + 12.6; one bf16 row,
+// top-k 100, top-p 1: 11.2 + 21.0 -> 11.6 + 12.4). A wave alone finds the k-th
+// largest of the values its lanes hold with 32 ballots (kth_key), no LDS and
+// no barrier, so:
+// * a slice's floor is the top_k-th largest of the 128 maxima of its lanes'
+//   16-value halves (from top_k = 65 of the 512 maxima of 4 values): at least
+//   top_k values of the slice reach it, so the row's top_k-th largest does
+//   too, and 1.1-1.2 top_k values pass (more than kSliceCap, at top_k near it:
+//   the slice's exact top_k-th largest instead);
+// * the row's floor is the larger of two bounds on the row's top_k-th largest:
+//   the largest slice floor, and the smallest over the slices of their
+//   ceil(top_k / slices)-th largest half maximum (each slice has that many
+//   values from there up) -- a few hundred of the candidates pass it;
+// * if at most kFinMax pass, wave 0 holds them, eight per lane, and takes the
+//   exact top-k threshold, the top-p threshold and the draw by itself; else the
+//   workgroup runs draw_tempered on all candidates.
+// A slice with more than kSliceCap values at its floor (a tie group) marks its
+// count -1, and the row is sampled by sample_row instead.
 // ---------------------------------------------------------------------------
-constexpr int kCandSlice = 2 * kSmpThreads;  // 2 logits per thread
-constexpr int kCandMax = 128;                // candidates kept per slice
+constexpr int kCandE = 32;                   // logits per lane of a slice
+constexpr int kCandSlice = kCandE * kWave;   // 2048
+constexpr int kCandMax = 128;                // the largest top_k: half maxima per slice
+constexpr int kSliceCap = 128;               // candidates kept per slice
 constexpr int kCandSlices = kSmpMaxV / kCandSlice;
-constexpr int kCandE = kCandSlices * kCandMax / kSmpThreads;  // candidates per thread in the finish
+constexpr int kFinE = kCandSlices * kSliceCap / kSmpThreads;  // candidates per thread in the finish
+constexpr int kFinMax = 512;                 // candidates wave 0 finishes by itself
+static_assert(kFinE == 4 && kCandSlices == 32, "a half wave per slice in the finish");
 
 struct CandBuf {
-  int *cnt;     // [B][G]: candidates of each slice, -1 when more than kCandMax
-  float *val;   // [B][G][kCandMax]
-  int *idx;     // [B][G][kCandMax]
+  int *cnt;          // [B][G]: candidates of each slice, -1 when more than kSliceCap
+  uint32_t *floors;  // [B][G][2]: keys of the slice's two bounds
+  float *val;        // [B][G][kSliceCap]
+  int *idx;          // [B][G][kSliceCap]
   int G;
 };
 
-template <int FMT>
-RWKV7_DEV float load1(const void *row_ptr, int i) {
-  if (FMT == 1) return static_cast<const float *>(row_ptr)[i];
-  return F16T<FMT == 2>::to_f(static_cast<const uint16_t *>(row_ptr)[i]);
+// The key of a value in the order-preserving integer order, 0 for one that is
+// not there (-inf or NaN).
+RWKV7_DEV uint32_t vkey(float x) { return x > -kInf ? okey(x) : 0u; }
+
+// The k-th largest (k >= 1) of the N keys each lane of the wave holds, 0 when
+// fewer than k are nonzero: bit by bit, the largest key that k of them reach.
+template <int N>
+RWKV7_DEV uint32_t kth_key(const uint32_t (&key)[N], int k) {
+  uint32_t t = 0;
+#pragma unroll 1
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t c = t | (1u << bit);
+    int n = 0;
+#pragma unroll
+    for (int e = 0; e < N; ++e) n += __popcll(__ballot(key[e] >= c));
+    if (n >= k) t = c;
+  }
+  return t;
 }
 
-template <int FMT>
-__global__ __launch_bounds__(kSmpThreads) void sample_cand_kernel(SampleArgs a, CandBuf cb) {
-  __shared__ SampleLds s;
-  const int g = blockIdx.x, row = blockIdx.y, V = a.V;
+// The 32 logits of a lane, V past the row (-inf there); VEC: 16-byte loads.
+template <bool VEC, int FMT>
+__global__ __launch_bounds__(256) void sample_cand_kernel(SampleArgs a, CandBuf cb) {
+  const int lane = threadIdx.x & 63, g = 4 * blockIdx.x + (threadIdx.x >> 6), row = blockIdx.y, V = a.V;
+  if (g >= cb.G) return;
   const void *src = static_cast<const char *>(a.logits) + (int64_t)row * a.ld * (FMT == 1 ? 4 : 2);
-  const int i0 = g * kCandSlice + 2 * threadIdx.x;
-  float l[2];
+  const int i0 = g * kCandSlice + kCandE * lane;
+  float l[kCandE];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) l[e] = i0 + e < V ? load1<FMT>(src, i0 + e) : -kInf;
+  for (int c = 0; c < kCandE / 8; ++c) load8<VEC, FMT>(src, i0 + 8 * c, V, &l[8 * c]);
   if (a.seen && a.pen != 1.f) {  // the same operations, in the same order, as sample_row
-    const uint32_t *sr = a.seen + (int64_t)row * a.seen_ld;
+    const uint32_t w = i0 < V ? a.seen[(int64_t)row * a.seen_ld + (i0 >> 5)] : 0u;
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int i = i0 + e;
-      if (i < V && ((sr[i >> 5] >> (i & 31)) & 1u)) l[e] = l[e] > 0.f ? l[e] / a.pen : l[e] * a.pen;
-    }
+    for (int e = 0; e < kCandE; ++e)
+      if ((w >> e) & 1u) l[e] = l[e] > 0.f ? l[e] / a.pen : l[e] * a.pen;
   }
 #pragma unroll
-  for (int e = 0; e < 2; ++e) l[e] = (l[e] + 0.f) / a.temp;
-  float lo = kInf, hi = -kInf;
+  for (int e = 0; e < kCandE; ++e) l[e] = (l[e] + 0.f) / a.temp;
+  // maxima of the lane's eights of four values, then of its halves
+  uint32_t pk[8], hk[2];
 #pragma unroll
-  for (int e = 0; e < 2; ++e)
-    if (l[e] > -kInf) lo = fminf(lo, l[e]), hi = fmaxf(hi, l[e]);
-  block_minmax(lo, hi, s);
-  // the slice's top_k-th largest value (lo when it holds fewer values)
-  const float u = select_gt<false, 2>(l, lo, hi, hi, (u64)(a.top_k - 1), s);
-  bool keep[2];
+  for (int q = 0; q < 8; ++q) pk[q] = vkey(fmaxf(fmaxf(l[4 * q], l[4 * q + 1]), fmaxf(l[4 * q + 2], l[4 * q + 3])));
+#pragma unroll
+  for (int h = 0; h < 2; ++h) hk[h] = max(max(pk[4 * h], pk[4 * h + 1]), max(pk[4 * h + 2], pk[4 * h + 3]));
+  const uint32_t fl = a.top_k <= kWave ? kth_key<2>(hk, a.top_k) : kth_key<8>(pk, a.top_k);
+  const uint32_t few = kth_key<2>(hk, (a.top_k + cb.G - 1) / cb.G);
+  float thr = fl ? okey_inv(fl) : -kInf;
+  int own, inc, total;  // this lane's kept values, their inclusive prefix over the lanes, the slice's
+  auto count = [&]() {
+    own = 0;
+#pragma unroll
+    for (int e = 0; e < kCandE; ++e) own += l[e] > -kInf && l[e] >= thr;
+    inc = own;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int o = __shfl_up(inc, d);
+      if (lane >= d) inc += o;
+    }
+    total = __shfl(inc, kWave - 1);
+  };
+  count();
+  if (total > kSliceCap) {  // the slice's exact top_k-th largest (top_k near kCandMax, or ties)
+    uint32_t key[kCandE];
+#pragma unroll
+    for (int e = 0; e < kCandE; ++e) key[e] = vkey(l[e]);
+    const uint32_t k = kth_key<kCandE>(key, a.top_k);
+    thr = k ? okey_inv(k) : -kInf;
+    count();
+  }
+  const int64_t slot = (int64_t)row * cb.G + g;
+  if (lane == 0) {
+    cb.cnt[slot] = total <= kSliceCap ? total : -1;
+    cb.floors[2 * slot] = fl;
+    cb.floors[2 * slot + 1] = few;
+  }
+  if (total > kSliceCap) return;
+  int64_t at = slot * kSliceCap + inc - own;
+#pragma unroll
+  for (int e = 0; e < kCandE; ++e) {
+    if (l[e] > -kInf && l[e] >= thr) {
+      cb.val[at] = l[e];
+      cb.idx[at] = i0 + e;
+      ++at;
+    }
+  }
+}
+
+RWKV7_DEV u64 wave_sum64(u64 v) {
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) v += shfl_xor64(v, d);
+  return v;
+}
+
+// draw_tempered for the values wave 0 holds (kFinMax / 64 per lane, in
+// vocabulary order lane by lane; -inf: none), by that wave alone. buf: kFinMax
+// floats of LDS. Returns the token on the lane that draws it, -1 on the others.
+template <int N>
+RWKV7_DEV int draw_in_wave(float (&l)[N], const int (&ix)[N], const SampleArgs &a, int row, float *buf) {
+  const int L = threadIdx.x;
+  uint32_t key[N];
+  float m = -kInf;
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    key[e] = vkey(l[e]);
+    m = fmaxf(m, l[e]);
+  }
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+  const uint32_t tk = kth_key<N>(key, a.top_k);
+  float thr = tk ? okey_inv(tk) : -kInf;  // sampling.py:56-60
   int own = 0;
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    keep[e] = l[e] > -kInf && l[e] >= u;
-    own += keep[e];
+  for (int e = 0; e < N; ++e) {
+    if (!(l[e] >= thr)) l[e] = -kInf;
+    own += l[e] > -kInf;
   }
-  u64 total;
-  int at = (int)block_excl_scan((u64)own, total, s);
-  const int64_t slot = (int64_t)row * cb.G + g;
-  if (threadIdx.x == 0) cb.cnt[slot] = total <= (u64)kCandMax ? (int)total : -1;
-  if (total <= (u64)kCandMax) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      if (keep[e]) {
-        cb.val[slot * kCandMax + at] = l[e];
-        cb.idx[slot * kCandMax + at] = i0 + e;
-        ++at;
-      }
-    }
-  }
-}
-
-template <bool VEC, int FMT>
-__global__ __launch_bounds__(kSmpThreads) void sample_finish_kernel(SampleArgs a, CandBuf cb) {
-  __shared__ SampleLds s;
-  __shared__ int s_off[kCandSlices + 1];
-  __shared__ int s_bad;
-  const int row = blockIdx.x, G = cb.G;
-  if (threadIdx.x < kWave) {  // slice offsets: inclusive prefix of the counts
-    const int L = threadIdx.x;
-    const int c = L < G ? cb.cnt[(int64_t)row * G + L] : 0;
-    int inc = c < 0 ? 0 : c;
+  if (a.top_p < 1.f) {  // sampling.py:62-68
+    int inc = own;
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       const int o = __shfl_up(inc, d);
       if (L >= d) inc += o;
     }
-    const bool bad = __ballot(c < 0) != 0;
-    if (L <= kCandSlices - 1) s_off[L + 1] = inc;
-    if (L == 0) {
-      s_off[0] = 0;
-      s_bad = bad;
+    const int total = __shfl(inc, kWave - 1);
+    u64 z = 0;
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+      if (l[e] > -kInf) z += mass(l[e], m);
+    z = wave_sum64(z);
+    const u64 W = (u64)((double)a.top_p * (double)z);
+    if (total <= 2 * kWave) {  // sorted over the lanes (value i on lane i % 64), the first whose running mass exceeds W
+      int at = inc - own;
+#pragma unroll
+      for (int e = 0; e < N; ++e)
+        if (l[e] > -kInf) buf[at++] = l[e];
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      float v0 = L < total ? buf[L] : -kInf, v1 = L + kWave < total ? buf[L + kWave] : -kInf;
+      const bool two = total > kWave;  // uniform
+      auto cmp = [&](float &v, int i, int k, int j) {  // one descending bitonic step of value i against value i ^ j
+        const float o = __shfl_xor(v, j);
+        const bool take_max = ((i & j) == 0) == ((i & k) == 0);
+        v = take_max ? fmaxf(v, o) : fminf(v, o);
+      };
+#pragma unroll
+      for (int k = 2; k <= kWave; k <<= 1) {
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          cmp(v0, L, k, j);
+          if (two) cmp(v1, L + kWave, k, j);
+        }
+      }
+      if (two) {  // merge the two halves, sorted in opposite directions
+        const float hi = fmaxf(v0, v1), lo = fminf(v0, v1);
+        v0 = hi;
+        v1 = lo;
+#pragma unroll
+        for (int j = kWave / 2; j > 0; j >>= 1) {
+          cmp(v0, L, 2 * kWave, j);
+          cmp(v1, L + kWave, 2 * kWave, j);
+        }
+      }
+      auto scan = [&](float v) {
+        u64 c = v > -kInf ? mass(v, m) : 0ull;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+          const u64 o = shfl_up64(c, d);
+          if (L >= d) c += o;
+        }
+        return c;
+      };
+      const u64 c0 = scan(v0);
+      u64 pass = __ballot(c0 > W);
+      if (pass == 0 && two) {  // (one of them passes: the last value's running mass is z > W)
+        const u64 c1 = scan(v1) + (u64)(uint32_t)__shfl((int)(uint32_t)c0, kWave - 1) +
+                       ((u64)(uint32_t)__shfl((int)(uint32_t)(c0 >> 32), kWave - 1) << 32);
+        pass = __ballot(c1 > W);
+        v0 = v1;
+      }
+      thr = __shfl(v0, __ffsll((unsigned long long)pass) - 1);
+    } else {  // the largest key whose mass from there up exceeds W, bit by bit
+      uint32_t t = 0;
+#pragma unroll 1
+      for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t c = t | (1u << bit);
+        u64 q = 0;
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          if (l[e] > -kInf && key[e] >= c) q += mass(l[e], m);
+        if (wave_sum64(q) > W) t = c;
+      }
+      thr = okey_inv(t);
     }
   }
-  __syncthreads();
-  if (s_bad) {  // a tie group overflowed a slice: the whole row here
+  u64 own_z = 0;
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    if (l[e] < thr) l[e] = -kInf;
+    if (l[e] > -kInf) own_z += mass(l[e], m);
+  }
+  u64 inc = own_z;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const u64 o = shfl_up64(inc, d);
+    if (L >= d) inc += o;
+  }
+  const u64 excl = inc - own_z, z = wave_sum64(own_z);
+  uint32_t c[4] = {a.off_lo, a.off_hi, (uint32_t)row, 0u};
+  philox4x32_10(c, a.seed_lo, a.seed_hi);
+  const u64 target = __umul64hi(z, (u64)c[0] | ((u64)c[1] << 32));  // in [0, z)
+  int token = -1;
+  if (excl <= target && target < excl + own_z) {
+    u64 acc = excl;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      if (l[e] > -kInf) acc += mass(l[e], m);
+      if (token < 0 && acc > target) token = ix[e];
+    }
+  }
+  return token;
+}
+
+template <bool VEC, int FMT>
+__global__ __launch_bounds__(kSmpThreads) void sample_finish_kernel(SampleArgs a, CandBuf cb) {
+  __shared__ SampleLds s;
+  __shared__ int s_wave[kSmpWaves + 1], s_ix[kFinMax];
+  const int row = blockIdx.x, G = cb.G, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  // half wave -> slice, four candidates per thread
+  const int g = t >> 5, p0 = kFinE * (t & 31);
+  const int64_t slot = (int64_t)row * G + min(g, G - 1);
+  const int cnt = g < G ? cb.cnt[slot] : 0;
+  float l[kFinE];
+  int ix[kFinE];
+  {
+    // (all of a slice's places are readable; those past its count are dropped)
+    const float4 v = p0 < cnt ? *reinterpret_cast<const float4 *>(cb.val + slot * kSliceCap + p0) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int4 q = p0 < cnt ? *reinterpret_cast<const int4 *>(cb.idx + slot * kSliceCap + p0) : make_int4(0, 0, 0, 0);
+    const float vv[4] = {v.x, v.y, v.z, v.w};
+    const int qq[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int e = 0; e < kFinE; ++e) {
+      l[e] = p0 + e < cnt ? vv[e] : -kInf;
+      ix[e] = p0 + e < cnt ? qq[e] : a.V;
+    }
+  }
+  // the row's floor: every wave from the slices' bounds (lane -> slice)
+  const int gl = min(lane & 31, G - 1);
+  const uint32_t *fp = cb.floors + 2 * ((int64_t)row * G + gl);
+  uint32_t top = fp[0], few = fp[1];
+#pragma unroll
+  for (int d = 1; d < 32; d <<= 1) {
+    top = max(top, (uint32_t)__shfl_xor((int)top, d));
+    few = min(few, (uint32_t)__shfl_xor((int)few, d));
+  }
+  const uint32_t fkey = max(top, few);
+  const float fl = fkey ? okey_inv(fkey) : -kInf;
+  if (__syncthreads_or(cnt < 0)) {  // a tie group overflowed a slice: the whole row here
     put_token(a, row, sample_row<VEC, FMT>(a, row, s));
     return;
   }
-  const int n = s_off[G];
-  float l[kCandE];
-  int ix[kCandE];
+  // candidates from the floor up, compacted in order
+  int own = 0;
 #pragma unroll
-  for (int e = 0; e < kCandE; ++e) {
-    const int d = kCandE * threadIdx.x + e;
-    l[e] = -kInf;
-    ix[e] = a.V;
-    if (d < n) {
-      int g = 0;
-      while (g + 1 < G && s_off[g + 1] <= d) ++g;
-      const int64_t at = ((int64_t)row * G + g) * kCandMax + (d - s_off[g]);
-      l[e] = cb.val[at];
-      ix[e] = cb.idx[at];
+  for (int e = 0; e < kFinE; ++e) own += l[e] > -kInf && l[e] >= fl;
+  int inc = own;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int o = __shfl_up(inc, d);
+    if (lane >= d) inc += o;
+  }
+  if (lane == kWave - 1) s_wave[wv] = inc;
+  __syncthreads();
+  int base = 0, n = 0;
+#pragma unroll
+  for (int w = 0; w < kSmpWaves; ++w) {
+    const int c = s_wave[w];
+    base += w < wv ? c : 0;
+    n += c;
+  }
+  if (n > kFinMax) {  // block-uniform
+    put_token(a, row, draw_tempered<kFinE, false>(l, [&ix](int e) { return ix[e]; }, a, row, nullptr, s));
+    return;
+  }
+  int at = base + inc - own;
+#pragma unroll
+  for (int e = 0; e < kFinE; ++e) {
+    if (l[e] > -kInf && l[e] >= fl) {
+      s.cand[at] = l[e];
+      s_ix[at] = ix[e];
+      ++at;
     }
   }
-  put_token(a, row, draw_tempered<kCandE, false>(l, [&ix](int e) { return ix[e]; }, a, row, nullptr, s));
+  __syncthreads();
+  if (wv > 0) return;
+  constexpr int N = kFinMax / kWave;
+  float x[N];
+  int xi[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const int d = N * lane + e;
+    x[e] = d < n ? s.cand[d] : -kInf;
+    xi[e] = d < n ? s_ix[d] : a.V;
+  }
+  put_token(a, row, draw_in_wave<N>(x, xi, a, row, s.cand + kFinMax));
 }
 
 }  // namespace
@@ -631,7 +860,7 @@ __global__ __launch_bounds__(kSmpThreads) void sample_finish_kernel(SampleArgs a
 
 static int64_t cand_bytes(int B, int G) {
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
-  return al((int64_t)B * G * 4) + 2 * al((int64_t)B * G * rwkv7::kCandMax * 4);
+  return al((int64_t)B * G * 4) + al((int64_t)B * G * 8) + 2 * al((int64_t)B * G * rwkv7::kSliceCap * 4);
 }
 
 extern "C" int64_t rwkv7_sample_workspace_bytes(int32_t B, int32_t V) {
@@ -670,17 +899,20 @@ extern "C" int rwkv7_sample(const void *logits, int32_t logits_dtype, int64_t ld
   const bool cand = workspace && workspace_bytes >= cand_bytes(B, G) && a.temp > 0.f && a.top_k >= 1 &&
                     a.top_k <= kCandMax && a.top_k < V && !probs && G >= 2;
   if (cand) {
+    auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
     char *w = static_cast<char *>(workspace);
-    const int64_t c0 = cand_bytes(B, G) - 2 * (((int64_t)B * G * kCandMax * 4 + 255) / 256 * 256);
+    const int64_t c0 = al((int64_t)B * G * 4), c1 = c0 + al((int64_t)B * G * 8), nv = al((int64_t)B * G * kSliceCap * 4);
     CandBuf cb;
     cb.cnt = reinterpret_cast<int *>(w);
-    cb.val = reinterpret_cast<float *>(w + c0);
-    cb.idx = reinterpret_cast<int *>(w + c0 + ((int64_t)B * G * kCandMax * 4 + 255) / 256 * 256);
+    cb.floors = reinterpret_cast<uint32_t *>(w + c0);
+    cb.val = reinterpret_cast<float *>(w + c1);
+    cb.idx = reinterpret_cast<int *>(w + c1 + nv);
     cb.G = G;
+    const dim3 grid((G + 3) / 4, B);
     switch (logits_dtype) {
-      case 0: sample_cand_kernel<0><<<dim3(G, B), kSmpThreads, 0, st>>>(a, cb); break;
-      case 1: sample_cand_kernel<1><<<dim3(G, B), kSmpThreads, 0, st>>>(a, cb); break;
-      default: sample_cand_kernel<2><<<dim3(G, B), kSmpThreads, 0, st>>>(a, cb); break;
+      case 0: vec ? sample_cand_kernel<true, 0><<<grid, 256, 0, st>>>(a, cb) : sample_cand_kernel<false, 0><<<grid, 256, 0, st>>>(a, cb); break;
+      case 1: vec ? sample_cand_kernel<true, 1><<<grid, 256, 0, st>>>(a, cb) : sample_cand_kernel<false, 1><<<grid, 256, 0, st>>>(a, cb); break;
+      default: vec ? sample_cand_kernel<true, 2><<<grid, 256, 0, st>>>(a, cb) : sample_cand_kernel<false, 2><<<grid, 256, 0, st>>>(a, cb); break;
     }
     RWKV7_CHECK_LAUNCH();
     switch (logits_dtype) {

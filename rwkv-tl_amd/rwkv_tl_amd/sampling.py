@@ -4,7 +4,7 @@
 penalty on ``seen``, greedy argmax when ``temperature`` is None or <= 0, else
 temperature, top-k, top-p and one draw, along the last dimension. All of it is
 one call of ``rwkv7_sample``: one workgroup per row, or for top-k sampling
-one workgroup per 2048 logits that keeps its slice's candidates and a second
+one wavefront per 2048 logits that keeps its slice's candidates and a second
 launch that draws from them (the same token either way). The
 draw comes from a counter-based generator (Philox4x32-10) keyed by a seed
 taken from torch's CPU generator, so ``torch.manual_seed`` makes it

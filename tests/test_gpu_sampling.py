@@ -322,3 +322,25 @@ def test_sampler_with_workspace_updates_seen_like_without():
             toks.append(out.cpu().clone())
         runs.append((torch.stack(toks), smp.seen.cpu()))
     assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
+
+
+@pytest.mark.parametrize("top_k,top_p", [(64, 0.9), (65, 0.9), (100, 0.97), (128, 1.0), (3, 0.5)])
+def test_candidate_path_on_uneven_rows(top_k, top_p):
+    """Rows whose largest values sit in one slice, whose slices hold fewer than
+    top_k values (-inf elsewhere), with NaNs and with coarse ties: the wave-wide
+    selections (one or two values per lane) and the slices' bounds pick the
+    token of the one-workgroup kernel, an integer result: equal."""
+    V = 65536
+    g = torch.Generator().manual_seed(top_k)
+    rows = torch.randn(6, V, generator=g)
+    rows[0, 8192:10240] += 9.0                      # one slice holds every kept value
+    rows[1, 40:] = float("-inf")                    # fewer values than top_k
+    rows[2, ::2] = float("nan")
+    rows[3] = (rows[3] * 4).round() / 4             # tie groups at every threshold
+    rows[4, 4096:] -= 30.0                          # the other slices' bounds far below
+    rows[5, ::1024] += 6.0                          # two values per slice stand out
+    for dtype in (torch.float32, torch.float16):
+        logits = rows.to(dtype).to(DEV)
+        for off in range(4):
+            a, b, _ = _both_paths(logits, 6, V, offset=off, temperature=0.9, top_k=top_k, top_p=top_p)
+            assert torch.equal(a, b), (dtype, off, a.tolist(), b.tolist())
