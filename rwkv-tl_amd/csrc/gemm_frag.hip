@@ -20,6 +20,8 @@
 // order, where the accumulator layout also becomes rows for vector stores.
 #include "rwkv7_kernels.h"
 
+#include <algorithm>
+
 namespace rwkv7 {
 
 constexpr int kFragProbs = 8;
@@ -51,13 +53,124 @@ RWKV7_DEV float frag_epi(int epi, float v) {
   }
 }
 
+// Output piece u of a thread: four columns of a row of the tile.
+template <int BM, int BN>
+RWKV7_DEV bool frag_piece(int u, int &row, int &col) {
+  const int e = (int)threadIdx.x + kFragThreads * u;
+  row = e / (BN / 4);
+  col = 4 * (e % (BN / 4));
+  return e < BM * BN / 4;
+}
+template <int BM, int BN>
+constexpr int kFragPieces = BM * BN / 4 / kFragThreads > 0 ? BM * BN / 4 / kFragThreads : 1;
+
+// The values an add epilogue accumulates into.
+template <int BM, int BN>
+RWKV7_DEV void frag_yres(const GemmProb &P, int M, int m0, int n0, float4 (&yres)[kFragPieces<BM, BN>]) {
+#pragma unroll
+  for (int u = 0; u < kFragPieces<BM, BN>; ++u) {
+    int row, col;
+    frag_piece<BM, BN>(u, row, col);
+    yres[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(P.Y) +
+                                                (int64_t)min(m0 + row, M - 1) * P.ldy + min(n0 + col, P.N - 4));
+  }
+}
+
+// A tile's SK partial products in LDS: summed in order, epilogue, stored.
+template <int BM, int BN, int SK, bool BF>
+RWKV7_DEV void frag_store(const FragGroup &g, const GemmProb &P, const float (*s_red)[BM][BN + 4],
+                          const float4 (&yres)[kFragPieces<BM, BN>], int m0, int n0, int split) {
+  constexpr int PPT = kFragPieces<BM, BN>;
+  const int M = g.M, N = P.N, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const bool add = P.epi == GEPI_ADD_F32;
+  const int epi = P.epi;
+  if (epi >= GEPI_SPLIT) {
+    // the next product's A: a wave per 16 x 32 block of the tile, one
+    // contiguous KiB per part; columns up to the next k-step are zeros
+    constexpr int NBLK = BM / 16 * (BN / 32);
+#pragma unroll
+    for (int q = 0; q < (NBLK + 7) / 8; ++q) {
+      const int blk = wv + 8 * q, row = 16 * (blk / (BN / 32)) + (lane & 15), col = 32 * (blk % (BN / 32)) + 8 * (lane >> 4);
+      const int m = m0 + row, n = n0 + col;
+      if (blk >= NBLK || m >= M || n >= (N + 31) / 32 * 32) continue;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll
+      for (int s = 0; s < SK; ++s) {
+        const float4 x = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
+        const float4 y = *reinterpret_cast<const float4 *>(&s_red[s][row][col + 4]);
+        v[0] += x.x;
+        v[1] += x.y;
+        v[2] += x.z;
+        v[3] += x.w;
+        v[4] += y.x;
+        v[5] += y.y;
+        v[6] += y.z;
+        v[7] += y.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = n + e < N ? frag_epi(epi, v[e]) : 0.f;
+      split_put8<BF>(static_cast<uint16_t *>(P.Y), (N + 31) / 32, m, n, v);
+    }
+    return;
+  }
+  const bool vec = N % 4 == 0 && P.ldy % 4 == 0;
+#pragma unroll
+  for (int u = 0; u < PPT; ++u) {
+    int row, col;
+    if (!frag_piece<BM, BN>(u, row, col)) continue;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < SK; ++s) {
+      const float4 q = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
+      v[0] += q.x;
+      v[1] += q.y;
+      v[2] += q.z;
+      v[3] += q.w;
+    }
+    const int m = m0 + row, n = n0 + col;
+    if (m >= M) continue;
+    if (n >= N) continue;
+    const int64_t o = (int64_t)m * P.ldy + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = frag_epi(epi, v[e]);
+    if (epi == GEPI_F16) {
+      uint16_t *y = static_cast<uint16_t *>(P.Y) + o;
+      uint16_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = F16T<BF>::from_f(v[e]);
+      if (vec) {
+        *reinterpret_cast<uint2 *>(y) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) y[e] = h[e];
+      }
+    } else {
+      float *y = static_cast<float *>(P.Y) + split * g.part_stride + o;
+      if (add) {
+        v[0] += yres[u].x;
+        v[1] += yres[u].y;
+        v[2] += yres[u].z;
+        v[3] += yres[u].w;
+      }
+      if (vec) {
+        *reinterpret_cast<float4 *>(y) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) y[e] = v[e];
+      }
+    }
+  }
+}
+
 // Workgroup order as in gemm.hip: the m-tiles of a column tile get indices 8
 // apart, so they run on one XCD and read W from its L2.
 template <int MB, int NB, int SM, int SN, int SK, int KB, bool BF>
 __global__ __launch_bounds__(kFragThreads) void gemm_frag_kernel(FragGroup g) {
   constexpr int BM = 16 * MB * SM, BN = 16 * NB * SN, LD = BN + 4;
-  constexpr int UPT = BM * BN / 4 / kFragThreads;  // 4-column output pieces per thread
-  constexpr int PPT = UPT > 0 ? UPT : 1;
   static_assert(SM * SN * SK * 64 == kFragThreads, "eight waves");
   __shared__ __align__(16) float s_red[SK][BM][LD];
 
@@ -128,23 +241,8 @@ __global__ __launch_bounds__(kFragThreads) void gemm_frag_kernel(FragGroup g) {
   load(0, 0);
   load(KB, 1);
   // the values an add epilogue accumulates into, behind the first operands
-  float4 yres[PPT];
-  const bool add = P.epi == GEPI_ADD_F32;
-  auto piece = [&](int u, int &row, int &col) {
-    const int e = tid + kFragThreads * u;
-    row = e / (BN / 4);
-    col = 4 * (e % (BN / 4));
-    return e < BM * BN / 4;
-  };
-  if (add) {
-#pragma unroll
-    for (int u = 0; u < PPT; ++u) {
-      int row, col;
-      piece(u, row, col);
-      yres[u] = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(P.Y) +
-                                                  (int64_t)min(m0 + row, M - 1) * P.ldy + min(n0 + col, N - 4));
-    }
-  }
+  float4 yres[kFragPieces<BM, BN>];
+  if (P.epi == GEPI_ADD_F32) frag_yres<BM, BN>(P, M, m0, n0, yres);
   __builtin_amdgcn_sched_barrier(0);
   for (int k = 0; k < len; k += 2 * KB) {
     compute(k, 0);
@@ -164,95 +262,166 @@ __global__ __launch_bounds__(kFragThreads) void gemm_frag_kernel(FragGroup g) {
       for (int r = 0; r < 4; ++r)
         s_red[wk][16 * (wm * MB + i) + 4 * (lane >> 4) + r][16 * (wn * NB + j) + (lane & 15)] = acc[i][j][r];
   __syncthreads();
-  const int epi = P.epi;
-  if (epi >= GEPI_SPLIT) {
-    // the next product's A: a wave per 16 x 32 block of the tile, one
-    // contiguous KiB per part; columns up to the next k-step are zeros
-    constexpr int NBLK = BM / 16 * (BN / 32);
+  frag_store<BM, BN, SK, BF>(g, P, s_red, yres, m0, n0, split);
+}
+
+// Many rows: the operands by LDS DMA. The register loads above pass every
+// block through the CU's L1 once per wave that multiplies it -- twice for a
+// 2 x 2 arrangement of sub-tiles, 32 KiB per k-step of a 64 x 128 tile, 512
+// cycles of the L1's 64 bytes against 256 of MFMA. Here each block of a stage
+// (SK k-steps, one per slice) is one DMA into a ring of NBUF stages, NBUF - 1
+// ahead of the products, and the waves read it from LDS: a stage's fragments
+// are read into one of two register sets while the previous stage's are
+// multiplied.
+template <int MB, int NB, int SM, int SN, int SK, int NBUF, bool BF>
+__global__ __launch_bounds__(kFragThreads) void gemm_frag_ring_kernel(FragGroup g) {
+  constexpr int BM = 16 * MB * SM, BN = 16 * NB * SN, LD = BN + 4;
+  constexpr int NA = 2 * MB * SM, NW = NB * SN, BLK = SK * (NA + NW);  // blocks of a k-step, of a stage
+  constexpr int WPS = 8 / SK, PA = NA / WPS, PW = NW / WPS;            // waves per k-step, blocks each loads
+  static_assert(SM * SN * SK == 8 && NA % WPS == 0 && NW % WPS == 0, "eight waves, whole blocks each");
+  constexpr int kVm = (NBUF - 2) * (PA + PW);  // this wave's DMAs behind the stage waited for
+  static_assert(kVm < 64, "vmcnt field");
+  constexpr int kWaitImm = 0x0F70 | (kVm & 15) | ((kVm >> 4) << 14);
+  constexpr int kBytes = NBUF * BLK * 1024 > SK * BM * LD * 4 ? NBUF * BLK * 1024 : SK * BM * LD * 4;
+  __shared__ __align__(1024) unsigned char smem[kBytes];
+
+  const int bx = blockIdx.x;
+  int pi = 0;
 #pragma unroll
-    for (int q = 0; q < (NBLK + 7) / 8; ++q) {
-      const int blk = wv + 8 * q, row = 16 * (blk / (BN / 32)) + (lane & 15), col = 32 * (blk % (BN / 32)) + 8 * (lane >> 4);
-      const int m = m0 + row, n = n0 + col;
-      if (blk >= NBLK || m >= M || n >= (N + 31) / 32 * 32) continue;
-      float v[8];
+  for (int i = 1; i < kFragProbs; ++i) pi += (i < g.nprob && bx >= g.wg_begin[i]);
+  const GemmProb &P = g.p[pi];
+  const int local = bx - g.wg_begin[pi], mtl = g.m_tiles;
+  const int unit = local / (8 * mtl) * 8 + (local & 7), mt = local % (8 * mtl) / 8;
+  const int N = P.N, M = g.M, S = g.splits;
+  const int nt = unit / S, split = unit & (S - 1);
+  if (nt * BN >= N) return;  // padding of the last group of 8 units
+  const int m0 = mt * BM, n0 = nt * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wv % SM, wn = wv / SM % SN, wk = wv / (SM * SN);
+
+  const int nks = (P.K + 31) / 32, per = (nks + S - 1) / S;
+  const int k0 = split * per, len = max(0, min(nks, k0 + per) - k0);
+  const int nst = (len + SK - 1) / SK;
+  const int rot = nst > 0 ? 3 * mt % nst : 0;  // each row tile starts elsewhere, as above
+  const int mblk = (M + 15) / 16, nstrip = (N + 15) / 16;
+  // this wave's DMAs: blocks wq * PA .. of A (strip, part) and wq * PW .. of W,
+  // k-step ws of the stage; rows past the matrices clamp to their last block
+  const int ws = wv / WPS, wq = wv % WPS;
+  const i32x4 ra = buffer_words(P.A, mblk * nks * 2048), rw = buffer_words(P.Wf, nstrip * P.nksf * 1024);
+  int oa[PA], ow[PW];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 0.f;
-#pragma unroll
-      for (int s = 0; s < SK; ++s) {
-        const float4 x = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
-        const float4 y = *reinterpret_cast<const float4 *>(&s_red[s][row][col + 4]);
-        v[0] += x.x;
-        v[1] += x.y;
-        v[2] += x.z;
-        v[3] += x.w;
-        v[4] += y.x;
-        v[5] += y.y;
-        v[6] += y.z;
-        v[7] += y.w;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = n + e < N ? frag_epi(epi, v[e]) : 0.f;
-      split_put8<BF>(static_cast<uint16_t *>(P.Y), (N + 31) / 32, m, n, v);
-    }
-    return;
+  for (int u = 0; u < PA; ++u) {
+    const int b = wq * PA + u;
+    oa[u] = min(m0 / 16 + (b >> 1), mblk - 1) * nks * 2048 + (b & 1) * 1024 + lane * 16;
   }
-  const bool vec = N % 4 == 0 && P.ldy % 4 == 0;
 #pragma unroll
-  for (int u = 0; u < PPT; ++u) {
-    int row, col;
-    if (!piece(u, row, col)) continue;
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int u = 0; u < PW; ++u) ow[u] = min(n0 / 16 + wq * PW + u, nstrip - 1) * P.nksf * 1024 + lane * 16;
+  auto stage_k = [&](int st) __attribute__((always_inline)) {  // first k-step of stage st, in the rotated order
+    int t = min(st, nst - 1) + rot;
+    t = t >= nst ? t - nst : t;
+    return max(t, 0) * SK;
+  };
+  // (past the last stage the last one again, into a buffer nobody reads: the
+  // vmcnt bookkeeping stays uniform)
+  const uint32_t lds0 = lds_addr(smem) + (uint32_t)(ws * (NA + NW)) * 1024;
+  auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+    const int kk = min(k0 + stage_k(st) + ws, nks - 1);
+    const uint32_t base = lds0 + (uint32_t)buf * (BLK * 1024);
 #pragma unroll
-    for (int s = 0; s < SK; ++s) {
-      const float4 q = *reinterpret_cast<const float4 *>(&s_red[s][row][col]);
-      v[0] += q.x;
-      v[1] += q.y;
-      v[2] += q.z;
-      v[3] += q.w;
+    for (int u = 0; u < PA; ++u) dma16(ra, base + (uint32_t)(wq * PA + u) * 1024, oa[u], kk * 2048);
+#pragma unroll
+    for (int u = 0; u < PW; ++u) dma16(rw, base + (uint32_t)(NA + wq * PW + u) * 1024, ow[u], kk * 1024);
+  };
+  floatx4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  struct Frags {
+    uint4 a[MB][2], w[NB];
+  };
+  const unsigned char *fa = smem + (wk * (NA + NW) + wm * MB * 2) * 1024 + lane * 16;
+  const unsigned char *fw = smem + (wk * (NA + NW) + NA + wn * NB) * 1024 + lane * 16;
+  auto read = [&](Frags &f, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) f.w[j] = *reinterpret_cast<const uint4 *>(fw + buf * (BLK * 1024) + j * 1024);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl)
+        f.a[i][pl] = *reinterpret_cast<const uint4 *>(fa + buf * (BLK * 1024) + (2 * i + pl) * 1024);
+  };
+  auto compute = [&](const Frags &f, int st) __attribute__((always_inline)) {
+    if (stage_k(st) + wk >= len) return;  // the last stage may be short
+#pragma unroll
+    for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = mfma16<BF>(f.a[i][pl], f.w[j], acc[i][j]);
+  };
+  float4 yres[kFragPieces<BM, BN>];
+  if (P.epi == GEPI_ADD_F32) frag_yres<BM, BN>(P, M, m0, n0, yres);
+#pragma unroll
+  for (int b = 0; b < NBUF - 1; ++b) issue(b, b);
+  int buf = 0;
+  // stage st has landed for every wave, and every read of the buffer that the
+  // next DMA overwrites is complete
+  auto arrive = [&](int st) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(kWaitImm);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    issue(st + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
+  };
+  auto next = [&]() __attribute__((always_inline)) { buf = buf == NBUF - 1 ? 0 : buf + 1; };
+  Frags f0, f1;
+  if (nst > 0) {
+    arrive(0);
+    read(f0, buf);
+    next();
+    int st = 1;
+    for (; st + 1 < nst; st += 2) {
+      arrive(st);
+      read(f1, buf);
+      next();
+      __builtin_amdgcn_sched_barrier(0);
+      compute(f0, st - 1);
+      arrive(st + 1);
+      read(f0, buf);
+      next();
+      __builtin_amdgcn_sched_barrier(0);
+      compute(f1, st);
     }
-    const int m = m0 + row, n = n0 + col;
-    if (m >= M) continue;
-    if (n >= N) continue;
-    const int64_t o = (int64_t)m * P.ldy + n;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = frag_epi(epi, v[e]);
-    if (epi == GEPI_F16) {
-      uint16_t *y = static_cast<uint16_t *>(P.Y) + o;
-      uint16_t h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = F16T<BF>::from_f(v[e]);
-      if (vec) {
-        *reinterpret_cast<uint2 *>(y) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) y[e] = h[e];
-      }
+    if (st < nst) {
+      arrive(st);
+      read(f1, buf);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(f0, st - 1);
+      compute(f1, st);
     } else {
-      float *y = static_cast<float *>(P.Y) + split * g.part_stride + o;
-      if (add) {
-        v[0] += yres[u].x;
-        v[1] += yres[u].y;
-        v[2] += yres[u].z;
-        v[3] += yres[u].w;
-      }
-      if (vec) {
-        *reinterpret_cast<float4 *>(y) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) y[e] = v[e];
-      }
+      compute(f0, st - 1);
     }
   }
+  // every DMA and every read of the ring is done before the partials replace it
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  float(*s_red)[BM][LD] = reinterpret_cast<float(*)[BM][LD]>(smem);
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        s_red[wk][16 * (wm * MB + i) + 4 * (lane >> 4) + r][16 * (wn * NB + j) + (lane & 15)] = acc[i][j][r];
+  __syncthreads();
+  frag_store<BM, BN, SK, BF>(g, P, s_red, yres, m0, n0, split);
 }
 
 // Tiles, smallest first.
 struct FragTile {
   int bm, bn;
 };
-constexpr FragTile kFragTiles[] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {32, 128}, {64, 128}};
-constexpr int kFragNumTiles = 6;
+constexpr FragTile kFragTiles[] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {32, 128}, {64, 128}, {128, 128}};
+constexpr int kFragOneRound = 6;  // the tiles before it; the last is for several rounds
 
 static int64_t frag_units(const FragTile &t, int M, int N) {
   return (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
@@ -263,17 +432,35 @@ static int64_t frag_units(const FragTile &t, int M, int N) {
 // rounds (measured, us, 0.4B FFN key 4096 x 1024: 64 rows 32 x 32 7.9, 16 x 32
 // 8.9, 32 x 64 8.7; 128 rows 32 x 64 9.1, 32 x 32 11.9, 64 x 64 11.4; 512 rows
 // 64 x 128 16.1, 64 x 64 18.4; FFN value's and the 1.5B sizes order alike).
-// Where none fits at once the largest, with as few rows as M has
-// (an eighth more than the CUs still passes: two of the smaller tiles fit on
-// one).
+// Where none fits at once (an eighth more than the CUs still passes: two of the
+// smaller tiles fit on one) the largest, with as few rows as M has.
+//
+// From 64 x 128 the operands come through LDS (gemm_frag_ring_kernel) if K is
+// long enough to pay for filling the ring, and of several rounds each takes
+// 128 x 128 if K covers its unoverlapped ends as well: two register-fed
+// workgroups share a CU and hide theirs in each other. Measured, whole
+// prefills in us, register-fed / ring: 1.5B 1 x 129 3411 / 2862, 4 x 64 4245 /
+// 3665, 8 x 96 9268 / 8374 (64 x 128 ring 8517), 0.4B 3 x 129 2734 / 2609, 1 x
+// 509 3229 / 3133, 16 x 100 7031 / 6692 (6997); 0.1B (K 768) 8 x 60 1198 / 1168,
+// but 16 x 96, three rounds, 2806 / 2891 (2939).
+constexpr int kFragRingMinK = 512, kFragRoundsMinK = 1024;
+static bool frag_ring(const GemmProb *probs, int nprob, int M, int min_k) {
+  int k = 0;
+  for (int q = 0; q < nprob; ++q) {
+    const int64_t nks = (probs[q].K + 31) / 32, blocks = std::max((M + 15) / 16 * 2, (probs[q].N + 15) / 16);
+    if (blocks * nks * 1024 > INT32_MAX) return false;  // the DMA's offsets are 32-bit
+    k = std::max(k, probs[q].K);
+  }
+  return k >= min_k;
+}
 static int frag_tile(const GemmProb *probs, int nprob, int M, int cus) {
-  for (int i = 0; i < kFragNumTiles; ++i) {
+  for (int i = 0; i < kFragOneRound; ++i) {
     if (i == 4 && M > 32) continue;
     int64_t n = 0;
     for (int q = 0; q < nprob; ++q) n += frag_units(kFragTiles[i], M, probs[q].N);
     if (n <= cus + (i < 4 ? cus / 8 : 0)) return i;
   }
-  return M <= 32 ? 4 : 5;
+  return M <= 32 ? 4 : frag_ring(probs, nprob, M, kFragRoundsMinK) ? 6 : 5;
 }
 
 // K slices of a product whose partials the next stage can sum. Few rows and a
@@ -291,7 +478,7 @@ static int frag_plan(int M, int N, int K, int cus, int *splits) {
   *splits = 1;
   if (M > 256) return best;
   int64_t bytes = INT64_MAX;
-  for (int i = 0; i < kFragNumTiles; ++i) {
+  for (int i = 0; i < kFragOneRound; ++i) {
     for (int s = 1; s <= 4 && K / s >= 1024; s *= 2) {
       if (frag_units(kFragTiles[i], M, N) * s > cus) break;
       const int64_t b = (int64_t)(4 * kFragTiles[i].bm + 2 * kFragTiles[i].bn) * ((K + s - 1) / s);
@@ -331,29 +518,40 @@ int launch_gemm_frag(const GemmProb *probs, int nprob, int M, hipStream_t st, in
   g.m_tiles = (M + t.bm - 1) / t.bm;
   g.splits = splits;
   g.part_stride = part_stride;
-  int64_t wgs = 0;
+  int64_t wgs = 0, units = 0;
   for (int i = 0; i < kFragProbs; ++i) {
     g.wg_begin[i] = (int)wgs;
     g.p[i] = probs[i < nprob ? i : 0];
+    if (i < nprob) units += frag_units(t, M, probs[i].N) * splits;
     if (i < nprob) wgs += (int64_t)((probs[i].N + t.bn - 1) / t.bn * splits + 7) / 8 * 8 * g.m_tiles;
   }
   if (wgs > INT32_MAX) return RWKV7_ESHAPE;
   g.wg_begin[kFragProbs] = (int)wgs;
-  const bool bf = probs[0].bf != 0;
+  const bool bf = probs[0].bf != 0, ring = units <= cus && frag_ring(probs, nprob, M, kFragRingMinK);
   const dim3 grid((unsigned)wgs);
 #define RWKV7_FRAG(...)                                                            \
   if (bf) gemm_frag_kernel<__VA_ARGS__, true><<<grid, kFragThreads, 0, st>>>(g);   \
   else gemm_frag_kernel<__VA_ARGS__, false><<<grid, kFragThreads, 0, st>>>(g);     \
   break;
+#define RWKV7_FRAG_RING(...)                                                              \
+  {                                                                                       \
+    if (bf) gemm_frag_ring_kernel<__VA_ARGS__, true><<<grid, kFragThreads, 0, st>>>(g);   \
+    else gemm_frag_ring_kernel<__VA_ARGS__, false><<<grid, kFragThreads, 0, st>>>(g);     \
+    break;                                                                                \
+  }
   switch (ti) {
     case 0: RWKV7_FRAG(1, 2, 1, 1, 8, 2)
     case 1: RWKV7_FRAG(2, 2, 1, 1, 8, 2)
     case 2: RWKV7_FRAG(2, 4, 1, 1, 8, 1)
     case 3: RWKV7_FRAG(2, 4, 2, 1, 4, 1)
     case 4: RWKV7_FRAG(2, 4, 1, 2, 4, 1)
-    default: RWKV7_FRAG(2, 4, 2, 2, 2, 1)
+    case 5:
+      if (ring) RWKV7_FRAG_RING(2, 4, 2, 2, 2, 4)
+      RWKV7_FRAG(2, 4, 2, 2, 2, 1)
+    default: RWKV7_FRAG_RING(4, 4, 2, 2, 2, 3)
   }
 #undef RWKV7_FRAG
+#undef RWKV7_FRAG_RING
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;
 }

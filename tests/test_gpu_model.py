@@ -578,9 +578,12 @@ def test_persistent_decode_abort_is_visible(cuda):
     (1024, 4096, (64, 64, 32, 128), 3, 21),   # four slices
     (1024, 1024, (64, 64, 32, 128), 97, 8),   # 776 rows: eight rows per LayerNorm workgroup, several sequences in one
     (2048, 4096, (64, 64, 32, 128), 1, 33),   # two pieces per LayerNorm thread
+    (1280, 4352, (64, 64, 32, 128), 3, 107),  # 321 rows: operands through LDS, columns past the last tile
+    (1280, 4352, (64, 64, 32, 128), 6, 107),  # 642 rows: 128 x 128 tiles in several rounds
+    (256, 4096, (24, 8, 16, 40), 97, 8),      # several rounds at K = 256: register-fed tiles
 ])
 def test_fragment_gemm_steps_match_row_major_weights(dtype, C, F, ranks, B, T, cuda):
-    """Steps of more than 16 rows on the fragment arenas (activations stored in
+    """Steps of more than eight rows on the fragment arenas (activations stored in
     split order by their producers, gemm_frag.hip) against the same steps on
     the row-major arenas (f32 activations split inside gemm.hip's kernels): the
     same 16-bit products with fp32 sums in another order, so the state agrees
