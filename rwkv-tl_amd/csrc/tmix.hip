@@ -938,8 +938,8 @@ constexpr int kCk = 16;
 // Chunk record (f32). G1, G2, Y0: [token][channel]; B^, K^: [wave][lane][kk];
 // U, V: [quarter][lane][kk]; gam: [64]. The chain kernel's lane l of wave w
 // (rows 16 q .. of the state) reads element kk of [w or q][l] as its operand
-// of the kk-th MFMA step; its DMA gathers G1, G2 and Y0 into that order from
-// the plain rows, which the prep kernel can store one channel per lane.
+// of the kk-th MFMA step; it reads G1, G2 and Y0 from plain rows, which the
+// prep kernel can store one channel per lane.
 constexpr int kRecG1 = 0, kRecG2 = 1024, kRecBh = 2048, kRecKh = 3072, kRecU = 4096, kRecY0 = 5120,
               kRecV = 6144, kRecGam = 7168, kRecFloats = 7232;
 
@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
 // wave (with NQ = 2 the last wave fetches gam again).
 template <int NQ>
 struct ChainSlot {
-  float4 g[4][4][64];   // [G1, G2, B^, K^][column block][lane]
+  float4 g[4][4][64];   // G1, G2: [row][permuted piece]; B^, K^: [column block][lane]
   float p5[4 * NQ][256];  // U, V, Y0 of each quarter, gam, padding
 };
 constexpr int kRing = 3;  // chunk records in LDS: the current one and the next two in flight
@@ -1394,12 +1394,17 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
   const int psrc = wv < NQ ? kRecU * 4 + (q0 + wv) * 1024 : wv < 2 * NQ ? kRecV * 4 + (q0 + wv - NQ) * 1024
                  : wv < 3 * NQ ? kRecY0 * 4 + (q0 + wv - 2 * NQ) * 64 : kRecGam * 4;
   // byte offsets in a record of this lane's 16 bytes: of B^ or K^ in operand
-  // order, of G1 or G2 (row `row`, channels 16 cb + 4 kq ..), of the wave's piece
-  const int vfrag = (64 * cb + lane) * 16, vrow = (row * kN + 16 * cb + 4 * kq) * 4;
+  // order; of G1 or G2, four whole rows per wave with the 16-byte pieces of row
+  // t permuted by XOR with t, so that the 16 rows of an operand read lie in
+  // different banks (a wave fetching its own 16 columns of every row asks for
+  // 16 segments of 64 bytes instead of one KiB: the chain of 32 heads, 4 x 1024
+  // tokens took 86.8 us, now 82.2); of the wave's piece
+  const int vfrag = (64 * cb + lane) * 16, grow = 4 * cb + kq, vrow = (grow * 16 + (row ^ grow)) * 16;
+  const int gidx = 16 * row + ((4 * cb + kq) ^ row);  // G1, G2: row `row`, channels 16 cb + 4 kq ..
   const bool py0 = wv >= 2 * NQ && wv < 3 * NQ;
   const int vpiece = py0 ? psrc + (lane >> 2) * (kN * 4) + (lane & 3) * 16 : psrc + lane * 16;
-  // Record of chunk c into a ring slot: block cb of G1, G2, B^, K^ and one
-  // piece per wave (16 bytes per lane landing in lane order). Past the last
+  // Record of chunk c into a ring slot: rows 4 cb .. of G1, G2, block cb of B^,
+  // K^ and one piece per wave (16 bytes per lane landing in lane order). Past the last
   // chunk the last one is loaded again (unused), so the count per step never
   // changes.
   constexpr int kDmaPerWave = 4 / NQ + 1;
@@ -1452,7 +1457,7 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
       for (int r = 0; r < 4; ++r)
         store_y(br, (unsigned)((ct * kN + 16 * q + 4 * kq + r) * kN + 16 * cb + row) * 4u, (float)st[r]);
     }
-    const float4 g1 = sl.g[0][cb][lane], g2 = sl.g[1][cb][lane], kh = sl.g[3][cb][lane];
+    const float4 g1 = (&sl.g[0][0][0])[gidx], g2 = (&sl.g[1][0][0])[gidx], kh = sl.g[3][cb][lane];
     const float4 vv = reinterpret_cast<const float4 *>(sl.p5[NQ + qq])[lane];
     const float G1[4] = {g1.x, g1.y, g1.z, g1.w}, G2[4] = {g2.x, g2.y, g2.z, g2.w};
     const float V[4] = {vv.x, vv.y, vv.z, vv.w}, KH[4] = {kh.x, kh.y, kh.z, kh.w};
@@ -2470,6 +2475,7 @@ int launch_ln_shift(const LnShiftArgs &a, hipStream_t st) {
 
 
 // GroupNorm + r.k.r_k bonus + gate (demo/rwkv7_torch.py:234-242).
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void gn_gate_kernel(GnGateArgs a) {
   const int C = a.C, H = C / kN;
   const int gh = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -2484,7 +2490,7 @@ __global__ __launch_bounds__(256) void gn_gate_kernel(GnGateArgs a) {
   const float yn = d * rsqrtf(var + kGnEps) * a.vec[RWKV7_V_LNX_W * C + ch] + a.vec[RWKV7_V_LNX_B * C + ch];
   const float rk = wave_sum(a.r[o] * a.kn[o] * a.vec[RWKV7_V_R_K * C + ch]);
   const float out = (yn + rk * a.v[o]) * a.g[o];
-  if (a.split) {
+  if constexpr (SPLIT) {
     uint16_t *f = static_cast<uint16_t *>(a.out);
     if (a.bf) split_put1<true>(f, C / 32, m, ch, out);
     else split_put1<false>(f, C / 32, m, ch, out);
@@ -2494,7 +2500,8 @@ __global__ __launch_bounds__(256) void gn_gate_kernel(GnGateArgs a) {
 
 int launch_gn_gate(const GnGateArgs &a, hipStream_t st) {
   const int waves = a.M * (a.C / kN);
-  gn_gate_kernel<<<(waves + 3) / 4, 256, 0, st>>>(a);
+  if (a.split) gn_gate_kernel<true><<<(waves + 3) / 4, 256, 0, st>>>(a);
+  else gn_gate_kernel<false><<<(waves + 3) / 4, 256, 0, st>>>(a);
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;
 }
