@@ -495,8 +495,8 @@ struct AdjStager {
     sink(0, st_tok, q, g_w);
     sink(1, st_tok, q, g_b);
     sink(2, st_tok, q, g_a);
-    sink(3, st_tok, q, make_float4(fmaf(d.x, g_a.x, g_w.x * g_r.x), fmaf(d.x, g_a.y, g_w.y * g_r.y),
-                                   fmaf(d.x, g_a.z, g_w.z * g_r.z), fmaf(d.x, g_a.w, g_w.w * g_r.w)));
+    sink(3, st_tok, q, make_float4(fmaf(g_w.x, g_r.x, d.x * g_a.x), fmaf(g_w.y, g_r.y, d.x * g_a.y),
+                                   fmaf(g_w.z, g_r.z, d.x * g_a.z), fmaf(g_w.w, g_r.w, d.x * g_a.w)));
     sink(4, st_tok, q, g_k);
     sink(5, st_tok, q, g_y);
     if (q == 0) diag[st_tok] = live(c0 + st_tok) ? d.y : 0.f;
@@ -1060,8 +1060,12 @@ RWKV7_DEV void lora2_chunk(const PrefillScanArgs &p, St &st, int h, int bi, int 
 // record is stored from the registers that hold it. Three barriers after the
 // staging (four where U passes between waves) against eight when each
 // intermediate went through LDS. Measured (kernel trace): 1024 chunks of raw
-// half inputs 20.4 -> 14.0 us; 2048 of f32 inputs 23 us, 109 MB moved (4.7
-// TB/s, the rate of a large copy here).
+// half inputs 20.4 -> 14.8 us; 2048 of f32 inputs 25 us, 109 MB moved (4.4
+// TB/s; a large copy reaches 4.9 here).
+// Error: no larger than the serial scan's against 64 bits (512 tokens, f32: y
+// 0.94e-7 and 1.00e-7, state 0.43e-7 and 0.50e-7). That takes the products of w
+// in 64 bits and sums that are short or run from the smallest term up on their
+// own; with 32-bit products and single running sums it was 1.40e-7 and 1.08e-7.
 //
 // L2: the model path with the LoRA second steps formed here (GateStager and
 // p.l1 set); a separate instance, whose registers and LDS those products no
@@ -1070,12 +1074,15 @@ constexpr int kXs = kN + 4;  // floats per staged row (16-byte aligned, rows 4 b
 
 // acc[t] += sum over s < t (s <= t with DIAG) of M[t][s] x[s], one channel per
 // lane; M's rows are read as LDS broadcasts. With SOLVE x is acc itself:
-// forward substitution with the unit lower triangular I - M.
+// forward substitution with the unit lower triangular I - M. The sum runs on
+// its own, oldest term (mostly the smallest) first, so that its steps don't
+// each round at the size of what is already in acc.
 template <bool DIAG, bool SOLVE>
 RWKV7_DEV void tri_apply(const float (*M)[kCk], const float (&x)[kCk], float (&acc)[kCk]) {
 #pragma unroll
   for (int t = DIAG ? 0 : 1; t < kCk; ++t) {
     const float4 *m4 = reinterpret_cast<const float4 *>(M[t]);
+    float sum = 0.f;
 #pragma unroll
     for (int g = 0; g <= (DIAG ? t : t - 1) / 4; ++g) {
       const float4 q = m4[g];
@@ -1083,9 +1090,10 @@ RWKV7_DEV void tri_apply(const float (*M)[kCk], const float (&x)[kCk], float (&a
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int s = 4 * g + e;
-        if (s < t || (DIAG && s == t)) acc[t] = fmaf(c[e], SOLVE ? acc[s] : x[s], acc[t]);
+        if (s < t || (DIAG && s == t)) sum = fmaf(c[e], SOLVE ? acc[s] : x[s], sum);
       }
     }
+    acc[t] += sum;
   }
 }
 
@@ -1177,48 +1185,55 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
     s_m[3][t][s] = bkr;
     __syncthreads();
   }
-  // a~ = a D(-1, t-1], r~ = r D(-1, t] and (for the MFMA form) k / P, b / P
-  {
-    float P = 1.f;
-    if (wv == 0) {
+  // a~ = a D(-1, t-1], r~ = r D(-1, t] and (for the MFMA form) k / P, b / P,
+  // the products of w in 64 bits: in 32 their roundings add up along the chunk
+  if (wv == 0) {
+    double P = 1.;
 #pragma unroll
-      for (int t = 0; t < kCk; ++t) {
-        x[t] *= P;
-        P *= w[t];
-        s_x[1][t][lane] = x[t];
-      }
-    } else if (wv == 2) {
+    for (int t = 0; t < kCk; ++t) {
+      x[t] = (float)(x[t] * P);
+      P *= w[t];
+      s_x[1][t][lane] = x[t];
+    }
+  } else if (wv == 2) {
+    double P = 1.;
 #pragma unroll
-      for (int t = 0; t < kCk; ++t) {
-        if (!ADJ) P *= w[t];
-        s_x[4][t][lane] = x[t] * P;
-        if (ADJ) P *= w[t];
-      }
-    } else if (fast) {
+    for (int t = 0; t < kCk; ++t) {
+      if (!ADJ) P *= w[t];
+      s_x[4][t][lane] = (float)(x[t] * P);
+      if (ADJ) P *= w[t];
+    }
+  } else if (fast) {
+    double P = 1.;
 #pragma unroll
-      for (int t = 0; t < kCk; ++t) {
-        P *= w[t];
-        s_x[xi][t][lane] = x[t] / P;
-      }
+    for (int t = 0; t < kCk; ++t) P *= w[t];
+    double Q = 1. / P;  // D(s, 15] / D(-1, 15] = 1 / P_s
+#pragma unroll
+    for (int t = kCk - 1; t >= 0; --t) {
+      s_x[xi][t][lane] = (float)(x[t] * Q);
+      Q *= w[t];
     }
   }
   __syncthreads();
   if (fast) {  // wave m: token matrix m, (a~ or r~) (b / P or k / P)^T, masked
     const float4 *X = reinterpret_cast<const float4 *>(&s_x[wv < 2 ? 1 : 4][row][16 * kq]);
     const float4 *Y = reinterpret_cast<const float4 *>(&s_x[(wv & 1) ? 3 : 2][row][16 * kq]);
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+    // (eight sums of 8 channels: the shorter the sums, the smaller the partial
+    // sums that each step rounds)
+    floatx4 acc[8] = {};
 #pragma unroll
     for (int u = 0; u < 4; ++u) {  // channels 16 kq + 4 u + e
       const float4 xv = X[u], yv = Y[u];
-      acc = mfma4(xv.x, yv.x, acc);
-      acc2 = mfma4(xv.y, yv.y, acc2);
-      acc = mfma4(xv.z, yv.z, acc);
-      acc2 = mfma4(xv.w, yv.w, acc2);
+      acc[2 * u] = mfma4(xv.x, yv.x, acc[2 * u]);
+      acc[2 * u + 1] = mfma4(xv.y, yv.y, acc[2 * u + 1]);
+      acc[2 * u] = mfma4(xv.z, yv.z, acc[2 * u]);
+      acc[2 * u + 1] = mfma4(xv.w, yv.w, acc[2 * u + 1]);
     }
+    const floatx4 sum = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 4 * kq + r, s = row;
-      float m = (wv < 2 || ADJ ? s < t : s <= t) ? acc[r] + acc2[r] : 0.f;
+      float m = (wv < 2 || ADJ ? s < t : s <= t) ? sum[r] : 0.f;
       if (ADJ && wv == 3 && s == t) m = s_diag[t];
       s_m[wv][t][s] = m;
     }
@@ -1236,15 +1251,15 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
 #pragma unroll
     for (int t = 0; t < kCk; ++t) R[off + t * kN + lane] = f[t];
   };
-  // x D(t, 15] by suffix products, exact products of w; returns D(-1, 15]
+  // x D(t, 15] by suffix products of w; returns D(-1, 15]
   auto suffix = [&](const float (&f)[kCk], float (&out)[kCk]) {
-    float Q = 1.f;
+    double Q = 1.;
 #pragma unroll
     for (int t = kCk - 1; t >= 0; --t) {
-      out[t] = f[t] * Q;
+      out[t] = (float)(f[t] * Q);
       Q *= w[t];
     }
-    return Q;
+    return (float)Q;
   };
   float f[kCk], y0[kCk];  // wave 3, across the barrier below
   if (wv == 0) {  // G1 = T A~, G2 = R~ + Bbr G1
@@ -1489,13 +1504,16 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
     const float4 u = reinterpret_cast<const float4 *>(sl.p5[qq])[lane];
     const float BH[4] = {bh.x, bh.y, bh.z, bh.w}, U[4] = {u.x, u.y, u.z, u.w};
     float xv[4];
+    // Sig's part on its own, oldest token first like the one above: added onto
+    // that sum, each of its 16 steps would round at the state's full size
+    floatx4 bc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int t = 4 * kk + kq;
       xv[kk] = ((s_xp[qq][0][t][row] + s_xp[qq][1][t][row]) + (s_xp[qq][2][t][row] + s_xp[qq][3][t][row])) + U[kk];
-      acc = mfma4(xv[kk], BH[kk], acc);
+      bc = mfma4(xv[kk], BH[kk], bc);
     }
-    st = acc;
+    st = acc + bc;
     if constexpr (GRAD) {  // Sig of token 4 cb + kq, value row 16 q + row (every block holds all of them)
       const float sv1 = cb == 0 ? xv[0] : cb == 1 ? xv[1] : cb == 2 ? xv[2] : xv[3];
       const int tt = token(c * kCk + 4 * cb + kq);
@@ -1576,17 +1594,20 @@ template int launch_wkv7_chunked<float, float, float>(const ScanArgs<float, floa
 // registers, so a chunk runs as two halves, the later one first (its entering
 // state recomputed from the chunk's). Bound by its VALU work: 11 operations
 // per token and state element, three of them the recomputation.
-// Measured at B = 4, T = 512, H = 16 (2048 chunks): 80 us, 184 MB moved; with
+// Measured at B = 4, T = 512, H = 16 (2048 chunks): 83 us, 184 MB moved; with
 // 129 registers, one workgroup per CU instead of two, 110 us. With the two
-// prep launches (23 + 25 us, 4.7 TB/s of inputs and records) and the chain
-// (62 us) the gradient takes 190 us there; the history-recording scan and the
-// reverse scan over it took 110 + 2887 us.
+// prep launches (25 + 26 us, 4.4 TB/s of inputs and records) and the chain
+// (59 us) the gradient takes 193 us there; the history-recording scan and the
+// reverse scan over it took 110 + 2887 us. Errors against 64 bits, this / the
+// reverse scan: gS0 0.45 / 0.45, gr 0.86 / 0.85, gw 0.89 / 0.92, gk 0.77 / 0.77,
+// gv 0.87 / 0.91, ga 1.18 / 1.24, gb 1.23 / 1.24 e-7 (single sums of eight rows
+// and a serial sum of the waves' parts: up to 1.65e-7).
 // ---------------------------------------------------------------------------
 struct GradArgs {
   const float *r, *w, *k, *v, *a, *b, *gy;
   const float *sbound, *gbound;  // [B, H, chunk, 64, 64]: S entering, G' leaving
   const float *sa, *gsig;        // [B, T, H, 64]: S a, G' b
-  float *gr, *gw, *gk, *ga, *gb;
+  float *gr, *gw, *gk, *ga, *gb, *gS0;
   int B, T, H;
 };
 constexpr int kGradRows = 8, kGradHalf = 8, kGradBatch = 4;
@@ -1662,23 +1683,24 @@ __global__ __launch_bounds__(512, 4) void wkv7_grad_kernel(GradArgs p) {
         const int tt = tb + t;
         const float r = s_c[0][tt][lane], w = s_c[1][tt][lane], a = s_c[3][tt][lane], rb = s_rb[tt];
         const Rows gy = rows(6, tt), v = rows(5, tt), sa = rows(7, tt), gs = rows(8, tt);
-        float pr = 0.f, pw = 0.f, pk = 0.f, pa = 0.f, pb = 0.f;
+        float pr = 0.f, pa = 0.f, pb = 0.f;
+        float pw[2] = {}, pk[2] = {};  // two sums of four rows round at half the size
 #pragma unroll
         for (int e = 0; e < kGradRows; ++e) {
           const float gsa = fmaf(gy.x[e], rb, gs.x[e]);
           const float g = fmaf(gy.x[e], r, G[e]);
           pr = fmaf(S[e], gy.x[e], pr);
-          pw = fmaf(g, hist[t][e], pw);
-          pk = fmaf(g, v.x[e], pk);
+          pw[e / 4] = fmaf(g, hist[t][e], pw[e / 4]);
+          pk[e / 4] = fmaf(g, v.x[e], pk[e / 4]);
           pb = fmaf(g, sa.x[e], pb);
           pa = fmaf(hist[t][e], gsa, pa);
-          G[e] = fmaf(gsa, a, g * w);
+          G[e] = fmaf(g, w, gsa * a);
           S[e] = hist[t][e];
         }
         float(*o)[kN] = s_part[t % kGradBatch][wv];
         o[0][lane] = pr;
-        o[1][lane] = pw;
-        o[2][lane] = pk;
+        o[1][lane] = pw[0] + pw[1];
+        o[2][lane] = pk[0] + pk[1];
         o[3][lane] = pa;
         o[4][lane] = pb;
       }
@@ -1687,11 +1709,12 @@ __global__ __launch_bounds__(512, 4) void wkv7_grad_kernel(GradArgs p) {
         for (int e = tid; e < kGradBatch * 5 * kN; e += 512) {
           const int u = e / (5 * kN), q = e / kN % 5, j = e % kN;
           if (tb + t + u < nt) {
-            float x = 0.f;
+            float x[8];
 #pragma unroll
-            for (int w = 0; w < 8; ++w) x += s_part[u][w][q][j];
+            for (int w = 0; w < 8; ++w) x[w] = s_part[u][w][q][j];
             float *d = q == 0 ? dst[0] : q == 1 ? dst[1] : q == 2 ? dst[2] : q == 3 ? dst[3] : dst[4];
-            d[tok0 + (int64_t)(tb + t + u) * C + j] = x;
+            d[tok0 + (int64_t)(tb + t + u) * C + j] =
+                ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
           }
         }
         __syncthreads();
@@ -1708,6 +1731,11 @@ __global__ __launch_bounds__(512, 4) void wkv7_grad_kernel(GradArgs p) {
 #pragma unroll
   for (int e = 0; e < kGradRows; ++e) S[e] = S0[e];
   half(S, 0);
+  if (c == 0) {  // G' entering the sequence
+    float *o = p.gS0 + (((int64_t)bi * H + h) * kN + kGradRows * wv) * kN + lane;
+#pragma unroll
+    for (int e = 0; e < kGradRows; ++e) o[e * kN] = G[e];
+  }
 }
 
 // floats of the workspace: two sets of chunk records, the two scans' boundary
@@ -1733,7 +1761,7 @@ int launch_wkv7_grad(const Wkv7GradArgs &p, float *ws, hipStream_t st) {
   RWKV7_CHECK_LAUNCH();
   wkv7_chunk_prep_kernel<Adj, false><<<grid, 256, 0, st>>>(aa, rec_b, p.T, p.H);
   RWKV7_CHECK_LAUNCH();
-  const ChainArgs2 ch = {{{p.S0, nullptr, rec_f, nullptr, sbound, sa, 0}, {p.gS_T, p.gS0, rec_b, p.gv, gbound, gsig, 1}}};
+  const ChainArgs2 ch = {{{p.S0, nullptr, rec_f, nullptr, sbound, sa, 0}, {p.gS_T, nullptr, rec_b, p.gv, gbound, gsig, 1}}};
   // as launch_chunked, with both scans' workgroups counted
   if (4 * p.B * p.H >= (mk_cus() > 0 ? mk_cus() : 256))
     wkv7_chunk_chain_kernel<float, 2, true><<<dim3(2 * p.H, p.B, 2), 512, 0, st>>>(nullptr, nullptr, nullptr, p.T, p.H, ch);
@@ -1741,7 +1769,7 @@ int launch_wkv7_grad(const Wkv7GradArgs &p, float *ws, hipStream_t st) {
     wkv7_chunk_chain_kernel<float, 1, true><<<dim3(4 * p.H, p.B, 2), 256, 0, st>>>(nullptr, nullptr, nullptr, p.T, p.H, ch);
   RWKV7_CHECK_LAUNCH();
   const GradArgs g = {p.r, p.w, p.k, p.v, p.a, p.b, p.gy, sbound, gbound, sa, gsig, p.gr, p.gw, p.gk, p.ga, p.gb,
-                      p.B, p.T, p.H};
+                      p.gS0, p.B, p.T, p.H};
   wkv7_grad_kernel<<<grid, 512, 0, st>>>(g);
   RWKV7_CHECK_LAUNCH();
   return RWKV7_OK;

@@ -596,3 +596,42 @@ def test_dplr_seq_gradient_many_heads_matches_history_backward(cuda):
     want = K.wkv7_backward(hist, S1, *d[1:], gy, None)
     for x, xr in zip(K.dplr_seq_backward(*d, gy, None), want):
         assert _rel(x, xr) < 1e-5
+
+
+def _grads64(ins, gy, gS):
+    """y, S_T and the seven gradients of the recurrence, step by step in 64 bits."""
+    S, r, w, k, v, a, b = xs = [x.double().requires_grad_(True) for x in ins]
+    ys = []
+    for t in range(r.shape[1]):
+        sa = torch.matmul(S, a[:, t].unsqueeze(-1))
+        S = S * w[:, t].unsqueeze(-2) + sa * b[:, t].unsqueeze(-2) + v[:, t].unsqueeze(-1) * k[:, t].unsqueeze(-2)
+        ys.append(torch.matmul(S, r[:, t].unsqueeze(-1)).squeeze(-1))
+    y = torch.stack(ys, dim=1)
+    return [y.detach(), S.detach(), *torch.autograd.grad((y, S), xs, (gy.double(), gS.double()))]
+
+
+def test_chunked_scans_are_as_exact_as_the_serial_scan(cuda):
+    """Against 64 bits, the chunked forward and gradient may be no further off
+    than the serial scan and the history backward, whose every step rounds: the
+    same error to the 5 % by which the rounding of 0.4 million values varies
+    between inputs (measured ratios 0.86 to 1.01)."""
+    B, T, H = 2, 160, 10
+    ins = [x.to(cuda) for x in _dplr_inputs(B, T, H, seed=3)]
+    g = torch.Generator().manual_seed(4)
+    gy = torch.randn(B, T, H, 64, generator=g).to(cuda)
+    gS = torch.randn(B, H, 64, 64, generator=g).to(cuda) * 0.1
+    ref = _grads64(ins, gy, gS)
+    S1 = ins[0].clone()
+    hist = torch.empty(B, H, T, 64, 64, device=cuda)
+    y1 = K.wkv7_f32(S1, *ins[1:], hist=hist)
+    serial = [y1, S1, *K.wkv7_backward(hist, S1, *ins[1:], gy, gS)]
+    chunked = [*K.dplr_seq_forward(*ins), *K.dplr_seq_backward(*ins, gy, gS)]
+    for name, c, s, e in zip(("y", "S_T", "gS0", "gr", "gw", "gk", "gv", "ga", "gb"), chunked, serial, ref):
+        assert _rel(c, e) <= 1.05 * _rel(s, e), f"{name}: {_rel(c, e):.3e} chunked, {_rel(s, e):.3e} serial"
+    # 16-bit operands: the f32 state
+    h = [x.half() for x in ins[1:]]
+    S2, S3, S64 = ins[0].clone(), ins[0].clone(), ins[0].double()
+    K.wkv7(S2, *h, chunked=True)
+    K.wkv7(S3, *h, chunked=False)
+    S64 = _grads64([S64, *h], gy, gS)[1]
+    assert _rel(S2, S64) <= 1.05 * _rel(S3, S64), f"state: {_rel(S2, S64):.3e} chunked, {_rel(S3, S64):.3e} serial"
