@@ -296,7 +296,7 @@ using StageBuf = float4[6][CH][kN / 4];
 template <int CH>
 struct GateStager {
   using Args = PrefillScanArgs;
-  static constexpr bool kAdj = false;
+  static constexpr bool kAdj = false, kWide = false;  // (w >= 0.545: a chunk's products stay above 6e-5)
   const PrefillScanArgs &p;
   int64_t base, MC;
   int t1, quarter, st_tok, q, C;
@@ -403,6 +403,7 @@ template <int CH, typename TI, typename TW, typename TY>
 struct RawStager {
   using Args = ScanArgs<TI, TW, TY>;
   static constexpr bool kAdj = false;
+  static constexpr bool kWide = !std::is_same<TI, uint16_t>::value;  // inputs of more range than half
   const Args &p;
   int64_t base;
   int t1, st_tok, q, C;
@@ -458,7 +459,7 @@ struct AdjStager {
     const float *r, *w, *k, *a, *b, *gy;
     int B, T, H;
   };
-  static constexpr bool kAdj = true;
+  static constexpr bool kAdj = true, kWide = true;
   const Args &p;
   int64_t base;
   int Tp, st_tok, q, C;
@@ -922,7 +923,7 @@ int prefill_segments(int T, int B, int H, int cus, int *seg_len) {
 //    once: stages the chunk through the serial scan's staging policies, forms
 //    the token matrices -- on MFMA as (a~)(b / P_s)^T etc. with the prefix
 //    products P_t = D(-1, t] when every P_t of the chunk lies in [1e-30,
-//    1e30], otherwise straight from products of w -- applies T by forward
+//    1e30] and the scaled rows keep f32's range, otherwise straight from products of w -- applies T by forward
 //    substitution, and writes G1, G2, B^, K^, U, Y0, V and gam as a chunk
 //    record.
 // 2. wkv7_chunk_chain_kernel, grid (4 H / NQ, B): each workgroup carries
@@ -1104,6 +1105,7 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
   __shared__ float s_d[L2 ? 3 * kCk * kN : 1];      // the LoRA steps v, w, a
   constexpr bool ADJ = St::kAdj;  // rows taken before the step's update (AdjStager)
   __shared__ float s_diag[ADJ ? kCk : 1];
+  __shared__ int s_ok[St::kWide ? 4 : 1];  // whether the scaled form holds, by wave
 
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = lane & 15, kq = lane >> 4;
@@ -1157,8 +1159,20 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
     }
   }
   // the same w in every wave, so the same answer: uniform over the workgroup
-  const bool fast = __all(ok);
+  bool fast = __all(ok);
+  if constexpr (St::kWide) {
+    // Inputs of f32's range scaled by P or 1 / P may leave it: at 1e30 a row
+    // keeps its precision if its largest value is in [1e-7, 1e7] (below, what
+    // the last denormal cuts off shows; half's whole range passes)
+#pragma unroll
+    for (int t = 0; t < kCk; ++t) {
+      const float m = fabsf(x[t]);
+      fast = fast && __all(m <= 1e7f) && (__any(m >= 1e-7f) || !__any(m > 0.f));  // false for NaN
+    }
+    if (lane == 0) s_ok[wv] = fast;
+  }
   __syncthreads();  // the rows are read: they may be overwritten
+  if constexpr (St::kWide) fast = s_ok[0] && s_ok[1] && s_ok[2] && s_ok[3];
   if (!fast) {      // token matrices straight from products of w: thread (t, s)
     const int t = tid >> 4, s = tid & 15;
     float aba = 0.f, aka = 0.f, bbr = 0.f, bkr = 0.f;

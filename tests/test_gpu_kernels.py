@@ -635,3 +635,21 @@ def test_chunked_scans_are_as_exact_as_the_serial_scan(cuda):
     K.wkv7(S3, *h, chunked=False)
     S64 = _grads64([S64, *h], gy, gS)[1]
     assert _rel(S2, S64) <= 1.05 * _rel(S3, S64), f"state: {_rel(S2, S64):.3e} chunked, {_rel(S3, S64):.3e} serial"
+
+
+@pytest.mark.parametrize("which,scale", [(1, 1e-15), (3, 1e-15), (5, 1e-15), (1, 1e10), (3, 1e10)],
+                         ids=["tiny_r", "tiny_k", "tiny_a", "large_r", "large_k"])
+def test_chunked_f32_scans_keep_the_range_of_their_inputs(which, scale, cuda):
+    """Decays whose products over a chunk come close to 1e-30 (0.016^16 = 2e-29)
+    with inputs that leave f32's range when scaled by them: the chunked forward
+    (130 tokens) and gradient (40) against 64 bits. fp32 sums of up to 64 + 130
+    terms; measured below 2e-7, asserted at ten times that."""
+    for T in (130, 40):
+        ins = [x.to(cuda) for x in _dplr_inputs(1, T, 2, seed=T)]
+        ins[2] = torch.full_like(ins[2], 0.016)
+        ins[which] = ins[which] * scale
+        gy = torch.randn(1, T, 2, 64, generator=torch.Generator().manual_seed(T)).to(cuda)
+        ref = _grads64(ins, gy, torch.zeros_like(ins[0]))
+        got = [*K.dplr_seq_forward(*ins), *K.dplr_seq_backward(*ins, gy, None)]
+        for name, x, e in zip(("y", "S_T", "gS0", "gr", "gw", "gk", "gv", "ga", "gb"), got, ref):
+            assert _rel(x, e) < 2e-6, f"T={T} {name}: {_rel(x, e):.2e}"
