@@ -1177,19 +1177,26 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
     const int t = tid >> 4, s = tid & 15;
     float aba = 0.f, aka = 0.f, bbr = 0.f, bkr = 0.f;
     if (s <= t) {
-      for (int j = 0; j < kN; ++j) {
-        float d = 1.f;  // D(s, t-1]
-        for (int m = s + 1; m < t; ++m) d *= s_x[0][m][j];
-        const float dt = s < t ? d * s_x[0][t][j] : 1.f;  // D(s, t]
-        const float bs = s_x[2][s][j], ks = s_x[3][s][j], at = s_x[1][t][j], rt = s_x[4][t][j];
-        if (s < t) {
-          aba = fmaf(bs * d, at, aba);
-          aka = fmaf(ks * d, at, aka);
+      for (int j0 = 0; j0 < kN; j0 += 8) {  // sums of 8 channels, as below
+        float q[4] = {};
+        for (int j = j0; j < j0 + 8; ++j) {
+          float d = 1.f;  // D(s, t-1]
+          for (int m = s + 1; m < t; ++m) d *= s_x[0][m][j];
+          const float dt = s < t ? d * s_x[0][t][j] : 1.f;  // D(s, t]
+          const float bs = s_x[2][s][j], ks = s_x[3][s][j], at = s_x[1][t][j], rt = s_x[4][t][j];
+          if (s < t) {
+            q[0] = fmaf(bs * d, at, q[0]);
+            q[1] = fmaf(ks * d, at, q[1]);
+          }
+          if (!ADJ || s < t) {
+            q[2] = fmaf(bs * (ADJ ? d : dt), rt, q[2]);
+            q[3] = fmaf(ks * (ADJ ? d : dt), rt, q[3]);
+          }
         }
-        if (!ADJ || s < t) {
-          bbr = fmaf(bs * (ADJ ? d : dt), rt, bbr);
-          bkr = fmaf(ks * (ADJ ? d : dt), rt, bkr);
-        }
+        aba += q[0];
+        aka += q[1];
+        bbr += q[2];
+        bkr += q[3];
       }
     }
     if (ADJ && s == t) bkr = s_diag[t];
