@@ -1177,8 +1177,10 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
     const int t = tid >> 4, s = tid & 15;
     float aba = 0.f, aka = 0.f, bbr = 0.f, bkr = 0.f;
     if (s <= t) {
+#pragma unroll 1
       for (int j0 = 0; j0 < kN; j0 += 8) {  // sums of 8 channels, as below
         float q[4] = {};
+#pragma unroll 1  // (unrolled, the kernel takes 72 registers for 64, and 125 us for 111 where it is not even run)
         for (int j = j0; j < j0 + 8; ++j) {
           float d = 1.f;  // D(s, t-1]
           for (int m = s + 1; m < t; ++m) d *= s_x[0][m][j];
