@@ -1499,14 +1499,10 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
     const float4 vv = reinterpret_cast<const float4 *>(sl.p5[NQ + qq])[lane];
     const float G1[4] = {g1.x, g1.y, g1.z, g1.w}, G2[4] = {g2.x, g2.y, g2.z, g2.w};
     const float V[4] = {vv.x, vv.y, vv.z, vv.w}, KH[4] = {kh.x, kh.y, kh.z, kh.w};
-    // S diag(gam) + V^T K^ does not depend on Sig: formed while the Sig
-    // products run
     const float gam = sl.p5[3 * NQ][16 * cb + row];
-    floatx4 acc;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] = st[r] * gam;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) acc = mfma4(V[kk], KH[kk], acc);
+    const float4 bh = sl.g[2][cb][lane];
+    const float4 u = reinterpret_cast<const float4 *>(sl.p5[qq])[lane];
+    const float BH[4] = {bh.x, bh.y, bh.z, bh.w}, U[4] = {u.x, u.y, u.z, u.w};
     // Sig^T and Y over this wave's 16 key columns: D[t][i] = sum_j G[t][j] S[i][j]
     const float4 s4 = *reinterpret_cast<const float4 *>(&s_s[16 * qq + row][16 * cb + 4 * kq]);
     const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
@@ -1522,18 +1518,26 @@ __global__ __launch_bounds__(256 * NQ) void wkv7_chunk_chain_kernel(
       s_yp[qq][cb][4 * kq + r][row] = ya[r];
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    // S <- S diag(gam) + V^T K^ + Sig^T B^ (this wave's 16 columns)
-    const float4 bh = sl.g[2][cb][lane];
-    const float4 u = reinterpret_cast<const float4 *>(sl.p5[qq])[lane];
-    const float BH[4] = {bh.x, bh.y, bh.z, bh.w}, U[4] = {u.x, u.y, u.z, u.w};
-    float xv[4];
+    // S <- S diag(gam) + V^T K^ + Sig^T B^ (this wave's 16 columns). The first
+    // two do not depend on Sig: formed while its partials are read
+    float xp[4][4], xv[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) xp[kk][w] = s_xp[qq][w][4 * kk + kq][row];
+    __builtin_amdgcn_sched_barrier(0);
+    floatx4 acc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = st[r] * gam;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) acc = mfma4(V[kk], KH[kk], acc);
+    __builtin_amdgcn_sched_barrier(0);
     // Sig's part on its own, oldest token first like the one above: added onto
     // that sum, each of its 16 steps would round at the state's full size
     floatx4 bc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      const int t = 4 * kk + kq;
-      xv[kk] = ((s_xp[qq][0][t][row] + s_xp[qq][1][t][row]) + (s_xp[qq][2][t][row] + s_xp[qq][3][t][row])) + U[kk];
+      xv[kk] = ((xp[kk][0] + xp[kk][1]) + (xp[kk][2] + xp[kk][3])) + U[kk];
       bc = mfma4(xv[kk], BH[kk], bc);
     }
     st = acc + bc;
