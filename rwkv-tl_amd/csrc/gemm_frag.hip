@@ -29,13 +29,33 @@ constexpr int kFragThreads = 512;
 
 struct FragGroup {
   GemmProb p[kFragProbs];
-  int wg_begin[kFragProbs + 1];  // first workgroup of each problem
+  int unit_begin[kFragProbs];  // first unit (column tile and K slice) of each problem
   int nprob, M, m_tiles;
+  int items, per_xcd;  // tiles of all units, and of each XCD's run of them
   // K cut into `splits` (a power of two), each slice's f32 partial product
   // stored at Y + slice * part_stride floats: the next stage sums them
   int splits;
   int64_t part_stride;
 };
+
+// A workgroup's tile. The tiles of the group, row tiles of a unit together, are
+// cut into eight equal runs, one per XCD (workgroups are dealt to the XCDs in
+// turn): every XCD gets as many, and the row tiles of a unit read W from its
+// L2. (Padded to eight units per problem instead, the 22 units of an r, k, v and
+// LoRA group of 768 columns left two XCDs idle, and its LoRA tiles all ran on
+// one: 656 rows 32.0 -> 13.2 us; of 1024 columns, 509 rows 27.3 -> 15.7.)
+struct FragItem {
+  int prob, unit, mt;  // unit -1: none
+};
+RWKV7_DEV FragItem frag_item(const FragGroup &g) {
+  const int item = (int)(blockIdx.x & 7) * g.per_xcd + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= g.per_xcd || item >= g.items) return {0, -1, 0};
+  const int u = item / g.m_tiles;
+  int pi = 0;
+#pragma unroll
+  for (int i = 1; i < kFragProbs; ++i) pi += (i < g.nprob && u >= g.unit_begin[i]);
+  return {pi, u - g.unit_begin[pi], item - u * g.m_tiles};
+}
 
 // The epilogue's value for one element (the add epilogue reads Y elsewhere).
 RWKV7_DEV float frag_epi(int epi, float v) {
@@ -166,24 +186,17 @@ RWKV7_DEV void frag_store(const FragGroup &g, const GemmProb &P, const float (*s
   }
 }
 
-// Workgroup order as in gemm.hip: the m-tiles of a column tile get indices 8
-// apart, so they run on one XCD and read W from its L2.
 template <int MB, int NB, int SM, int SN, int SK, int KB, bool BF>
 __global__ __launch_bounds__(kFragThreads) void gemm_frag_kernel(FragGroup g) {
   constexpr int BM = 16 * MB * SM, BN = 16 * NB * SN, LD = BN + 4;
   static_assert(SM * SN * SK * 64 == kFragThreads, "eight waves");
   __shared__ __align__(16) float s_red[SK][BM][LD];
 
-  const int bx = blockIdx.x;
-  int pi = 0;
-#pragma unroll
-  for (int i = 1; i < kFragProbs; ++i) pi += (i < g.nprob && bx >= g.wg_begin[i]);
-  const GemmProb &P = g.p[pi];
-  const int local = bx - g.wg_begin[pi], mtl = g.m_tiles;
-  const int unit = local / (8 * mtl) * 8 + (local & 7), mt = local % (8 * mtl) / 8;
-  const int N = P.N, M = g.M, S = g.splits;
-  const int nt = unit / S, split = unit & (S - 1);
-  if (nt * BN >= N) return;  // padding of the last group of 8 units
+  const FragItem it = frag_item(g);
+  if (it.unit < 0) return;
+  const GemmProb &P = g.p[it.prob];
+  const int N = P.N, M = g.M, S = g.splits, mt = it.mt;
+  const int nt = it.unit / S, split = it.unit & (S - 1);
   const int m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wv % SM, wn = wv / SM % SN, wk = wv / (SM * SN);
@@ -285,16 +298,11 @@ __global__ __launch_bounds__(kFragThreads) void gemm_frag_ring_kernel(FragGroup 
   constexpr int kBytes = NBUF * BLK * 1024 > SK * BM * LD * 4 ? NBUF * BLK * 1024 : SK * BM * LD * 4;
   __shared__ __align__(1024) unsigned char smem[kBytes];
 
-  const int bx = blockIdx.x;
-  int pi = 0;
-#pragma unroll
-  for (int i = 1; i < kFragProbs; ++i) pi += (i < g.nprob && bx >= g.wg_begin[i]);
-  const GemmProb &P = g.p[pi];
-  const int local = bx - g.wg_begin[pi], mtl = g.m_tiles;
-  const int unit = local / (8 * mtl) * 8 + (local & 7), mt = local % (8 * mtl) / 8;
-  const int N = P.N, M = g.M, S = g.splits;
-  const int nt = unit / S, split = unit & (S - 1);
-  if (nt * BN >= N) return;  // padding of the last group of 8 units
+  const FragItem it = frag_item(g);
+  if (it.unit < 0) return;
+  const GemmProb &P = g.p[it.prob];
+  const int N = P.N, M = g.M, S = g.splits, mt = it.mt;
+  const int nt = it.unit / S, split = it.unit & (S - 1);
   const int m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wv % SM, wn = wv / SM % SN, wk = wv / (SM * SN);
@@ -518,17 +526,18 @@ int launch_gemm_frag(const GemmProb *probs, int nprob, int M, hipStream_t st, in
   g.m_tiles = (M + t.bm - 1) / t.bm;
   g.splits = splits;
   g.part_stride = part_stride;
-  int64_t wgs = 0, units = 0;
+  int64_t units = 0;
   for (int i = 0; i < kFragProbs; ++i) {
-    g.wg_begin[i] = (int)wgs;
+    g.unit_begin[i] = (int)units;
     g.p[i] = probs[i < nprob ? i : 0];
-    if (i < nprob) units += frag_units(t, M, probs[i].N) * splits;
-    if (i < nprob) wgs += (int64_t)((probs[i].N + t.bn - 1) / t.bn * splits + 7) / 8 * 8 * g.m_tiles;
+    if (i < nprob) units += (int64_t)((probs[i].N + t.bn - 1) / t.bn) * splits;
   }
-  if (wgs > INT32_MAX) return RWKV7_ESHAPE;
-  g.wg_begin[kFragProbs] = (int)wgs;
-  const bool bf = probs[0].bf != 0, ring = units <= cus && frag_ring(probs, nprob, M, kFragRingMinK);
-  const dim3 grid((unsigned)wgs);
+  const int64_t items = units * g.m_tiles;
+  if (items > INT32_MAX - 8) return RWKV7_ESHAPE;
+  g.items = (int)items;
+  g.per_xcd = (int)((items + 7) / 8);
+  const bool bf = probs[0].bf != 0, ring = items <= cus && frag_ring(probs, nprob, M, kFragRingMinK);
+  const dim3 grid(8u * (unsigned)g.per_xcd);
 #define RWKV7_FRAG(...)                                                            \
   if (bf) gemm_frag_kernel<__VA_ARGS__, true><<<grid, kFragThreads, 0, st>>>(g);   \
   else gemm_frag_kernel<__VA_ARGS__, false><<<grid, kFragThreads, 0, st>>>(g);     \
