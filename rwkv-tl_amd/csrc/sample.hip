@@ -293,6 +293,16 @@ RWKV7_DEV void load8(const void *row_ptr, int i0, int V, float *f) {
                              : make_uint4(ninf2, ninf2, ninf2, ninf2);
       F16T<BF>::to_f8(u, f);
     }
+  } else if (i0 + 8 <= V) {
+    // rows of any alignment: whole eights in one copy (unaligned 16-byte loads;
+    // eight narrow ones per eight touch a line each)
+    if (F32) {
+      __builtin_memcpy(f, static_cast<const float *>(row_ptr) + i0, 32);
+    } else {
+      uint4 u;
+      __builtin_memcpy(&u, static_cast<const uint16_t *>(row_ptr) + i0, 16);
+      F16T<BF>::to_f8(u, f);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -502,8 +512,9 @@ __global__ __launch_bounds__(kSmpThreads) void sample_kernel(SampleArgs a) {
 
 // ---------------------------------------------------------------------------
 // Top-k over many CUs (temperature > 0, 1 <= top_k <= kCandMax, no probs): the
-// row is cut into slices of kCandSlice logits, one wave each
-// (sample_cand_kernel), that keep a superset of the values top-k can keep, in
+// row is cut into equal slices of at most kCandSlice logits, one wave each
+// (sample_cand_kernel; equal also over its lanes, in whole eights, so that no
+// slice is left with too few maxima for a sharp floor), that keep a superset of the values top-k can keep, in
 // index order; sample_finish_kernel finds the exact thresholds among them and
 // draws. The candidates hold the same values at the same vocabulary positions
 // as in the one-workgroup kernel and every sum is exact, so the token is the
@@ -511,20 +522,20 @@ __global__ __launch_bounds__(kSmpThreads) void sample_kernel(SampleArgs a) {
 //
 // What bounds the two kernels is not the row's bytes (128 KB) but the chain of
 // dependent selections. As histogram passes of a 1024-thread workgroup, with
-// barriers between them, they took 15.3 + 23.4 us at 16 f16 rows of V = 65536,
-// top-k 50, top-p 0.9; now 9.9 + 14.7 (top-k 100: 15.4 + 28.2 -> 12.0 + 16.0;
-// 64 f32 rows, top-k 20, top-p 1: 48.5 + 20.2 -> 13.6 + 12.6; one bf16 row,
-// top-k 100, top-p 1: 11.2 + 21.0 -> 11.6 + 12.4). A wave alone finds the k-th
-// largest of the values its lanes hold with 32 ballots (kth_key), no LDS and
-// no barrier, so:
-// * a slice's floor is the top_k-th largest of the 128 maxima of its lanes'
-//   16-value halves (from top_k = 65 of the 512 maxima of 4 values): at least
-//   top_k values of the slice reach it, so the row's top_k-th largest does
+// barriers between them, they took 15.1 + 23.8 us at 16 f16 rows of V = 65536,
+// top-k 50, top-p 0.9; now 8.2 + 12.7 (whole calls, 16 f16 rows: V = 65536 top-k 1
+// 30.2 -> 15.3, top-k 100 38.3 -> 22.5; V = 5000 top-k 50 25.0 -> 19.4, top-k 100
+// 22.9 -> 18.8, top-k 128 69.6 -> 71.6 where a tie group sends rows to
+// sample_row). A wave alone finds the k-th largest of the values its lanes hold
+// with a ballot per bit (kth_key), no LDS and no barrier, so:
+// * a slice's floor is the top_k-th largest of 128 maxima, two of each lane, its
+//   odd and even fours of values (from top_k = 65 of the 512 maxima of 4): at
+//   least top_k values of the slice reach it, so the row's top_k-th largest does
 //   too, and 1.1-1.2 top_k values pass (more than kSliceCap, at top_k near it:
 //   the slice's exact top_k-th largest instead);
 // * the row's floor is the larger of two bounds on the row's top_k-th largest:
 //   the largest slice floor, and the smallest over the slices of their
-//   ceil(top_k / slices)-th largest half maximum (each slice has that many
+//   ceil(top_k / slices)-th largest of the 128 maxima (each slice has that many
 //   values from there up) -- a few hundred of the candidates pass it;
 // * if at most kFinMax pass, wave 0 holds them, eight per lane, and takes the
 //   exact top-k threshold, the top-p threshold and the draw by itself; else the
@@ -534,8 +545,10 @@ __global__ __launch_bounds__(kSmpThreads) void sample_kernel(SampleArgs a) {
 // ---------------------------------------------------------------------------
 constexpr int kCandE = 32;                   // logits per lane of a slice
 constexpr int kCandSlice = kCandE * kWave;   // 2048
-constexpr int kCandMax = 128;                // the largest top_k: half maxima per slice
+constexpr int kCandMax = 128;                // the largest top_k, and the coarse maxima of a slice
 constexpr int kSliceCap = 128;               // candidates kept per slice
+constexpr int kFloorLow = 12;                // lowest bit of a floor's key that is decided
+constexpr int kSliceSel = 256;               // values at the floor among which a wave selects again
 constexpr int kCandSlices = kSmpMaxV / kCandSlice;
 constexpr int kFinE = kCandSlices * kSliceCap / kSmpThreads;  // candidates per thread in the finish
 constexpr int kFinMax = 512;                 // candidates wave 0 finishes by itself
@@ -555,11 +568,13 @@ RWKV7_DEV uint32_t vkey(float x) { return x > -kInf ? okey(x) : 0u; }
 
 // The k-th largest (k >= 1) of the N keys each lane of the wave holds, 0 when
 // fewer than k are nonzero: bit by bit, the largest key that k of them reach.
-template <int N>
-RWKV7_DEV uint32_t kth_key(const uint32_t (&key)[N], int k) {
-  uint32_t t = 0;
+// With LOW > 0 down to that bit only: a key that k of them reach, less than
+// 2^LOW below. Each bit is a chain of ballots and scalar counts. t and bit:
+// where to start, the bits above `bit` that all nonzero keys share.
+template <int N, int LOW = 0>
+RWKV7_DEV uint32_t kth_key(const uint32_t (&key)[N], int k, uint32_t t = 0, int bit = 31) {
 #pragma unroll 1
-  for (int bit = 31; bit >= 0; --bit) {
+  for (; bit >= LOW; --bit) {
     const uint32_t c = t | (1u << bit);
     int n = 0;
 #pragma unroll
@@ -569,32 +584,48 @@ RWKV7_DEV uint32_t kth_key(const uint32_t (&key)[N], int k) {
   return t;
 }
 
-// The 32 logits of a lane, V past the row (-inf there); VEC: 16-byte loads.
+// VEC: 16-byte loads.
 template <bool VEC, int FMT>
 __global__ __launch_bounds__(256) void sample_cand_kernel(SampleArgs a, CandBuf cb) {
+  __shared__ float s_sel[4][kSliceSel];
   const int lane = threadIdx.x & 63, g = 4 * blockIdx.x + (threadIdx.x >> 6), row = blockIdx.y, V = a.V;
   if (g >= cb.G) return;
   const void *src = static_cast<const char *>(a.logits) + (int64_t)row * a.ld * (FMT == 1 ? 4 : 2);
-  const int i0 = g * kCandSlice + kCandE * lane;
+  // this lane's eights of logits, at most kCandE / 8 of them
+  const int n8 = (V + 7) / 8, lanes = kWave * cb.G, b0 = (kWave * g + lane) * n8 / lanes,
+            b1 = (kWave * g + lane + 1) * n8 / lanes, i0 = 8 * b0;
   float l[kCandE];
 #pragma unroll
-  for (int c = 0; c < kCandE / 8; ++c) load8<VEC, FMT>(src, i0 + 8 * c, V, &l[8 * c]);
+  for (int c = 0; c < kCandE / 8; ++c) load8<VEC, FMT>(src, b0 + c < b1 ? i0 + 8 * c : V, V, &l[8 * c]);
   if (a.seen && a.pen != 1.f) {  // the same operations, in the same order, as sample_row
-    const uint32_t w = i0 < V ? a.seen[(int64_t)row * a.seen_ld + (i0 >> 5)] : 0u;
+    const uint32_t *sr = a.seen + (int64_t)row * a.seen_ld;
+    const int nw = (V + 31) / 32, w0 = i0 >> 5;
+    const uint64_t two = (uint64_t)(w0 < nw ? sr[w0] : 0u) | ((uint64_t)(w0 + 1 < nw ? sr[w0 + 1] : 0u) << 32);
+    const uint32_t w = (uint32_t)(two >> (i0 & 31));
 #pragma unroll
     for (int e = 0; e < kCandE; ++e)
       if ((w >> e) & 1u) l[e] = l[e] > 0.f ? l[e] / a.pen : l[e] * a.pen;
   }
 #pragma unroll
   for (int e = 0; e < kCandE; ++e) l[e] = (l[e] + 0.f) / a.temp;
-  // maxima of the lane's eights of four values, then of its halves
+  // maxima of the lane's fours, then of its odd and even fours (its halves would
+  // be empty for lanes with sixteen values)
   uint32_t pk[8], hk[2];
 #pragma unroll
   for (int q = 0; q < 8; ++q) pk[q] = vkey(fmaxf(fmaxf(l[4 * q], l[4 * q + 1]), fmaxf(l[4 * q + 2], l[4 * q + 3])));
 #pragma unroll
-  for (int h = 0; h < 2; ++h) hk[h] = max(max(pk[4 * h], pk[4 * h + 1]), max(pk[4 * h + 2], pk[4 * h + 3]));
-  const uint32_t fl = a.top_k <= kWave ? kth_key<2>(hk, a.top_k) : kth_key<8>(pk, a.top_k);
-  const uint32_t few = kth_key<2>(hk, (a.top_k + cb.G - 1) / cb.G);
+  for (int h = 0; h < 2; ++h) hk[h] = max(max(pk[h], pk[h + 2]), max(pk[h + 4], pk[h + 6]));
+  // (floors to 2^-11 of a value; top_k 1: the largest; the second bound only
+  // where the slices' candidates can pass what one wave finishes)
+  uint32_t fl, few = 0u;
+  if (a.top_k == 1) {
+    fl = max(hk[0], hk[1]);
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) fl = max(fl, (uint32_t)__shfl_xor((int)fl, d));
+  } else {
+    fl = a.top_k <= kWave ? kth_key<2, kFloorLow>(hk, a.top_k) : kth_key<8, kFloorLow>(pk, a.top_k);
+    if (cb.G * kSliceCap > kFinMax) few = kth_key<2, kFloorLow>(hk, (a.top_k + cb.G - 1) / cb.G);
+  }
   float thr = fl ? okey_inv(fl) : -kInf;
   int own, inc, total;  // this lane's kept values, their inclusive prefix over the lanes, the slice's
   auto count = [&]() {
@@ -611,10 +642,28 @@ __global__ __launch_bounds__(256) void sample_cand_kernel(SampleArgs a, CandBuf 
   };
   count();
   if (total > kSliceCap) {  // the slice's exact top_k-th largest (top_k near kCandMax, or ties)
-    uint32_t key[kCandE];
+    uint32_t k;
+    if (total <= kSliceSel) {
+      // among the values at the floor, gathered over the lanes: an eighth of the
+      // ballots that all values take (16 rows of 5000 f16 logits, top-k 127:
+      // a call 38.1 -> 25.5 us)
+      constexpr int N = kSliceSel / kWave;
+      float *sel = s_sel[threadIdx.x >> 6];
+      int at = inc - own;
 #pragma unroll
-    for (int e = 0; e < kCandE; ++e) key[e] = vkey(l[e]);
-    const uint32_t k = kth_key<kCandE>(key, a.top_k);
+      for (int e = 0; e < kCandE; ++e)
+        if (l[e] > -kInf && l[e] >= thr) sel[at++] = l[e];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // one wave's own LDS
+      uint32_t key[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) key[e] = lane + kWave * e < total ? vkey(sel[lane + kWave * e]) : 0u;
+      k = kth_key<N>(key, a.top_k);
+    } else {
+      uint32_t key[kCandE];
+#pragma unroll
+      for (int e = 0; e < kCandE; ++e) key[e] = vkey(l[e]);
+      k = kth_key<kCandE>(key, a.top_k);
+    }
     thr = k ? okey_inv(k) : -kInf;
     count();
   }
@@ -655,9 +704,23 @@ RWKV7_DEV int draw_in_wave(float (&l)[N], const int (&ix)[N], const SampleArgs &
     key[e] = vkey(l[e]);
     m = fmaxf(m, l[e]);
   }
+  uint32_t lo = ~0u;  // the smallest key there is: above the highest bit it and m's differ in, all agree
 #pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-  const uint32_t tk = kth_key<N>(key, a.top_k);
+  for (int e = 0; e < N; ++e) lo = min(lo, key[e] ? key[e] : ~0u);
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    m = fmaxf(m, __shfl_xor(m, d));
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
+  }
+  const uint32_t hi = vkey(m);
+  uint32_t tk = hi;
+  if (a.top_k > 1 && hi != lo) {
+    const int bit = hi ? 31 - __clz((int)(hi ^ lo)) : 31;
+    int have = 0;  // fewer than top_k: none is cut
+#pragma unroll
+    for (int e = 0; e < N; ++e) have += __popcll(__ballot(key[e] != 0u));
+    tk = have < a.top_k ? 0u : kth_key<N>(key, a.top_k, bit == 31 ? 0u : hi & (~0u << (bit + 1)), bit);
+  }
   float thr = tk ? okey_inv(tk) : -kInf;  // sampling.py:56-60
   int own = 0;
 #pragma unroll
@@ -780,6 +843,10 @@ __global__ __launch_bounds__(kSmpThreads) void sample_finish_kernel(SampleArgs a
   const int g = t >> 5, p0 = kFinE * (t & 31);
   const int64_t slot = (int64_t)row * G + min(g, G - 1);
   const int cnt = g < G ? cb.cnt[slot] : 0;
+  if (__syncthreads_or(cnt < 0)) {  // a tie group overflowed a slice: the whole row here
+    put_token(a, row, sample_row<VEC, FMT>(a, row, s));
+    return;
+  }
   float l[kFinE];
   int ix[kFinE];
   {
@@ -805,10 +872,6 @@ __global__ __launch_bounds__(kSmpThreads) void sample_finish_kernel(SampleArgs a
   }
   const uint32_t fkey = max(top, few);
   const float fl = fkey ? okey_inv(fkey) : -kInf;
-  if (__syncthreads_or(cnt < 0)) {  // a tie group overflowed a slice: the whole row here
-    put_token(a, row, sample_row<VEC, FMT>(a, row, s));
-    return;
-  }
   // candidates from the floor up, compacted in order
   int own = 0;
 #pragma unroll

@@ -291,6 +291,27 @@ def test_candidate_path_draws_the_same_tokens(dtype, V):
                 assert float((counts > 0).float().mean()) > 0.5, counts.tolist()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [2049, 2056, 4097, 5000, 8191, 63495])
+def test_candidate_path_over_uneven_slices(dtype, V):
+    """Vocabularies that do not divide into slices of 2048: slices and lanes of
+    unequal length, rows of any alignment (odd V), one to 31 slices with few
+    values a lane, at the edges of the two floors (top-k 64 and 65) and of the
+    slice's capacity (128): the one-workgroup kernel's token, and no slice of
+    untied values (f32) falls back."""
+    g = torch.Generator().manual_seed(V)
+    B = 3
+    logits = (torch.randn(B, V, generator=g) * 2.5).to(dtype).to(DEV)
+    seen = seen_bitmap(torch.randint(0, V, (V // 2,), generator=g), B, V, DEV)
+    for k in (1, 2, 50, 64, 65, 100, 127, 128):
+        for p, pen in ((0.9, 1.0), (1.0, 1.3)):
+            a, b, counts = _both_paths(logits, B, V, seen=seen if pen != 1.0 else None, offset=k, temperature=0.8,
+                                       top_k=k, top_p=p, repetition_penalty=pen)
+            assert torch.equal(a, b), (k, p, a.tolist(), b.tolist())
+            ok = (counts >= k) & (counts <= 128)
+            assert bool((ok if dtype == torch.float32 else ok | (counts == -1)).all()), (k, counts.tolist())
+
+
 def test_candidate_path_falls_back_on_a_tie_group():
     """A slice whose top-k threshold falls in a tie group of more than 128
     values (here: a constant stretch of the row) marks its count -1 and the
