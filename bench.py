@@ -371,7 +371,7 @@ def bench_configs() -> dict:
     chunked_ms = time_cuda(chunked, 50)
     serial_ms = time_cuda(serial, 50)
     # the algorithm kernels.wkv7 picks for this shape
-    ms = chunked_ms if K._chunk_pays(B, T, H) else serial_ms
+    ms = chunked_ms if K._chunk_pays(T, H) else serial_ms
     c2_bytes = B * T * H * N * (5 * 2 + 4 + 2) + 2 * 4 * B * H * N * N
     out["C2_wkv7_B8_H16_T128"] = {"ms": round(ms, 4), "serial_ms": round(serial_ms, 4),
                                   "chunked_ms": round(chunked_ms, 4), "op_ms": round(op_ms, 4),

@@ -71,19 +71,61 @@ def _h16(*ts: Tensor) -> int:
 
 # The operators take the chunked scan for sequences at least this long
 # (measured on MI355X, us per call, serial / chunked: B=1, H=16, T=64 14.9 /
-# 19.2, T=128 21.4 / 19.1; B=8, H=16, T=64 15.4 / 20.5, T=128 28.1 / 24.4;
+# 19.2, T=128 21.4 / 19.1; B=8, H=16, T=64 15.4 / 20.5, T=128 28.1 / 24.9;
 # B=16, H=32, T=128 102 / 74, T=1024 840 / 539).
 CHUNK_MIN_T = 128
+# Bytes of chunk records (28,928 per 16 tokens and head) that one call holds at
+# most; beyond, the scan runs over ranges of the batch, or of one sequence's
+# tokens, that share them (the same results: records are per 16 tokens, and the
+# state between two ranges is the state between two of their chunks).
+CHUNK_WS_BYTES = 2 << 30
 
 
 def _chunk_fits(T: int, H: int) -> bool:
-    """Whether a sequence's chunk records (28,928 bytes per 16 tokens and
-    head) and its f32 outputs stay inside the chunked kernels' 32-bit offsets."""
+    """Whether a sequence's chunk records and its f32 outputs stay inside the
+    chunked kernels' 32-bit offsets."""
     return T <= 1 << 20 and T * H * N * 4 < 2**31 - 1
 
 
-def _chunk_pays(Bsz: int, T: int, H: int) -> bool:
+def _chunk_pays(T: int, H: int) -> bool:
     return T >= CHUNK_MIN_T and _chunk_fits(T, H)
+
+
+def _chunk_ranges(Bsz: int, T: int, seq_bytes: int, cut_tokens: bool) -> list[tuple[int, int, int, int]]:
+    """Ranges ``(b0, b1, t0, t1)`` of a batch whose sequences each take
+    ``seq_bytes`` of workspace, in order, within ``CHUNK_WS_BYTES``: whole
+    sequences, as many as fit; where not even one does, with ``cut_tokens``,
+    ranges of whole 16-token chunks of one (else single sequences)."""
+    n = CHUNK_WS_BYTES // seq_bytes
+    if n >= 1 or not cut_tokens:
+        n = max(n, 1)
+        return [(b, min(b + n, Bsz), 0, T) for b in range(0, Bsz, n)]
+    chunks = (T + 15) // 16
+    step = 16 * max(1, CHUNK_WS_BYTES * chunks // seq_bytes)
+    return [(b, b + 1, t, min(t + step, T)) for b in range(Bsz) for t in range(0, T, step)]
+
+
+def _at(x: Tensor, b: int, t: int = 0) -> int:
+    """Address of sequence b (from token t) of a contiguous [B, T, ...]."""
+    return x.data_ptr() + (b * x.stride(0) + t * x.stride(1)) * x.element_size()
+
+
+def _chunked_scan(call, what: str, S: Tensor, ins: tuple[Tensor, ...], y: Tensor) -> None:
+    """``call(S, ins, y, B, T, ws, nb)`` on the batch, or on the ranges of it that share one workspace."""
+    Bsz, T, H = y.shape[:3]
+    nbytes = _lib.load().rwkv7_wkv7_chunked_workspace_bytes
+    nb = int(nbytes(Bsz, T, H))
+    if nb <= CHUNK_WS_BYTES:
+        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+        _lib.check(call(S.data_ptr(), [x.data_ptr() for x in ins], y.data_ptr(), Bsz, T, ws.data_ptr(), nb), what)
+        return
+    ranges = _chunk_ranges(Bsz, T, int(nbytes(1, T, H)), _chunk_fits(T, H))
+    b0, b1, t0, t1 = ranges[0]  # the largest
+    nb = int(nbytes(b1 - b0, t1 - t0, H))
+    ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+    for b0, b1, t0, t1 in ranges:
+        _lib.check(call(_at(S, b0), [_at(x, b0, t0) for x in ins], _at(y, b0, t0), b1 - b0, t1 - t0,
+                        ws.data_ptr(), nb), what)
 
 
 def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Tensor,
@@ -93,8 +135,9 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
     ``r, k, v, a, b``: f16 or bf16 [B, T, H, 64]; ``w``: the same 16-bit
     dtype or f32. Returns ``y`` [B, T, H, 64] of r's dtype with ``y_t = S_t r_t``.
     ``chunked``: run the chunked (MFMA) algorithm, ``rwkv7_wkv7_chunked``,
-    with a workspace allocated per call, or the serial scan ``rwkv7_wkv7``;
-    ``None`` chooses the chunked one for ``T >= CHUNK_MIN_T``.
+    with a workspace allocated per call (1.8 KB per token and head, at most
+    ``CHUNK_WS_BYTES``), or the serial scan ``rwkv7_wkv7``; ``None`` chooses the
+    chunked one for ``T >= CHUNK_MIN_T``.
     """
     _dev(S, r, w, k, v, a, b)
     _need(S.dtype == torch.float32 and S.dim() == 4 and S.shape[2:] == (N, N), "S must be f32 [B,H,64,64]")
@@ -108,16 +151,18 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
     _need(w.shape == r.shape and w.dtype in (r.dtype, torch.float32), "w must be like r, or f32")
     y = torch.empty_like(r)
     lib = _lib.load()
-    args = (S.data_ptr(), r.data_ptr(), w.data_ptr(), int(w.dtype == torch.float32), k.data_ptr(), v.data_ptr(),
-            a.data_ptr(), b.data_ptr(), y.data_ptr(), Bsz, T, H, bf)
+    w32 = int(w.dtype == torch.float32)
     if chunked is None:
-        chunked = _chunk_pays(Bsz, T, H)
+        chunked = _chunk_pays(T, H)
     if chunked:
-        nb = int(lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H))
-        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        _lib.check(lib.rwkv7_wkv7_chunked(*args, ws.data_ptr(), nb, _lib.stream_handle()), "rwkv7_wkv7_chunked")
+        def call(S_, i, y_, B_, T_, ws, nb):
+            return lib.rwkv7_wkv7_chunked(S_, i[0], i[1], w32, *i[2:], y_, B_, T_, H, bf, ws, nb, _lib.stream_handle())
+
+        _chunked_scan(call, "rwkv7_wkv7_chunked", S, (r, w, k, v, a, b), y)
     else:
-        _lib.check(lib.rwkv7_wkv7(*args, _lib.stream_handle()), "rwkv7_wkv7")
+        _lib.check(lib.rwkv7_wkv7(S.data_ptr(), r.data_ptr(), w.data_ptr(), w32, k.data_ptr(), v.data_ptr(),
+                                  a.data_ptr(), b.data_ptr(), y.data_ptr(), Bsz, T, H, bf, _lib.stream_handle()),
+                   "rwkv7_wkv7")
     return y
 
 
@@ -172,19 +217,20 @@ def wkv7_backward(hist: Tensor, S_T: Tensor, r: Tensor, w: Tensor, k: Tensor, v:
 def dplr_seq_forward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: Tensor, B: Tensor):
     """Functional DPLR sequence for training: ``S`` [H,64,64] or [B,H,64,64]
     f32 is not modified; inputs [T,H,64] or [B,T,H,64] f32. Returns
-    ``(y, S_T)``."""
+    ``(y, S_T)``. Workspace as ``wkv7``'s."""
     batched = S.dim() == 4
     S1 = (S if batched else S.unsqueeze(0)).contiguous().clone()
     ins = [(x if batched else x.unsqueeze(0)).contiguous() for x in (R, W, K, V, A, B)]
     _dev(S1, *ins)
-    Bsz, T, H = _wkv7_f32_shapes(S1, *ins)
-    if _chunk_pays(Bsz, T, H):
+    _, T, H = _wkv7_f32_shapes(S1, *ins)
+    if _chunk_pays(T, H):
         y = torch.empty_like(ins[0])
         lib = _lib.load()
-        nb = int(lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H))
-        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        _lib.check(lib.rwkv7_wkv7_f32_chunked(S1.data_ptr(), *(x.data_ptr() for x in ins), y.data_ptr(), Bsz, T, H,
-                                              ws.data_ptr(), nb, _lib.stream_handle()), "rwkv7_wkv7_f32_chunked")
+
+        def call(S_, i, y_, B_, T_, ws, nb):
+            return lib.rwkv7_wkv7_f32_chunked(S_, *i, y_, B_, T_, H, ws, nb, _lib.stream_handle())
+
+        _chunked_scan(call, "rwkv7_wkv7_f32_chunked", S1, ins, y)
     else:
         y = wkv7_f32(S1, *ins)
     return (y, S1) if batched else (y[0], S1[0])
@@ -195,7 +241,8 @@ def dplr_seq_backward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: 
     """Gradients of ``dplr_seq_forward`` w.r.t. ``(S, R, W, K, V, A, B)`` from
     its inputs (the reference's plan, TODO.md:46-54, recomputes the states
     too): chunked scans of the states and of their adjoint, then every chunk at
-    once (``rwkv7_wkv7_grad``)."""
+    once (``rwkv7_wkv7_grad``; a workspace of 6.2 KB per token and head, of at
+    most ``CHUNK_WS_BYTES`` or one sequence's)."""
     batched = S.dim() == 4
     u = (lambda x: x) if batched else (lambda x: x.unsqueeze(0))
     S1 = u(S).contiguous()
@@ -215,11 +262,16 @@ def dplr_seq_backward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: 
             _need(gS.shape == S1.shape and gS.dtype == torch.float32, "gS must be like S")
         out = (torch.empty_like(S1), *(torch.empty_like(x) for x in ins))
         lib = _lib.load()
-        nb = int(lib.rwkv7_wkv7_grad_workspace_bytes(Bsz, T, H))
+        nb, ranges = int(lib.rwkv7_wkv7_grad_workspace_bytes(Bsz, T, H)), [(0, Bsz, 0, T)]
+        if nb > CHUNK_WS_BYTES:
+            ranges = _chunk_ranges(Bsz, T, int(lib.rwkv7_wkv7_grad_workspace_bytes(1, T, H)), False)
+            nb = int(lib.rwkv7_wkv7_grad_workspace_bytes(ranges[0][1], T, H))
         ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        rc = lib.rwkv7_wkv7_grad(S1.data_ptr(), *(x.data_ptr() for x in ins), gy.data_ptr(), _lib.ptr(gS),
-                                 *(g.data_ptr() for g in out), Bsz, T, H, ws.data_ptr(), nb, _lib.stream_handle())
-        _lib.check(rc, "rwkv7_wkv7_grad")
+        for b0, b1, _, _ in ranges:
+            rc = lib.rwkv7_wkv7_grad(_at(S1, b0), *(_at(x, b0) for x in ins), _at(gy, b0),
+                                     None if gS is None else _at(gS, b0), *(_at(g, b0) for g in out), b1 - b0, T, H,
+                                     ws.data_ptr(), nb, _lib.stream_handle())
+            _lib.check(rc, "rwkv7_wkv7_grad")
     return out if batched else tuple(g[0] for g in out)
 
 

@@ -656,3 +656,44 @@ def test_chunked_f32_scans_keep_the_range_of_their_inputs(which, scale, cuda):
         got = [*K.dplr_seq_forward(*ins), *K.dplr_seq_backward(*ins, gy, None)]
         for name, x, e in zip(("y", "S_T", "gS0", "gr", "gw", "gk", "gv", "ga", "gb"), got, ref):
             assert _rel(x, e) < 2e-6, f"T={T} {name}: {_rel(x, e):.2e}"
+
+
+def _peak(fn):
+    """fn() and the device bytes it took at most beyond what was held before."""
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    out = fn()
+    torch.cuda.synchronize()
+    return out, torch.cuda.max_memory_allocated() - base
+
+
+@pytest.mark.parametrize("B,T,H,limit", [(5, 130, 3, 2), (2, 200, 2, 1), (1, 333, 2, 0.3), (3, 129, 1, 0.5)])
+def test_chunked_scans_in_ranges_of_a_bounded_workspace(B, T, H, limit, cuda, monkeypatch):
+    """A workspace of ``limit`` sequences' records: batches in parts, sequences in
+    parts of whole chunks (the gradient: whole sequences), the same bits."""
+    ins = [x.to(cuda) for x in _dplr_inputs(B, T, H, seed=T)]
+    gy = torch.randn(B, T, H, 64, device=cuda)
+    h = [x.half() for x in ins[1:]]
+
+    def run():
+        S = ins[0].clone()
+        y = K.wkv7(S, *h, chunked=True)
+        return [y, S, *K.dplr_seq_forward(*ins), *K.dplr_seq_backward(*ins, gy, None)]
+
+    want = run()
+    nb = int(K._lib.load().rwkv7_wkv7_chunked_workspace_bytes(1, T, H))
+    monkeypatch.setattr(K, "CHUNK_WS_BYTES", int(limit * nb))
+    for x, e in zip(run(), want):
+        assert torch.equal(x, e)
+
+
+def test_large_chunked_calls_keep_to_the_workspace_bound(cuda):
+    """64 sequences x 2048 tokens x 32 heads, 7.6 GB of records in one piece:
+    the call takes the bound and y beyond its operands."""
+    B, T, H = 64, 2048, 32
+    x = torch.randn(B, T, H, 64, device=cuda, dtype=torch.float16) * 0.1
+    w = torch.full_like(x, 0.9)
+    S = torch.zeros(B, H, 64, 64, device=cuda)
+    y, peak = _peak(lambda: K.wkv7(S, x, w, x, x, x, x))
+    assert peak <= K.CHUNK_WS_BYTES + y.numel() * 2 + (1 << 22)

@@ -13,6 +13,7 @@ import torch
 from oracle import rwkv7_ref as R
 from oracle import sampling_ref as S
 from rwkv_tl_amd import _lib, make_rwkv7, sample_logits
+from rwkv_tl_amd import kernels as K
 from rwkv_tl_amd.checkpoint import SHAPES, make_random_state_dict
 from rwkv_tl_amd.state import State
 from rwkv_tl_amd.weight import RWKV7Weight, layer_layout, model_dims, quantize_rows_i8, to_fragments
@@ -356,3 +357,29 @@ def test_quantize_rows_i8_bounds():
     e = torch.arange(-127, 128, dtype=torch.float32)[None, :] * 0.5
     qe, se = quantize_rows_i8(e)
     assert float(se[0]) == 0.5 and torch.equal(qe[0].float(), torch.arange(-127, 128, dtype=torch.float32))
+
+
+@pytest.mark.parametrize("B,T,per16,cut", [
+    (64, 4096, 32 * 28928, True), (3, 100_000, 32 * 28928, True), (1, 1 << 20, 4 * 28928, True),
+    (5, 40_000, 16 * 28928, True), (7, 1000, 1, True), (4, 700_000, 98_816, False), (9, 50_000, 98_816, False),
+])
+def test_chunk_ranges_cover_the_batch_within_the_workspace(B, T, per16, cut):
+    """The ranges that share one workspace: every token once and in order, whole
+    16-token chunks, the first the largest, and none past the bound unless a
+    sequence may not be cut."""
+    seq = (T + 15) // 16 * per16
+    ranges = K._chunk_ranges(B, T, seq, cut)
+    seen = {b: 0 for b in range(B)}
+    size = [(b1 - b0) * ((t1 - t0 + 15) // 16) * per16 for b0, b1, t0, t1 in ranges]
+    for b0, b1, t0, t1 in ranges:
+        assert b0 < b1 and t0 < t1 and t0 % 16 == 0
+        for b in range(b0, b1):
+            assert seen[b] == t0
+            seen[b] = t1
+    assert all(t == T for t in seen.values())
+    assert size[0] == max(size)
+    if cut or seq <= K.CHUNK_WS_BYTES:
+        assert max(size) <= K.CHUNK_WS_BYTES
+        assert len(ranges) == 1 or max(size) > K.CHUNK_WS_BYTES // 2  # (no smaller than it need be)
+    else:
+        assert all(b1 == b0 + 1 and (t0, t1) == (0, T) for b0, b1, t0, t1 in ranges)
