@@ -110,22 +110,24 @@ def _at(x: Tensor, b: int, t: int = 0) -> int:
     return x.data_ptr() + (b * x.stride(0) + t * x.stride(1)) * x.element_size()
 
 
-def _chunked_scan(call, what: str, S: Tensor, ins: tuple[Tensor, ...], y: Tensor) -> None:
-    """``call(S, ins, y, B, T, ws, nb)`` on the batch, or on the ranges of it that share one workspace."""
+def _chunked_scan(call, S: Tensor, ins: tuple[Tensor, ...], y: Tensor) -> int:
+    """``call(ws, nb, B, T, S, y, *ins)`` (addresses; a C call's return code) on
+    the batch, or on the ranges of it that share one workspace."""
     Bsz, T, H = y.shape[:3]
     nbytes = _lib.load().rwkv7_wkv7_chunked_workspace_bytes
-    nb = int(nbytes(Bsz, T, H))
+    nb = nbytes(Bsz, T, H)
     if nb <= CHUNK_WS_BYTES:
         ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        _lib.check(call(S.data_ptr(), [x.data_ptr() for x in ins], y.data_ptr(), Bsz, T, ws.data_ptr(), nb), what)
-        return
-    ranges = _chunk_ranges(Bsz, T, int(nbytes(1, T, H)), _chunk_fits(T, H))
+        return call(ws.data_ptr(), nb, Bsz, T, S.data_ptr(), y.data_ptr(), *[x.data_ptr() for x in ins])
+    ranges = _chunk_ranges(Bsz, T, nbytes(1, T, H), _chunk_fits(T, H))
     b0, b1, t0, t1 = ranges[0]  # the largest
-    nb = int(nbytes(b1 - b0, t1 - t0, H))
+    nb = nbytes(b1 - b0, t1 - t0, H)
     ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
     for b0, b1, t0, t1 in ranges:
-        _lib.check(call(_at(S, b0), [_at(x, b0, t0) for x in ins], _at(y, b0, t0), b1 - b0, t1 - t0,
-                        ws.data_ptr(), nb), what)
+        rc = call(ws.data_ptr(), nb, b1 - b0, t1 - t0, _at(S, b0), _at(y, b0, t0), *[_at(x, b0, t0) for x in ins])
+        if rc:
+            return rc
+    return 0
 
 
 def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Tensor,
@@ -155,10 +157,12 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
     if chunked is None:
         chunked = _chunk_pays(T, H)
     if chunked:
-        def call(S_, i, y_, B_, T_, ws, nb):
-            return lib.rwkv7_wkv7_chunked(S_, i[0], i[1], w32, *i[2:], y_, B_, T_, H, bf, ws, nb, _lib.stream_handle())
+        f, st = lib.rwkv7_wkv7_chunked, _lib.stream_handle()
 
-        _chunked_scan(call, "rwkv7_wkv7_chunked", S, (r, w, k, v, a, b), y)
+        def call(ws, nb, B_, T_, S_, y_, r_, w_, k_, v_, a_, b_):
+            return f(S_, r_, w_, w32, k_, v_, a_, b_, y_, B_, T_, H, bf, ws, nb, st)
+
+        _lib.check(_chunked_scan(call, S, (r, w, k, v, a, b), y), "rwkv7_wkv7_chunked")
     else:
         _lib.check(lib.rwkv7_wkv7(S.data_ptr(), r.data_ptr(), w.data_ptr(), w32, k.data_ptr(), v.data_ptr(),
                                   a.data_ptr(), b.data_ptr(), y.data_ptr(), Bsz, T, H, bf, _lib.stream_handle()),
@@ -221,16 +225,16 @@ def dplr_seq_forward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: T
     batched = S.dim() == 4
     S1 = (S if batched else S.unsqueeze(0)).contiguous().clone()
     ins = [(x if batched else x.unsqueeze(0)).contiguous() for x in (R, W, K, V, A, B)]
-    _dev(S1, *ins)
-    _, T, H = _wkv7_f32_shapes(S1, *ins)
-    if _chunk_pays(T, H):
+    if ins[0].dim() == 4 and _chunk_pays(ins[0].shape[1], ins[0].shape[2]):
+        _dev(S1, *ins)
+        H = _wkv7_f32_shapes(S1, *ins)[2]
         y = torch.empty_like(ins[0])
-        lib = _lib.load()
+        f, st = _lib.load().rwkv7_wkv7_f32_chunked, _lib.stream_handle()
 
-        def call(S_, i, y_, B_, T_, ws, nb):
-            return lib.rwkv7_wkv7_f32_chunked(S_, *i, y_, B_, T_, H, ws, nb, _lib.stream_handle())
+        def call(ws, nb, B_, T_, S_, y_, *i):
+            return f(S_, *i, y_, B_, T_, H, ws, nb, st)
 
-        _chunked_scan(call, "rwkv7_wkv7_f32_chunked", S1, ins, y)
+        _lib.check(_chunked_scan(call, S1, ins, y), "rwkv7_wkv7_f32_chunked")
     else:
         y = wkv7_f32(S1, *ins)
     return (y, S1) if batched else (y[0], S1[0])
@@ -262,16 +266,21 @@ def dplr_seq_backward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: 
             _need(gS.shape == S1.shape and gS.dtype == torch.float32, "gS must be like S")
         out = (torch.empty_like(S1), *(torch.empty_like(x) for x in ins))
         lib = _lib.load()
-        nb, ranges = int(lib.rwkv7_wkv7_grad_workspace_bytes(Bsz, T, H)), [(0, Bsz, 0, T)]
-        if nb > CHUNK_WS_BYTES:
-            ranges = _chunk_ranges(Bsz, T, int(lib.rwkv7_wkv7_grad_workspace_bytes(1, T, H)), False)
-            nb = int(lib.rwkv7_wkv7_grad_workspace_bytes(ranges[0][1], T, H))
-        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        for b0, b1, _, _ in ranges:
-            rc = lib.rwkv7_wkv7_grad(_at(S1, b0), *(_at(x, b0) for x in ins), _at(gy, b0),
-                                     None if gS is None else _at(gS, b0), *(_at(g, b0) for g in out), b1 - b0, T, H,
-                                     ws.data_ptr(), nb, _lib.stream_handle())
+        nbytes, f, st = lib.rwkv7_wkv7_grad_workspace_bytes, lib.rwkv7_wkv7_grad, _lib.stream_handle()
+        nb = nbytes(Bsz, T, H)
+        if nb <= CHUNK_WS_BYTES:
+            ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+            rc = f(S1.data_ptr(), *(x.data_ptr() for x in ins), gy.data_ptr(), _lib.ptr(gS), *(g.data_ptr() for g in out),
+                   Bsz, T, H, ws.data_ptr(), nb, st)
             _lib.check(rc, "rwkv7_wkv7_grad")
+        else:
+            ranges = _chunk_ranges(Bsz, T, nbytes(1, T, H), False)
+            nb = nbytes(ranges[0][1], T, H)
+            ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+            for b0, b1, _, _ in ranges:
+                rc = f(_at(S1, b0), *(_at(x, b0) for x in ins), _at(gy, b0), None if gS is None else _at(gS, b0),
+                       *(_at(g, b0) for g in out), b1 - b0, T, H, ws.data_ptr(), nb, st)
+                _lib.check(rc, "rwkv7_wkv7_grad")
     return out if batched else tuple(g[0] for g in out)
 
 
