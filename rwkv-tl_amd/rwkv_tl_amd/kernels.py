@@ -91,6 +91,16 @@ def _chunk_pays(T: int, H: int) -> bool:
     return T >= CHUNK_MIN_T and _chunk_fits(T, H)
 
 
+def _history_pays(Bsz: int, T: int, H: int) -> bool:
+    """Whether the gradient records the states and walks them backward: one or
+    two tokens of many heads, where a chunk's records and products are mostly
+    padding. Measured on MI355X, us per call, recorded / chunked: 1 token of 256
+    heads 42.6 / 34.4, of 384 42.7 / 45, of 1024 43.5 / 78, of 4096 137 / 287; 2 tokens
+    of 384 heads 43 / 46, of 1024 65 / 80, of 4096 270 / 292; 3 tokens of 512 heads 48 /
+    52, of 1024 84 / 82, of 4096 362 / 298."""
+    return T <= 2 and Bsz * H >= 384
+
+
 def _chunk_ranges(Bsz: int, T: int, seq_bytes: int, cut_tokens: bool) -> list[tuple[int, int, int, int]]:
     """Ranges ``(b0, b1, t0, t1)`` of a batch whose sequences each take
     ``seq_bytes`` of workspace, in order, within ``CHUNK_WS_BYTES``: whole
@@ -246,21 +256,24 @@ def dplr_seq_backward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: 
     its inputs (the reference's plan, TODO.md:46-54, recomputes the states
     too): chunked scans of the states and of their adjoint, then every chunk at
     once (``rwkv7_wkv7_grad``; a workspace of 6.2 KB per token and head, of at
-    most ``CHUNK_WS_BYTES`` or one sequence's)."""
+    most ``CHUNK_WS_BYTES`` or one sequence's). One or two tokens of many heads,
+    and sequences past the chunk kernels' offsets, record every state in a
+    forward pass (16 KB per token and head) and walk them backward."""
     batched = S.dim() == 4
     u = (lambda x: x) if batched else (lambda x: x.unsqueeze(0))
     S1 = u(S).contiguous()
     ins = [u(x).contiguous() for x in (R, W, K, V, A, B)]
     gy = u(gy).contiguous()
     gS = None if gS is None else u(gS).contiguous()
-    _dev(S1, *ins, gy)
-    Bsz, T, H = _wkv7_f32_shapes(S1, *ins, gy)
-    if not _chunk_fits(T, H):
+    Bsz, T, H = ins[0].shape[:3] if ins[0].dim() == 4 else (0, 0, 0)
+    if not _chunk_fits(T, H) or _history_pays(Bsz, T, H):  # (both functions check the operands)
         S1 = S1.clone()
         hist = torch.empty(Bsz, H, T, N, N, dtype=torch.float32, device=S.device)
         wkv7_f32(S1, *ins, hist=hist)
         out = wkv7_backward(hist, S1, *ins, gy, gS)
     else:
+        _dev(S1, *ins, gy)
+        _wkv7_f32_shapes(S1, *ins, gy)
         if gS is not None:
             _dev(gS)
             _need(gS.shape == S1.shape and gS.dtype == torch.float32, "gS must be like S")

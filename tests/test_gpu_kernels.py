@@ -697,3 +697,21 @@ def test_large_chunked_calls_keep_to_the_workspace_bound(cuda):
     S = torch.zeros(B, H, 64, 64, device=cuda)
     y, peak = _peak(lambda: K.wkv7(S, x, w, x, x, x, x))
     assert peak <= K.CHUNK_WS_BYTES + y.numel() * 2 + (1 << 22)
+
+
+@pytest.mark.parametrize("T", [1, 2, 3])
+def test_gradient_of_a_few_tokens_of_many_heads(T, cuda):
+    """384 heads of 1 to 3 tokens against 64 bits (fp32 sums of 64 terms and a few
+    steps, 2e-6); one and two tokens take the recorded states, with no chunk
+    workspace."""
+    B, H = 24, 16
+    ins = [x.to(cuda) for x in _dplr_inputs(B, T, H, seed=T)]
+    g = torch.Generator().manual_seed(T)
+    gy = torch.randn(B, T, H, 64, generator=g).to(cuda)
+    gS = torch.randn(B, H, 64, 64, generator=g).to(cuda)
+    ref = _grads64(ins, gy, gS)[2:]
+    got, peak = _peak(lambda: K.dplr_seq_backward(*ins, gy, gS))
+    for name, x, e in zip(("gS0", "gr", "gw", "gk", "gv", "ga", "gb"), got, ref):
+        assert _rel(x, e) < 2e-6, f"{name}: {_rel(x, e):.2e}"
+    records = int(K._lib.load().rwkv7_wkv7_grad_workspace_bytes(B, T, H))
+    assert (peak < records) == (T <= 2)
