@@ -69,11 +69,18 @@ def _h16(*ts: Tensor) -> int:
     return int(dt == torch.bfloat16)
 
 
-# The operators take the chunked scan for sequences at least this long
-# (measured on MI355X, us per call, serial / chunked: B=1, H=16, T=64 14.9 /
-# 19.2, T=128 21.4 / 19.1; B=8, H=16, T=64 15.4 / 20.5, T=128 28.1 / 24.9;
-# B=16, H=32, T=128 102 / 74, T=1024 840 / 539).
-CHUNK_MIN_T = 128
+# The wkv7 operator takes the chunked scan for sequences at least this long
+# (measured on MI355X, us per call, serial / chunked, 16 heads: T=112 19.0 /
+# 20.1, T=120 20.4 / 20.4, T=127 21.1 / 20.2; 64 heads: T=104 18.2 / 21.5, T=112
+# 21.4 / 20.9; 128 heads: T=64 15.4 / 20.5, T=112 25.1 / 24.9, T=128 28.1 / 25.2;
+# 512 heads: T=96 78 / 62, T=128 102 / 76, T=1024 840 / 539: the line could lie
+# lower for many heads).
+CHUNK_MIN_T = 120
+# The f32 training forward pays more host time for its second launch: from 128
+# tokens with at least 48 heads, else from 144 (us per call, serial / chunked, 16
+# heads: T=128 22.7 / 24.3, T=144 24.6 / 24.4; 48 heads: T=128 26.1 / 24.5; 1024
+# heads: T=128 198 / 172).
+CHUNK_MIN_T_F32 = (128, 144)
 # Bytes of chunk records (28,928 per 16 tokens and head) that one call holds at
 # most; beyond, the scan runs over ranges of the batch, or of one sequence's
 # tokens, that share them (the same results: records are per 16 tokens, and the
@@ -89,6 +96,10 @@ def _chunk_fits(T: int, H: int) -> bool:
 
 def _chunk_pays(T: int, H: int) -> bool:
     return T >= CHUNK_MIN_T and _chunk_fits(T, H)
+
+
+def _chunk_pays_f32(Bsz: int, T: int, H: int) -> bool:
+    return T >= CHUNK_MIN_T_F32[Bsz * H < 48] and _chunk_fits(T, H)
 
 
 def _history_pays(Bsz: int, T: int, H: int) -> bool:
@@ -235,7 +246,7 @@ def dplr_seq_forward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: T
     batched = S.dim() == 4
     S1 = (S if batched else S.unsqueeze(0)).contiguous().clone()
     ins = [(x if batched else x.unsqueeze(0)).contiguous() for x in (R, W, K, V, A, B)]
-    if ins[0].dim() == 4 and _chunk_pays(ins[0].shape[1], ins[0].shape[2]):
+    if ins[0].dim() == 4 and _chunk_pays_f32(*ins[0].shape[:3]):
         _dev(S1, *ins)
         H = _wkv7_f32_shapes(S1, *ins)[2]
         y = torch.empty_like(ins[0])

@@ -610,16 +610,19 @@ def _grads64(ins, gy, gS):
     return [y.detach(), S.detach(), *torch.autograd.grad((y, S), xs, (gy.double(), gS.double()))]
 
 
-@pytest.mark.parametrize("decay", ["plain", "strong"])
+@pytest.mark.parametrize("decay", ["plain", "strong", "zero"])
 def test_chunked_scans_are_as_exact_as_the_serial_scan(decay, cuda):
     """Against 64 bits, the chunked forward and gradient may be no further off
     than the serial scan and the history backward, whose every step rounds: the
     same error to the 5 % by which the rounding of 0.2 million values varies
-    between inputs (strong: products of w below 1e-30, the direct form)."""
+    between inputs (strong: products of w below 1e-30, zero: some w = 0, the
+    direct form)."""
     B, T, H = 2, 160, 10
     ins = [x.to(cuda) for x in _dplr_inputs(B, T, H, seed=3)]
     if decay == "strong":
         ins[2] = ins[2] ** 12
+    elif decay == "zero":
+        ins[2] = ins[2] * (torch.rand(ins[2].shape, generator=torch.Generator().manual_seed(5)) >= 0.05).to(cuda)
     g = torch.Generator().manual_seed(4)
     gy = torch.randn(B, T, H, 64, generator=g).to(cuda)
     gS = torch.randn(B, H, 64, 64, generator=g).to(cuda) * 0.1
@@ -645,9 +648,9 @@ def test_chunked_scans_are_as_exact_as_the_serial_scan(decay, cuda):
 def test_chunked_f32_scans_keep_the_range_of_their_inputs(which, scale, cuda):
     """Decays whose products over a chunk come close to 1e-30 (0.016^16 = 2e-29)
     with inputs that leave f32's range when scaled by them: the chunked forward
-    (130 tokens) and gradient (40) against 64 bits. fp32 sums of up to 64 + 130
+    (146 tokens) and gradient (40) against 64 bits. fp32 sums of up to 64 + 146
     terms; measured below 2e-7, asserted at ten times that."""
-    for T in (130, 40):
+    for T in (146, 40):
         ins = [x.to(cuda) for x in _dplr_inputs(1, T, 2, seed=T)]
         ins[2] = torch.full_like(ins[2], 0.016)
         ins[which] = ins[which] * scale
@@ -668,7 +671,7 @@ def _peak(fn):
     return out, torch.cuda.max_memory_allocated() - base
 
 
-@pytest.mark.parametrize("B,T,H,limit", [(5, 130, 3, 2), (2, 200, 2, 1), (1, 333, 2, 0.3), (3, 129, 1, 0.5)])
+@pytest.mark.parametrize("B,T,H,limit", [(5, 150, 3, 2), (2, 200, 2, 1), (1, 333, 2, 0.3), (3, 145, 1, 0.5)])
 def test_chunked_scans_in_ranges_of_a_bounded_workspace(B, T, H, limit, cuda, monkeypatch):
     """A workspace of ``limit`` sequences' records: batches in parts, sequences in
     parts of whole chunks (the gradient: whole sequences), the same bits."""
@@ -715,3 +718,21 @@ def test_gradient_of_a_few_tokens_of_many_heads(T, cuda):
         assert _rel(x, e) < 2e-6, f"{name}: {_rel(x, e):.2e}"
     records = int(K._lib.load().rwkv7_wkv7_grad_workspace_bytes(B, T, H))
     assert (peak < records) == (T <= 2)
+
+
+@pytest.mark.parametrize("T", [119, 120, 127, 128, 143, 144])
+@pytest.mark.parametrize("B", [1, 24], ids=["2_heads", "48_heads"])
+def test_scans_around_the_lines_of_the_chunked_form(B, T, cuda):
+    """Both sides of the lengths from which the operator and the training forward
+    are chunked, against the serial scan (fp32 sums of 64 terms and 144 steps:
+    below 1e-6 apart; f16 outputs to half a unit, 2^-11 of a value)."""
+    ins = [x.to(cuda) for x in _dplr_inputs(B, T, 2, seed=T)]
+    S1 = ins[0].clone()
+    y1 = K.wkv7_f32(S1, *ins[1:])
+    y, S_T = K.dplr_seq_forward(*ins)
+    assert _rel(y, y1) < 1e-6 and _rel(S_T, S1) < 1e-6
+    h = [x.half() for x in ins[1:]]
+    S2, S3 = ins[0].clone(), ins[0].clone()
+    y2, y3 = K.wkv7(S2, *h), K.wkv7(S3, *h, chunked=False)
+    assert _rel(S2, S3) < 1e-6
+    assert _rel(y2.float(), y3.float()) < 2**-11
