@@ -136,10 +136,11 @@ struct BatchWs {
   float *x0, *rkv, *d, *vfirst, *kv, *y, *part;  // kv: gated k, mixed v [2][M][C]
   float *proj1;  // one-token steps: r, k, v, raw LoRA first steps [M, 3C+SR]
   void *xmix, *l1, *yg, *hid, *headin;
-  float *x1;  // the other residual buffer of split steps (LnShiftArgs::x_out)
+  float *x1;  // the other residual buffer of steps with a sliced FFN value (LnShiftArgs::x_out), else null
   float *U, *Send, *Pend;  // segmented scan of long sequences (null with one segment)
   float *rec;              // chunk records of the chunked scan (prefill_chunked)
 };
+static bool batch_a32(const rwkv7_dims &d, int M);
 static int64_t batch_ws(const rwkv7_dims &d, int64_t B, int64_t T, char *base, BatchWs *w) {
   const int64_t C = d.n_embd, F = d.n_ffn, SR = sum_ranks(d), M = B * T;
   int64_t off = fixed_bytes(d);
@@ -150,13 +151,14 @@ static int64_t batch_ws(const rwkv7_dims &d, int64_t B, int64_t T, char *base, B
   };
   BatchWs t;
   // operand buffers hold whole 16-row blocks (split order), the LoRA first
-  // steps' also whole 32-column blocks of each
+  // steps' of steps with f32 activations also whole 32-column blocks of each
   const int64_t M16 = (M + 15) / 16 * 16, B16 = (B + 15) / 16 * 16;
+  const int splits = gemm_frag_splits((int)M, (int)C, (int)F);
   t.x0 = reinterpret_cast<float *>(take(M * C * 4));
-  t.x1 = reinterpret_cast<float *>(take(M * C * 4));
+  t.x1 = splits > 1 ? reinterpret_cast<float *>(take(M * C * 4)) : nullptr;
   t.xmix = take(6 * M16 * C * 4);
   t.rkv = reinterpret_cast<float *>(take(3 * M * C * 4));
-  t.l1 = take(M16 * (SR + 4 * 32) * 4);
+  t.l1 = take(M16 * (SR + (batch_a32(d, (int)M) ? 4 * 32 : 0)) * 4);
   t.d = reinterpret_cast<float *>(take(4 * M * C * 4));
   t.vfirst = reinterpret_cast<float *>(take(M * C * 4));
   t.kv = reinterpret_cast<float *>(take(2 * M * C * 4));
@@ -166,7 +168,7 @@ static int64_t batch_ws(const rwkv7_dims &d, int64_t B, int64_t T, char *base, B
   t.headin = take(B16 * C * 4);
   t.proj1 = T == 1 ? reinterpret_cast<float *>(take(M * (3 * C + SR) * 4)) : nullptr;
   const int cus = mk_cus() > 0 ? mk_cus() : 256;
-  const int64_t gws = gemm_ws_bytes((int)(M > B ? M : B), cus), fws = gemm_frag_splits((int)M, (int)C, (int)F) * M * C * 4;
+  const int64_t gws = gemm_ws_bytes((int)(M > B ? M : B), cus), fws = splits > 1 ? splits * M * C * 4 : 0;
   t.part = reinterpret_cast<float *>(take(gws > fws ? gws : fws));
   int seg_len;
   const int64_t nseg = prefill_segments((int)T, (int)B, d.n_head, cus, &seg_len);

@@ -383,3 +383,20 @@ def test_chunk_ranges_cover_the_batch_within_the_workspace(B, T, per16, cut):
         assert len(ranges) == 1 or max(size) > K.CHUNK_WS_BYTES // 2  # (no smaller than it need be)
     else:
         assert all(b1 == b0 + 1 and (t0, t1) == (0, T) for b0, b1, t0, t1 in ranges)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the sizes of a host without a GPU (256 CUs)")
+@pytest.mark.parametrize("shape", ["0.4b", "1.5b"])
+def test_long_prefill_workspace_holds_what_a_long_prefill_uses(shape):
+    """4 x 1024 tokens: 19 rows of C floats a token (residual, six mixes, r/k/v,
+    four LoRA steps, v_first, two gated, y, gate input), the hidden row, the LoRA
+    first steps and the chunk records; the second residual row and the padded
+    LoRA columns belong to shorter steps."""
+    lib = _lib.load()
+    d = _dims(shape)
+    M, C = 4 * 1024, d.n_embd
+    SR = sum(getattr(d, f"rank_{c}") for c in "wavg")
+    rows = M * 4 * (19 * C + d.n_ffn + SR) + M // 16 * d.n_head * 28928
+    fixed = 24 << 20  # split-K partials (16 MiB) and the buffers of any size
+    got = lib.rwkv7_workspace_bytes(ctypes.byref(d), 4, 1024)
+    assert rows <= got <= rows + fixed, (got - rows, fixed)
