@@ -249,10 +249,6 @@ static int decode_one(const rwkv7_model &m, const rwkv7_state &s, const int64_t 
     t.layer0 = l == 0;
     t.yg16 = nullptr;
     t.bf = bf;
-    if (m.layers_frag) {
-      const char *Fl = static_cast<const char *>(m.layers_frag) + (int64_t)l * lay.frag_bytes;
-      for (int g = 0; g < 4; ++g) t.f_l2[g] = reinterpret_cast<const uint16_t *>(Fl + lay.f_l2[g]);
-    }
     RWKV7_TRY(launch_tmix_decode(t, 1, st));
 
     GemvArgs o = {};
