@@ -581,6 +581,11 @@ def test_persistent_decode_abort_is_visible(cuda):
     (1280, 4352, (64, 64, 32, 128), 3, 107),  # 321 rows: operands through LDS, columns past the last tile
     (1280, 4352, (64, 64, 32, 128), 6, 107),  # 642 rows: 128 x 128 tiles in several rounds
     (256, 4096, (24, 8, 16, 40), 97, 8),      # several rounds at K = 256: register-fed tiles
+    (2048, 8192, (96, 96, 64, 256), 1, 200),  # FFN value: 64 x 128 tiles through LDS, four K slices
+    (2048, 8192, (88, 104, 72, 248), 33, 1),  # LoRA second steps of the decode core from fragments, padded ranks
+    (2304, 2304, (64, 64, 32, 128), 3, 11),   # three pieces per LayerNorm thread, the last part idle
+    (2304, 2304, (64, 64, 32, 128), 19, 1),   # one-token steps of the same
+    (3328, 3328, (64, 64, 32, 128), 1, 20),   # four pieces
 ])
 def test_fragment_gemm_steps_match_row_major_weights(dtype, C, F, ranks, B, T, cuda):
     """Steps of more than eight rows on the fragment arenas (activations stored in
