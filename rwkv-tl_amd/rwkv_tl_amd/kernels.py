@@ -131,15 +131,11 @@ def _at(x: Tensor, b: int, t: int = 0) -> int:
     return x.data_ptr() + (b * x.stride(0) + t * x.stride(1)) * x.element_size()
 
 
-def _chunked_scan(call, S: Tensor, ins: tuple[Tensor, ...], y: Tensor) -> int:
+def _chunked_in_ranges(call, S: Tensor, ins: tuple[Tensor, ...], y: Tensor) -> int:
     """``call(ws, nb, B, T, S, y, *ins)`` (addresses; a C call's return code) on
-    the batch, or on the ranges of it that share one workspace."""
+    the ranges of a batch that share one workspace."""
     Bsz, T, H = y.shape[:3]
     nbytes = _lib.load().rwkv7_wkv7_chunked_workspace_bytes
-    nb = nbytes(Bsz, T, H)
-    if nb <= CHUNK_WS_BYTES:
-        ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
-        return call(ws.data_ptr(), nb, Bsz, T, S.data_ptr(), y.data_ptr(), *[x.data_ptr() for x in ins])
     ranges = _chunk_ranges(Bsz, T, nbytes(1, T, H), _chunk_fits(T, H))
     b0, b1, t0, t1 = ranges[0]  # the largest
     nb = nbytes(b1 - b0, t1 - t0, H)
@@ -179,11 +175,16 @@ def wkv7(S: Tensor, r: Tensor, w: Tensor, k: Tensor, v: Tensor, a: Tensor, b: Te
         chunked = _chunk_pays(T, H)
     if chunked:
         f, st = lib.rwkv7_wkv7_chunked, _lib.stream_handle()
-
-        def call(ws, nb, B_, T_, S_, y_, r_, w_, k_, v_, a_, b_):
-            return f(S_, r_, w_, w32, k_, v_, a_, b_, y_, B_, T_, H, bf, ws, nb, st)
-
-        _lib.check(_chunked_scan(call, S, (r, w, k, v, a, b), y), "rwkv7_wkv7_chunked")
+        nb = lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H)
+        if nb <= CHUNK_WS_BYTES:
+            ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+            rc = f(S.data_ptr(), r.data_ptr(), w.data_ptr(), w32, k.data_ptr(), v.data_ptr(), a.data_ptr(),
+                   b.data_ptr(), y.data_ptr(), Bsz, T, H, bf, ws.data_ptr(), nb, st)
+        else:
+            rc = _chunked_in_ranges(lambda ws, nb, B_, T_, S_, y_, r_, w_, k_, v_, a_, b_:
+                                    f(S_, r_, w_, w32, k_, v_, a_, b_, y_, B_, T_, H, bf, ws, nb, st),
+                                    S, (r, w, k, v, a, b), y)
+        _lib.check(rc, "rwkv7_wkv7_chunked")
     else:
         _lib.check(lib.rwkv7_wkv7(S.data_ptr(), r.data_ptr(), w.data_ptr(), w32, k.data_ptr(), v.data_ptr(),
                                   a.data_ptr(), b.data_ptr(), y.data_ptr(), Bsz, T, H, bf, _lib.stream_handle()),
@@ -246,16 +247,20 @@ def dplr_seq_forward(S: Tensor, R: Tensor, W: Tensor, K: Tensor, V: Tensor, A: T
     batched = S.dim() == 4
     S1 = (S if batched else S.unsqueeze(0)).contiguous().clone()
     ins = [(x if batched else x.unsqueeze(0)).contiguous() for x in (R, W, K, V, A, B)]
-    if ins[0].dim() == 4 and _chunk_pays_f32(*ins[0].shape[:3]):
+    Bsz, T, H = ins[0].shape[:3] if ins[0].dim() == 4 else (0, 0, 0)
+    if _chunk_pays_f32(Bsz, T, H):
         _dev(S1, *ins)
-        H = _wkv7_f32_shapes(S1, *ins)[2]
+        _wkv7_f32_shapes(S1, *ins)
         y = torch.empty_like(ins[0])
-        f, st = _lib.load().rwkv7_wkv7_f32_chunked, _lib.stream_handle()
-
-        def call(ws, nb, B_, T_, S_, y_, *i):
-            return f(S_, *i, y_, B_, T_, H, ws, nb, st)
-
-        _lib.check(_chunked_scan(call, S1, ins, y), "rwkv7_wkv7_f32_chunked")
+        lib = _lib.load()
+        f, st = lib.rwkv7_wkv7_f32_chunked, _lib.stream_handle()
+        nb = lib.rwkv7_wkv7_chunked_workspace_bytes(Bsz, T, H)
+        if nb <= CHUNK_WS_BYTES:
+            ws = torch.empty(nb, dtype=torch.uint8, device=S.device)
+            rc = f(S1.data_ptr(), *(x.data_ptr() for x in ins), y.data_ptr(), Bsz, T, H, ws.data_ptr(), nb, st)
+        else:
+            rc = _chunked_in_ranges(lambda ws, nb, B_, T_, S_, y_, *i: f(S_, *i, y_, B_, T_, H, ws, nb, st), S1, ins, y)
+        _lib.check(rc, "rwkv7_wkv7_f32_chunked")
     else:
         y = wkv7_f32(S1, *ins)
     return (y, S1) if batched else (y[0], S1[0])
