@@ -1061,7 +1061,7 @@ RWKV7_DEV void lora2_chunk(const PrefillScanArgs &p, St &st, int h, int bi, int 
 // record is stored from the registers that hold it. Three barriers after the
 // staging (four where U passes between waves) against eight when each
 // intermediate went through LDS. Measured (kernel trace): 1024 chunks of raw
-// half inputs 20.4 -> 14.8 us; 2048 of f32 inputs 25 us, 109 MB moved (4.4
+// half inputs 20.4 -> 14.9 us; 2048 of f32 inputs 25 us, 109 MB moved (4.4
 // TB/s; a large copy reaches 4.9 here).
 // Error: no larger than the serial scan's against 64 bits (512 tokens, f32: y
 // 0.94e-7 and 1.00e-7, state 0.43e-7 and 0.50e-7). That takes the products of w
@@ -1149,25 +1149,36 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
     x[t] = s_x[xi][t][lane];
     if (wv == 2) z[t] = s_x[3][t][lane];
   }
-  bool ok = true;
-  {
-    float P = 1.f;
+  // the smallest and largest prefix product (a NaN stays in the last one)
+  float P = 1.f, p_lo = 1.f, p_hi = 1.f;
 #pragma unroll
-    for (int t = 0; t < kCk; ++t) {
-      P *= w[t];
-      ok = ok && P >= 1e-30f && P <= 1e30f;  // false for NaN too
-    }
+  for (int t = 0; t < kCk; ++t) {
+    P *= w[t];
+    p_lo = fminf(p_lo, P);
+    p_hi = fmaxf(p_hi, P);
   }
   // the same w in every wave, so the same answer: uniform over the workgroup
-  bool fast = __all(ok);
+  bool fast = __all(p_lo >= 1e-30f && p_hi <= 1e30f && P == P);
   if constexpr (St::kWide) {
-    // Inputs of f32's range scaled by P or 1 / P may leave it: at 1e30 a row
-    // keeps its precision if its largest value is in [1e-7, 1e7] (below, what
-    // the last denormal cuts off shows; half's whole range passes)
+    // Inputs of f32's range scaled by P or 1 / P may leave it. Nearly always P is
+    // in [1e-12, 1e12] and every value zero or in [1e-25, 1e25]: nothing is lost.
+    // Otherwise, at 1e30, a row keeps its precision if its largest value is in
+    // [1e-7, 1e7] (below, what the last denormal cuts off shows; half's whole
+    // range passes).
+    uint32_t u_lo = ~0u, u_hi = 0u;
 #pragma unroll
     for (int t = 0; t < kCk; ++t) {
-      const float m = fabsf(x[t]);
-      fast = fast && __all(m <= 1e7f) && (__any(m >= 1e-7f) || !__any(m > 0.f));  // false for NaN
+      const uint32_t u = __float_as_uint(x[t]) & 0x7FFFFFFFu;
+      u_lo = min(u_lo, u - 1u);  // (a zero wraps around)
+      u_hi = max(u_hi, u);
+    }
+    if (!__all(p_lo >= 1e-12f && p_hi <= 1e12f && u_lo >= __float_as_uint(1e-25f) - 1u &&
+               u_hi <= __float_as_uint(1e25f))) {
+#pragma unroll 1
+      for (int t = 0; t < kCk; ++t) {
+        const float m = fabsf(s_x[xi][t][lane]);
+        fast = fast && __all(m <= 1e7f) && (__any(m >= 1e-7f) || !__any(m > 0.f));  // false for NaN
+      }
     }
     if (lane == 0) s_ok[wv] = fast;
   }
