@@ -308,7 +308,7 @@ int rwkv7_wkv7_f32_chunked(float *S, const float *r, const float *w, const float
  * S0 [B, H, 64, 64] is the state before the sequence (not written), no history
  * is read. Chunked scans of the states and of their adjoint, then every
  * 16-token chunk at once; the workspace holds the chunk records and boundary
- * states (about 5 KB per token and head). The gradient half of the DPLR
+ * states (6.2 KB per token and head, 90 KB at least). The gradient half of the DPLR
  * backward the reference plans (TODO.md:46-54), recomputing its states.
  * RWKV7_ESHAPE as rwkv7_wkv7_f32_chunked. */
 int64_t rwkv7_wkv7_grad_workspace_bytes(int32_t B, int32_t T, int32_t H);

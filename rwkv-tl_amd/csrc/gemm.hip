@@ -698,9 +698,10 @@ static int big_rows_per_launch(int64_t lda) {
 }
 
 // Problems of the large-M path: K a multiple of 64, at least 256 columns, and
-// enough 128 x 128 tiles for two workgroups per CU (measured: at M = 512 the
-// 32-row tiled kernels with split-K are 2-3x faster; at M = 4096 this path is
-// ~2x faster than them).
+// enough 128 x 128 tiles for two workgroups per CU (measured in the model's
+// steps: at M = 512 the 32-row tiled kernels with split-K are 2-3x faster; at M =
+// 4096 this path is ~2x faster than them. The gemm operator passes no workspace,
+// so its tiled kernels don't split K; the line was not measured for it).
 static bool big_fits(const GemmProb &p, int M, int cus) {
   return !p.a32 && p.K % kBigBK == 0 && p.N >= 256 &&
          (int64_t)((M + 127) / 128) * ((p.N + 127) / 128) >= 2 * cus && big_w_addressable(p) &&

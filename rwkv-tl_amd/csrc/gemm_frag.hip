@@ -447,10 +447,10 @@ static int64_t frag_units(const FragTile &t, int M, int N) {
 // long enough to pay for filling the ring, and of several rounds each takes
 // 128 x 128 if K covers its unoverlapped ends as well: two register-fed
 // workgroups share a CU and hide theirs in each other. Measured, whole
-// prefills in us, register-fed / ring: 1.5B 1 x 129 3411 / 2862, 4 x 64 4245 /
-// 3665, 8 x 96 9268 / 8374 (64 x 128 ring 8517), 0.4B 3 x 129 2734 / 2609, 1 x
-// 509 3229 / 3133, 16 x 100 7031 / 6692 (6997); 0.1B (K 768) 8 x 60 1198 / 1168,
-// but 16 x 96, three rounds, 2806 / 2891 (2939).
+// prefills in us, register-fed / ring: 1.5B 1 x 129 3371 / 2879, 4 x 64 3686 /
+// 3331, 8 x 96 8989 / 8443, 0.4B 3 x 129 2404 / 2325, 1 x 509 2859 / 2827, 16 x
+// 100 6484 / 6401; 0.1B (K 768) 8 x 60 1078 / 1052, but 16 x 96, three rounds,
+// 2505 / 2683.
 constexpr int kFragRingMinK = 512, kFragRoundsMinK = 1024;
 static bool frag_ring(const GemmProb *probs, int nprob, int M, int min_k) {
   int k = 0;
@@ -475,10 +475,14 @@ static int frag_tile(const GemmProb *probs, int nprob, int M, int cus) {
 // long K leave each CU a small tile with all of K: its operands' bytes are the
 // time. Cutting K lets the tiles be larger; the (tile, slices) with the fewest
 // bytes per workgroup among those that run at once. At most four slices of at
-// least 1024, and only up to 256 rows: beyond, the partials' bytes outweigh it
-// (measured, FFN value, us, best whole / best cut: 0.4B 64 rows 11.1 / 7.8, 128
-// rows 11.0 / 8.7, 512 rows 17.9 / 16.6; 1.5B 64 rows 19.6 / 14.6, and 14.2 with
-// eight slices, less than their extra partials cost the LayerNorm).
+// least 1024 (measured, FFN value, us, best whole / best cut: 0.4B 64 rows 11.1 /
+// 7.8, 128 rows 11.0 / 8.7; 1.5B 64 rows 19.6 / 14.6, and 14.2 with eight slices,
+// less than their extra partials cost the LayerNorm), and only up to 256 rows.
+// Beyond, the partials that the LayerNorm reads grow with the rows and the gain
+// depends on the shape (whole prefills, us, whole / cut: 0.4B 261 rows 2387 /
+// 2283, 300 2442 / 2449, 400 2578 / 2607, 512 2831 / 2893; 0.1B 480 rows 1206 /
+// 1226; 1.5B 257 rows 4592 / 4273, 512 5579 / 5335): one line for all leaves 4 to
+// 7 % of the 1.5B shape there, until the plan counts the partials' bytes.
 static int frag_plan(int M, int N, int K, int cus, int *splits) {
   GemmProb p = {};
   p.N = N;

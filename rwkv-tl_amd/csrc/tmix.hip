@@ -30,9 +30,12 @@ constexpr int kMaxRanks = 512;  // SR = rv + rw + ra + rg of the batched decode 
 // channels x 32 ranks; row-major, each lane reads its own channel's row, 64
 // lines per load of which 16 bytes are used, and the eight workgroups of a CU
 // thrash its L1. Taken from kFragRanks ranks in all and kFragGroups
-// workgroups, four per CU (measured, us, row-major / fragments: 1.5B, ranks
-// 96/96/64/256, 3 sequences 8.2 / 9.3, 64 sequences 31.8 / 27.5; 0.4B, ranks
-// 64/64/32/128, 24 sequences 10.0 / 11.2, 128 sequences 24.2 / 24.3).
+// workgroups, four per CU (measured, us per decode step, row-major / fragments:
+// 1.5B, ranks 96/96/64/256, 32 workgroups a sequence: 9 sequences 1525 / 1552, 16
+// 1592 / 1596, 20 1785 / 1782, 24 1825 / 1803, 32 1931 / 1894, 64 2364 / 2233; 0.4B,
+// ranks 64/64/32/128, 16 a sequence: 24 sequences 1087 / 1115, 128 1619 / 1666).
+// Fragments are 1 % ahead from 640 workgroups already; the line is where they
+// are clearly so.
 constexpr int kFragRanks = 384, kFragGroups = 1024;
 template <bool BF, bool FRAG>
 __global__ __launch_bounds__(256) void tmix_decode_kernel(TmixDecodeArgs a) {
