@@ -1187,39 +1187,43 @@ __global__ __launch_bounds__(256) void wkv7_chunk_prep_kernel(typename St::Args 
   }
   __syncthreads();  // the rows are read: they may be overwritten
   if constexpr (St::kWide) fast = s_ok[0] && s_ok[1] && s_ok[2] && s_ok[3];
-  if (!fast) {      // token matrices straight from products of w: thread (t, s)
-    const int t = tid >> 4, s = tid & 15;
-    float aba = 0.f, aka = 0.f, bbr = 0.f, bkr = 0.f;
-    if (s <= t) {
+  if (!fast) {
+    // Token matrices straight from products of w: wave m matrix m, lane -> token
+    // s = row and 16 of its channels, decayed on through the later tokens t as the
+    // serial scan decays its state. (A thread per (t, s) that forms each product
+    // anew took 36 us: one token with w = 0, as between packed sequences, made the
+    // operator at 8 x 128 tokens of 16 heads 62 us, now 31; the serial scan 29. At 16 x
+    // 1024, 32 heads, such a token per 100: 1767 us, now 760; serial 845.)
+    // (eight channels at a time: sixteen raise the kernel from 64 to 72 registers,
+    // and the prep of a 4 x 1024 prefill, which never comes here, from 106 to 123 us)
+    const bool strict = wv < 2 || ADJ;  // s < t and D(s, t-1], else s <= t and D(s, t]
 #pragma unroll 1
-      for (int j0 = 0; j0 < kN; j0 += 8) {  // sums of 8 channels, as below
-        float q[4] = {};
-#pragma unroll 1  // (unrolled, the kernel takes 72 registers for 64, and 125 us for 111 where it is not even run)
-        for (int j = j0; j < j0 + 8; ++j) {
-          float d = 1.f;  // D(s, t-1]
-          for (int m = s + 1; m < t; ++m) d *= s_x[0][m][j];
-          const float dt = s < t ? d * s_x[0][t][j] : 1.f;  // D(s, t]
-          const float bs = s_x[2][s][j], ks = s_x[3][s][j], at = s_x[1][t][j], rt = s_x[4][t][j];
-          if (s < t) {
-            q[0] = fmaf(bs * d, at, q[0]);
-            q[1] = fmaf(ks * d, at, q[1]);
-          }
-          if (!ADJ || s < t) {
-            q[2] = fmaf(bs * (ADJ ? d : dt), rt, q[2]);
-            q[3] = fmaf(ks * (ADJ ? d : dt), rt, q[3]);
-          }
+    for (int c0 = 16 * kq; c0 < 16 * kq + 16; c0 += 8) {
+      float y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = s_x[(wv & 1) ? 3 : 2][row][c0 + i];
+#pragma unroll 1
+      for (int t = 0; t < kCk; ++t) {
+        const float *xt = &s_x[wv < 2 ? 1 : 4][t][c0], *wt = &s_x[0][t][c0];
+        const bool later = row < t;
+        if (!strict && later) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) y[i] *= wt[i];
         }
-        aba += q[0];
-        aka += q[1];
-        bbr += q[2];
-        bkr += q[3];
+        float d = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d = fmaf(y[i], xt[i], d);
+        if (strict && later) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) y[i] *= wt[i];
+        }
+        d += __shfl_xor(d, 16);
+        d += __shfl_xor(d, 32);
+        d = later || (!strict && row == t) ? d : 0.f;
+        if (ADJ && wv == 3 && row == t) d = s_diag[t];
+        if (kq == 0) s_m[wv][t][row] = c0 == 0 || (ADJ && wv == 3 && row == t) ? d : s_m[wv][t][row] + d;
       }
     }
-    if (ADJ && s == t) bkr = s_diag[t];
-    s_m[0][t][s] = aba;
-    s_m[1][t][s] = aka;
-    s_m[2][t][s] = bbr;
-    s_m[3][t][s] = bkr;
     __syncthreads();
   }
   // a~ = a D(-1, t-1], r~ = r D(-1, t] and (for the MFMA form) k / P, b / P,
