@@ -154,11 +154,12 @@ int launch_wkv7_prefill(const PrefillScanArgs &p, hipStream_t st);
 // prefill_chunked: the model's prefill takes the chunked scan for sequences
 // of at least kChunkMinT tokens (measured on MI355X against the serial scan,
 // whose four workgroups per head each compute the head's gate math: 0.4B
-// 1 x 128 and 1 x 512 and the 1.5B-shaped 4 x 1024 faster, 0.4B 1 x 32 1253
-// us serial, 1296 chunked). From 56 tokens on the chunked scan measures 1 to 9 %
-// less per prefill as well (0.4B 1 x 64 1561 / 1432, 16 x 64 4653 / 4528); the
-// line stays here because the segmented serial scan, the path of sequences past
-// the chunk kernels' 32-bit offsets too, would be left with those alone.
+// 1 x 128 and 1 x 512 and the 1.5B-shaped 4 x 1024 faster, 0.4B 1 x 32 1236
+// us serial, 1274 chunked). From 48 tokens on the chunked scan measures 2 to 11 %
+// less per prefill as well (0.4B 1 x 48 1402 / 1368, 1 x 64 1518 / 1399, 1 x 127 1741 /
+// 1556, 16 x 64 4030 / 3886): the line can come down once sequences past the chunk
+// kernels' 32-bit offsets no longer need the segmented serial scan, which would be
+// left with those alone.
 constexpr int kChunkMinT = 128;
 bool prefill_chunked(int T, int B, int H, int cus);
 // the chunked scan's prep kernel can form the LoRA second steps of these
